@@ -27,13 +27,6 @@ template <> struct Mfma<float> {
     static __device__ __forceinline__ int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
-// Strided read-only view: element (r, k) at p[r*rs + k*cs].
-template <typename T> struct View {
-    const T *p;
-    int64_t rs, cs;
-    __device__ __forceinline__ T at(int r, int k) const { return p[(int64_t)r * rs + (int64_t)k * cs]; }
-};
-
 // 32x32 accumulator of one wave, as 2x2 MFMA blocks of 16x16.
 template <typename T> struct Quad {
     typename Mfma<T>::v4 c[2][2];
@@ -42,65 +35,12 @@ template <typename T> struct Quad {
             for (int n = 0; n < 2; n++)
                 for (int r = 0; r < 4; r++) c[m][n][r] = (T)0;
     }
+    // Block m takes the rows of parity m, block n the columns of parity n (a
+    // lane's two operand rows are then adjacent in LDS: one read for both).
     // Element of block (m,n), register r, owned by `lane`:
-    //   row = m*16 + Mfma<T>::drow(lane, r), col = n*16 + (lane&15)
+    //   row = 2*Mfma<T>::drow(lane, r) + m, col = 2*(lane&15) + n
 };
 
-// acc += A[0:32, 0:K] * B[0:32, 0:K]^T where rows >= ma of A and rows >= nb
-// of B read as zero.  K is consumed in groups of QG k-steps (4*QG columns):
-// all operand loads of group g+1 are issued before the MFMAs of group g, so
-// 16*QG independent loads per lane are in flight while the matrix core works.
-template <typename T>
-__device__ __forceinline__ void quad_load_group(View<T> A, View<T> B, int k0, int K, int i, int kq, bool ra0,
-                                                bool ra1, bool rb0, bool rb1, T (&a0)[4], T (&a1)[4], T (&b0)[4],
-                                                T (&b1)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int k = k0 + 4 * u + kq;
-        const bool ok = k < K;
-        a0[u] = (ok && ra0) ? A.at(i, k) : (T)0;
-        a1[u] = (ok && ra1) ? A.at(i + 16, k) : (T)0;
-        b0[u] = (ok && rb0) ? B.at(i, k) : (T)0;
-        b1[u] = (ok && rb1) ? B.at(i + 16, k) : (T)0;
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void quad_gemm_nt(Quad<T> &q, View<T> A, int ma, View<T> B, int nb, int K, int lane) {
-    const int i = lane & 15, kq = lane >> 4;
-    const bool ra0 = i < ma, ra1 = i + 16 < ma, rb0 = i < nb, rb1 = i + 16 < nb;
-    T a0[4], a1[4], b0[4], b1[4];
-    quad_load_group(A, B, 0, K, i, kq, ra0, ra1, rb0, rb1, a0, a1, b0, b1);
-    for (int k = 0; k < K; k += 16) {
-        T na0[4], na1[4], nb0[4], nb1[4];
-        if (k + 16 < K) quad_load_group(A, B, k + 16, K, i, kq, ra0, ra1, rb0, rb1, na0, na1, nb0, nb1);
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (k + 4 * u < K) {  // uniform across the wave
-                q.c[0][0] = Mfma<T>::mma(a0[u], b0[u], q.c[0][0]);
-                q.c[0][1] = Mfma<T>::mma(a0[u], b1[u], q.c[0][1]);
-                q.c[1][0] = Mfma<T>::mma(a1[u], b0[u], q.c[1][0]);
-                q.c[1][1] = Mfma<T>::mma(a1[u], b1[u], q.c[1][1]);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            a0[u] = na0[u]; a1[u] = na1[u]; b0[u] = nb0[u]; b1[u] = nb1[u];
-        }
-    }
-}
-
-// Workgroup-level D(64x64) = X(64xK) * Y(64xK)^T with operands staged through
-// LDS in chunks of CH columns (16 or 32): the 256 threads fetch each chunk
-// once with coalesced column segments (rows contiguous in memory), the 4
-// waves read their MFMA fragments from LDS.  Global loads of chunk c+1 are in
-// flight while chunk c is multiplied, so a chunk's MFMA time (CH/4 * 4
-// MFMAs per wave) is the latency the prefetch can hide.  Rows >= mx of X /
-// >= my of Y read as zero; X(r, k) = X[r + k*ldx].  Wave w owns the 32x32
-// quadrant (w>>1, w&1).  Must be called by all 256 threads (contains
-// barriers).
-// two elements: V2<T>::u with the alignment of one panel element (panels
-// start and lead at any element), V2<T>::a fully aligned (LDS staging rows)
 // Operand staging moves 16 bytes per lane: E = 16 / sizeof(T) consecutive
 // rows of one column (4 floats or 2 doubles).  Vec<T>::u has the alignment
 // of one panel element (panels start and lead at any element), Vec<T>::a is
@@ -128,6 +68,12 @@ template <typename T> __device__ __forceinline__ void ld_rows(const T *p, int r,
         for (int e = 0; e < E; e++) o[e] = (r + e < m) ? p[e] : (T)0;
     }
 }
+// E consecutive elements at p, unconditionally
+template <typename T> __device__ __forceinline__ void ld_vec(const T *p, T *o) {
+    const typename Vec<T>::u v = *reinterpret_cast<const typename Vec<T>::u *>(p);
+#pragma unroll
+    for (int e = 0; e < Vec<T>::E; e++) o[e] = v[e];
+}
 template <typename T> __device__ __forceinline__ void st_rows(T *p, const T *o) {
     typename Vec<T>::a v;
 #pragma unroll
@@ -135,61 +81,127 @@ template <typename T> __device__ __forceinline__ void st_rows(T *p, const T *o) 
     *reinterpret_cast<typename Vec<T>::a *>(p) = v;
 }
 
+// Workgroup-level D(64x64) = X(64xK) * Y(64xK)^T with operands staged through
+// LDS in chunks of CH columns (16 or 32): the 256 threads fetch each chunk
+// once with coalesced column segments (rows contiguous in memory), the 4
+// waves read their MFMA fragments from LDS.  Global loads of chunk c+1 are in
+// flight while chunk c is multiplied, so a chunk's MFMA time (CH/4 * 4
+// MFMAs per wave) is the latency the prefetch can hide.  X(r, k) =
+// X[r + k*ldx].  Wave w owns the 32x32 quadrant (w>>1, w&1); output rows >=
+// mx and columns >= my are not defined.  Must be called by all 256 threads
+// (contains barriers).
+//
+// The loads carry no row masks: a row >= mx of X only reaches output rows >=
+// mx, which nobody stores, so a lane past the last row reads row 0 again and
+// the lane that straddles it up to E - 1 elements more (every device
+// allocation ends in LOAD_PAD bytes of padding for the last column).  With
+// masks the compiler waited for all outstanding loads before every partial
+// one: up to four memory round trips per chunk on a tile with an odd row
+// count.  Columns >= K must count as zero; the last chunk clears them on
+// their way to LDS.  80^3 Laplacian, FP64, together with quad_sub below, one
+// stream: k_update_direct 23.6 -> 21.9 ms, k_update_seq 17.8 -> 14.2 ms,
+// panel steps 19.0 -> 16.2 ms.
 template <typename T, int CH = 16> struct StageBuf {
     T xs[CH][68];
     T ys[CH][68];
 };
 
+// an MFMA operand pair of one lane: rows 2i and 2i+1 of a 32-row fragment
+template <typename T> struct Frag { typedef T v __attribute__((ext_vector_type(2))); };
+
+// one chunk's MFMAs of a 32x32 quadrant, X fragments at xs[.][xr], Y at
+// ys[.][yr]; left columns of the chunk (and later) exist.  The steps stay
+// behind the test of left: without it (straight-line code) the direct update
+// ran 22.4 instead of 21.9 ms.
+template <typename T, int CH, int PX, int PY>
+__device__ __forceinline__ void quad_chunk(Quad<T> &q, const T (*xs)[PX], const T (*ys)[PY], int xr, int yr, int left,
+                                           int kq) {
+#pragma unroll
+    for (int s = 0; s < CH / 4; s++) {
+        if (4 * s >= left) break;  // uniform
+        const typename Frag<T>::v x = *reinterpret_cast<const typename Frag<T>::v *>(&xs[4 * s + kq][xr]);
+        const typename Frag<T>::v y = *reinterpret_cast<const typename Frag<T>::v *>(&ys[4 * s + kq][yr]);
+        q.c[0][0] = Mfma<T>::mma(x[0], y[0], q.c[0][0]);
+        q.c[0][1] = Mfma<T>::mma(x[0], y[1], q.c[0][1]);
+        q.c[1][0] = Mfma<T>::mma(x[1], y[0], q.c[1][0]);
+        q.c[1][1] = Mfma<T>::mma(x[1], y[1], q.c[1][1]);
+    }
+}
+
+// One operand's chunk loads: R rows (64 or 128) of CH columns by the 256
+// threads, 16 bytes per lane.  The column a wave's first lanes read is
+// uniform, so the address is a scalar base plus a 32-bit lane offset of at
+// most CPW - 1 columns and R rows.  It fits: a panel's rows are a clique of
+// the factor, so its leading dimension squared is at most twice the stored
+// entries.  No branches around the loads: with one for the last chunk the
+// compiler waited between them.
+template <typename T, int R, int CH> struct Stager {
+    static constexpr int E = Vec<T>::E, LPC = R / E, CPW = 64 / LPC, NP = CH / (4 * CPW);
+    static_assert(NP >= 1 && CH % (4 * CPW) == 0, "chunk of whole passes");
+    const char *base;
+    int64_t ldb;  // bytes from column to column
+    unsigned row;
+    int r, kl, kw;
+    T g[NP][E];
+    // rows [0, m) of P, column k at P + k*ld
+    __device__ __forceinline__ void init(const T *P, int m, int64_t ld, int lane, int wave) {
+        r = E * (lane % LPC);
+        kl = lane / LPC;
+        kw = CPW * wave;
+        ldb = ld * (int64_t)sizeof(T);
+        base = reinterpret_cast<const char *>(P);
+        row = (unsigned)((r < m ? r : 0) * sizeof(T));
+    }
+    // columns [k0, k0 + CH); those at and after K read column K - 1 again
+    __device__ __forceinline__ void load(int k0, int K) {
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+            const int c = min(k0 + kw + 4 * CPW * u, K - 1);  // uniform
+            const unsigned off = row + (unsigned)min(kl, K - 1 - c) * (unsigned)ldb;
+            ld_vec(reinterpret_cast<const T *>(base + (int64_t)c * ldb + off), g[u]);
+        }
+    }
+    // into s, columns at and after K as zeros
+    template <int P> __device__ __forceinline__ void store(T (*s)[P], int k0, int K) {
+        if (k0 + CH > K) {  // uniform
+#pragma unroll
+            for (int u = 0; u < NP; u++)
+#pragma unroll
+                for (int e = 0; e < E; e++)
+                    if (k0 + kw + 4 * CPW * u + kl >= K) g[u][e] = (T)0;
+        }
+#pragma unroll
+        for (int u = 0; u < NP; u++) st_rows(&s[kw + 4 * CPW * u + kl][r], g[u]);
+    }
+};
+
 template <typename T, int CH>
 __device__ __forceinline__ void wg_gemm_lds(Quad<T> &q, const T *X, int mx, int64_t ldx, const T *Y, int my,
                                             int64_t ldy, int K, StageBuf<T, CH> &sb, int tid) {
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    const int i = lane & 15, kq = lane >> 4;
-    // 16 bytes per lane: E rows of one column, 4E columns per pass of the
-    // workgroup, CH / 4E passes per chunk
-    constexpr int E = Vec<T>::E, NP = CH / (4 * E);
-    static_assert(CH % (4 * E) == 0, "chunk of whole passes");
-    const int re = E * (tid % (64 / E)), ke = tid / (64 / E);
-    T gx[NP][E], gy[NP][E];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int u = 0; u < NP; u++) {
-            const int k = k0 + ke + 4 * E * u;
-            ld_rows(X + re + (int64_t)k * ldx, re, k < K ? mx : 0, gx[u]);
-            ld_rows(Y + re + (int64_t)k * ldy, re, k < K ? my : 0, gy[u]);
-        }
-    };
-    auto sstore = [&]() {
-#pragma unroll
-        for (int u = 0; u < NP; u++) {
-            st_rows(&sb.xs[ke + 4 * E * u][re], gx[u]);
-            st_rows(&sb.ys[ke + 4 * E * u][re], gy[u]);
-        }
-    };
+    const int i = 2 * (lane & 15), kq = lane >> 4;
+    Stager<T, 64, CH> gx, gy;
+    gx.init(X, mx, ldx, lane, wave);
+    gy.init(Y, my, ldy, lane, wave);
     const bool active = (wr < mx) && (wc < my);
-    gload(0);
-    sstore();
+    gx.load(0, K);
+    gy.load(0, K);
+    gx.store(sb.xs, 0, K);
+    gy.store(sb.ys, 0, K);
     __syncthreads();
     for (int k0 = 0; k0 < K; k0 += CH) {
         const bool more = k0 + CH < K;
-        if (more) gload(k0 + CH);
-        if (active) {
-#pragma unroll
-            for (int s = 0; s < CH / 4; s++) {
-                if (k0 + 4 * s < K) {
-                    const int kr = 4 * s + kq;
-                    const T a0 = sb.xs[kr][wr + i], a1 = sb.xs[kr][wr + 16 + i];
-                    const T b0 = sb.ys[kr][wc + i], b1 = sb.ys[kr][wc + 16 + i];
-                    q.c[0][0] = Mfma<T>::mma(a0, b0, q.c[0][0]);
-                    q.c[0][1] = Mfma<T>::mma(a0, b1, q.c[0][1]);
-                    q.c[1][0] = Mfma<T>::mma(a1, b0, q.c[1][0]);
-                    q.c[1][1] = Mfma<T>::mma(a1, b1, q.c[1][1]);
-                }
-            }
+        if (more) {
+            gx.load(k0 + CH, K);
+            gy.load(k0 + CH, K);
         }
+        if (active) quad_chunk<T, CH>(q, sb.xs, sb.ys, wr + i, wc + i, K - k0, kq);
         __syncthreads();
-        if (more) sstore();
+        if (more) {
+            gx.store(sb.xs, k0 + CH, K);
+            gy.store(sb.ys, k0 + CH, K);
+        }
         __syncthreads();
     }
 }
@@ -207,64 +219,76 @@ template <typename T, int CH>
 __device__ __forceinline__ void wg_gemm_lds_64x128(Quad<T> &q0, Quad<T> &q1, const T *X, int mx, int64_t ldx,
                                                    const T *Y, int my, int64_t ldy, int K, StageBuf2<T, CH> &sb,
                                                    int tid) {
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = (wave >> 1) * 32, wc = (wave & 1) * 64;
-    const int i = lane & 15, kq = lane >> 4;
-    // 16 bytes per lane: X (64 rows) 4E columns per pass, Y (128 rows) 2E
-    constexpr int E = Vec<T>::E, NPX = CH / (4 * E), NPY = CH / (2 * E);
-    static_assert(CH % (4 * E) == 0, "chunk of whole passes");
-    const int rex = E * (tid % (64 / E)), kex = tid / (64 / E);
-    const int rey = E * (tid % (128 / E)), key = tid / (128 / E);
-    T gx[NPX][E], gy[NPY][E];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int u = 0; u < NPX; u++) {
-            const int k = k0 + kex + 4 * E * u;
-            ld_rows(X + rex + (int64_t)k * ldx, rex, k < K ? mx : 0, gx[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < NPY; u++) {
-            const int k = k0 + key + 2 * E * u;
-            ld_rows(Y + rey + (int64_t)k * ldy, rey, k < K ? my : 0, gy[u]);
-        }
-    };
-    auto sstore = [&]() {
-#pragma unroll
-        for (int u = 0; u < NPX; u++) st_rows(&sb.xs[kex + 4 * E * u][rex], gx[u]);
-#pragma unroll
-        for (int u = 0; u < NPY; u++) st_rows(&sb.ys[key + 2 * E * u][rey], gy[u]);
-    };
+    const int i = 2 * (lane & 15), kq = lane >> 4;
+    Stager<T, 64, CH> gx;
+    Stager<T, 128, CH> gy;
+    gx.init(X, mx, ldx, lane, wave);
+    gy.init(Y, my, ldy, lane, wave);
     const bool act0 = (wr < mx) && (wc < my), act1 = act0 && (wc + 32 < my);
-    gload(0);
-    sstore();
+    gx.load(0, K);
+    gy.load(0, K);
+    gx.store(sb.xs, 0, K);
+    gy.store(sb.ys, 0, K);
     __syncthreads();
     for (int k0 = 0; k0 < K; k0 += CH) {
         const bool more = k0 + CH < K;
-        if (more) gload(k0 + CH);
+        if (more) {
+            gx.load(k0 + CH, K);
+            gy.load(k0 + CH, K);
+        }
         if (act0) {
 #pragma unroll
             for (int s = 0; s < CH / 4; s++) {
                 if (k0 + 4 * s < K) {
-                    const int kr = 4 * s + kq;
-                    const T a0 = sb.xs[kr][wr + i], a1 = sb.xs[kr][wr + 16 + i];
-                    const T b0 = sb.ys[kr][wc + i], b1 = sb.ys[kr][wc + 16 + i];
-                    q0.c[0][0] = Mfma<T>::mma(a0, b0, q0.c[0][0]);
-                    q0.c[0][1] = Mfma<T>::mma(a0, b1, q0.c[0][1]);
-                    q0.c[1][0] = Mfma<T>::mma(a1, b0, q0.c[1][0]);
-                    q0.c[1][1] = Mfma<T>::mma(a1, b1, q0.c[1][1]);
+                    const typename Frag<T>::v x = *reinterpret_cast<const typename Frag<T>::v *>(&sb.xs[4 * s + kq][wr + i]);
+                    const typename Frag<T>::v y = *reinterpret_cast<const typename Frag<T>::v *>(&sb.ys[4 * s + kq][wc + i]);
+                    q0.c[0][0] = Mfma<T>::mma(x[0], y[0], q0.c[0][0]);
+                    q0.c[0][1] = Mfma<T>::mma(x[0], y[1], q0.c[0][1]);
+                    q0.c[1][0] = Mfma<T>::mma(x[1], y[0], q0.c[1][0]);
+                    q0.c[1][1] = Mfma<T>::mma(x[1], y[1], q0.c[1][1]);
                     if (act1) {
-                        const T b2 = sb.ys[kr][wc + 32 + i], b3 = sb.ys[kr][wc + 48 + i];
-                        q1.c[0][0] = Mfma<T>::mma(a0, b2, q1.c[0][0]);
-                        q1.c[0][1] = Mfma<T>::mma(a0, b3, q1.c[0][1]);
-                        q1.c[1][0] = Mfma<T>::mma(a1, b2, q1.c[1][0]);
-                        q1.c[1][1] = Mfma<T>::mma(a1, b3, q1.c[1][1]);
+                        const typename Frag<T>::v z = *reinterpret_cast<const typename Frag<T>::v *>(&sb.ys[4 * s + kq][wc + 32 + i]);
+                        q1.c[0][0] = Mfma<T>::mma(x[0], z[0], q1.c[0][0]);
+                        q1.c[0][1] = Mfma<T>::mma(x[0], z[1], q1.c[0][1]);
+                        q1.c[1][0] = Mfma<T>::mma(x[1], z[0], q1.c[1][0]);
+                        q1.c[1][1] = Mfma<T>::mma(x[1], z[1], q1.c[1][1]);
                     }
                 }
             }
         }
         __syncthreads();
-        if (more) sstore();
+        if (more) {
+            gx.store(sb.xs, k0 + CH, K);
+            gy.store(sb.ys, k0 + CH, K);
+        }
         __syncthreads();
+    }
+}
+
+// The quadrant subtracted from memory: at(row, col, ok) gives the address of
+// element (row, col) of the quadrant and whether it exists (the address must
+// be readable either way).  Eight elements' loads go out together: written as
+// C -= q one element at a time, every load waited for the store before it
+// (they may alias), sixteen memory round trips in a row per tile.
+template <typename T, class At> __device__ __forceinline__ void quad_sub(const Quad<T> &q, int lane, At at) {
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        T *p[2][4], v[2][4];
+        bool ok[2][4];
+#pragma unroll
+        for (int n = 0; n < 2; n++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                p[n][r] = at(2 * Mfma<T>::drow(lane, r) + m, 2 * (lane & 15) + n, ok[n][r]);
+                v[n][r] = *p[n][r];
+            }
+#pragma unroll
+        for (int n = 0; n < 2; n++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (ok[n][r]) *p[n][r] = v[n][r] - q.c[m][n][r];
     }
 }
 

@@ -5,6 +5,10 @@
 
 namespace pxa {
 
+// bytes past the end of every device allocation that the tiles' unmasked
+// 16-byte operand loads may touch (the last rows of the last column)
+constexpr int LOAD_PAD = 64;
+
 // Flattened SolverMatrix (reference blend/solver.h:83-213) in device memory.
 // Panels use the 1D layout: cblk c owns coef[cblk_coef[c] .. +stride*width),
 // column-major with ld = stride; block b is rows [blok_roff[b], +nrows).

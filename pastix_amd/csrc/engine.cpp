@@ -47,7 +47,7 @@ int Engine::fail(const std::string &m) {
 void *Engine::alloc(size_t bytes) {
     void *p = nullptr;
     if (bytes == 0) bytes = 8;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
+    if (hipMalloc(&p, bytes + LOAD_PAD) != hipSuccess) {
         fail("hipMalloc of " + std::to_string(bytes) + " bytes failed");
         return nullptr;
     }

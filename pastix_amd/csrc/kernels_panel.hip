@@ -28,8 +28,8 @@ namespace pxa {
     for (int m_ = 0; m_ < 2; m_++)                                       \
         for (int n_ = 0; n_ < 2; n_++)                                   \
             for (int r_ = 0; r_ < 4; r_++) {                             \
-                const int qrow = m_ * 16 + Mfma<T>::drow(lane, r_);       \
-                const int qcol = n_ * 16 + (lane & 15);                   \
+                const int qrow = 2 * Mfma<T>::drow(lane, r_) + m_;        \
+                const int qcol = 2 * (lane & 15) + n_;                    \
                 __VA_ARGS__                                              \
             }
 
@@ -416,8 +416,11 @@ __device__ __forceinline__ void panel_upd_tile(const DevSymbol &S, const PanelIt
     wg_gemm_lds<T, 16>(q, X + r0, mr, ld, Y + c0, mc, ld, kn, sb, tid);
     if (wr < mr && wc < mc) {
         const bool diag = r0 == c0;
-        QFOR(if (qrow < mr - wr && qcol < mc - wc && (!diag || wr + qrow > wc + qcol - (strict ? 0 : 1)))
-                 P[(r0 + wr + qrow) + (int64_t)(c0 + wc + qcol) * ld] -= q.c[m_][n_][r_];)
+        T *C = P + (r0 + wr) + (int64_t)(c0 + wc) * ld;
+        quad_sub(q, lane, [&](int qrow, int qcol, bool &ok) -> T * {
+            ok = qrow < mr - wr && qcol < mc - wc && (!diag || wr + qrow > wc + qcol - (strict ? 0 : 1));
+            return ok ? C + qrow + (int64_t)qcol * ld : C;
+        });
     }
 }
 
@@ -482,34 +485,39 @@ __global__ __launch_bounds__(256) void k_panel_upd_potrf(DevSymbol S, const int3
 // the members' 64-column inverses into the W and WT of nodes of several
 // cblks (a node of one cblk already holds them in place).
 
-// D(64x64) += X(64xK) Y(64xK)^T as wg_gemm_lds, where xcol(k) points at
-// X(0, k) (rows contiguous; called with increasing k, also for k >= K, whose
-// rows are not read) and Y(r, k) = Y[k + r*ldy] (consecutive k contiguous)
+// D(64x64) += X(64xK) Y(64xK)^T as wg_gemm_lds (K >= 1), where xcol(k) points
+// at X(0, k) (rows contiguous; called with increasing k, also for k >= K,
+// where it must still point at readable rows) and Y(r, k) = Y[k + r*ldy] (consecutive k contiguous)
 template <typename T, int CH, class XCol>
 __device__ __forceinline__ void wg_gemm_lds_xcol_yt(Quad<T> &q, XCol &xcol, int mx, const T *Y, int my, int64_t ldy,
                                                     int K, StageBuf<T, CH> &sb, int tid) {
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    const int i = lane & 15, kq = lane >> 4;
+    const int i = 2 * (lane & 15), kq = lane >> 4;
     constexpr int E = Vec<T>::E, NP = CH / (4 * E), NY = CH / 4;
-    static_assert(CH % (4 * E) == 0 && CH % 4 == 0, "chunk of whole passes");
     const int re = E * (tid % (64 / E)), ke = tid / (64 / E);
     // Y: thread (row yr, k group yk) fetches NY consecutive k of its row
     const int yr = tid & 63, yk = (tid >> 6) * NY;
+    const int rx = re < mx ? re : 0;
+    const T *py = Y + (int64_t)min(yr, my - 1) * ldy;
     T gx[NP][E], gy[NY];
     auto gload = [&](int k0) {
 #pragma unroll
-        for (int u = 0; u < NP; u++) {
-            const int k = k0 + ke + 4 * E * u;
-            ld_rows(xcol(k) + re, re, k < K ? mx : 0, gx[u]);
-        }
+        for (int u = 0; u < NP; u++) ld_vec(xcol(k0 + ke + 4 * E * u) + rx, gx[u]);
 #pragma unroll
-        for (int e = 0; e < NY; e++) {
-            const int k = k0 + yk + e;
-            gy[e] = (k < K && yr < my) ? Y[k + (int64_t)yr * ldy] : (T)0;
-        }
+        for (int e = 0; e < NY; e++) gy[e] = py[min(k0 + yk + e, K - 1)];
     };
-    auto sstore = [&]() {
+    auto sstore = [&](int k0) {
+        if (k0 + CH > K) {  // uniform: the last chunk, columns >= K cleared
+#pragma unroll
+            for (int u = 0; u < NP; u++)
+#pragma unroll
+                for (int e = 0; e < E; e++)
+                    if (k0 + ke + 4 * E * u >= K) gx[u][e] = (T)0;
+#pragma unroll
+            for (int e = 0; e < NY; e++)
+                if (k0 + yk + e >= K) gy[e] = (T)0;
+        }
 #pragma unroll
         for (int u = 0; u < NP; u++) st_rows(&sb.xs[ke + 4 * E * u][re], gx[u]);
 #pragma unroll
@@ -517,27 +525,14 @@ __device__ __forceinline__ void wg_gemm_lds_xcol_yt(Quad<T> &q, XCol &xcol, int 
     };
     const bool active = (wr < mx) && (wc < my);
     gload(0);
-    sstore();
+    sstore(0);
     __syncthreads();
     for (int k0 = 0; k0 < K; k0 += CH) {
         const bool more = k0 + CH < K;
         if (more) gload(k0 + CH);
-        if (active) {
-#pragma unroll
-            for (int s = 0; s < CH / 4; s++) {
-                if (k0 + 4 * s < K) {
-                    const int kr = 4 * s + kq;
-                    const T a0 = sb.xs[kr][wr + i], a1 = sb.xs[kr][wr + 16 + i];
-                    const T b0 = sb.ys[kr][wc + i], b1 = sb.ys[kr][wc + 16 + i];
-                    q.c[0][0] = Mfma<T>::mma(a0, b0, q.c[0][0]);
-                    q.c[0][1] = Mfma<T>::mma(a0, b1, q.c[0][1]);
-                    q.c[1][0] = Mfma<T>::mma(a1, b0, q.c[1][0]);
-                    q.c[1][1] = Mfma<T>::mma(a1, b1, q.c[1][1]);
-                }
-            }
-        }
+        if (active) quad_chunk<T, CH>(q, sb.xs, sb.ys, wr + i, wc + i, K - k0, kq);
         __syncthreads();
-        if (more) sstore();
+        if (more) sstore(k0 + CH);
         __syncthreads();
     }
 }

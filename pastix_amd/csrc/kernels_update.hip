@@ -25,7 +25,8 @@ namespace pxa {
 
 // K columns staged per LDS chunk in the single-tile GEMMs (16 measured
 // faster than 32 on gfx950: the smaller LDS footprint keeps 6 workgroups per
-// CU resident).
+// CU resident; two buffers of 8 columns with one barrier each were no faster,
+// two of 16 slower, 24.0 against 21.9 ms).
 constexpr int UPD_CH = 16;
 
 // register budget held to seven waves per SIMD (72 registers in FP64, no
@@ -58,13 +59,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
     const int64_t stf = S.cblk_stride[f];
     T *C = Ccoef + S.cblk_coef[f] + r0 + (int64_t)c0 * stf;
     if (wr < nq && wc < np) {
-        UQFOR({
+        quad_sub(q, lane, [&](int qrow, int qcol, bool &ok) -> T * {
             const int qj = wr + qrow, pi = wc + qcol;
-            if (qj < nq && pi < np) {
-                const bool keep = (MODE == 0) ? (rblk[pi] >= qblk[qj]) : (rblk[pi] > qblk[qj]);
-                if (keep) C[rmap[pi] + (int64_t)cmap[qj] * stf] -= q.c[m_][n_][r_];
-            }
-        })
+            ok = qj < nq && pi < np && ((MODE == 0) ? (rblk[pi] >= qblk[qj]) : (rblk[pi] > qblk[qj]));
+            return ok ? C + rmap[pi] + (int64_t)cmap[qj] * stf : C;
+        });
     }
 }
 
@@ -75,7 +74,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
 // element another wave wrote sees it.  The direct kernel's LDS footprint
 // (no 64x64 accumulator), so six waves per SIMD instead of three.
 template <typename T, int MODE>
-__global__ __launch_bounds__(256) void k_update_seq(DevSymbol S, const UpdItem *__restrict__ items, int nitems,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_update_seq(DevSymbol S, const UpdItem *__restrict__ items, int nitems,
                                                     const UpdEntry *__restrict__ ents, const int32_t *__restrict__ shift,
                                                     const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
                                                     T *__restrict__ Ccoef) {
@@ -105,13 +104,11 @@ __global__ __launch_bounds__(256) void k_update_seq(DevSymbol S, const UpdItem *
         wg_gemm_lds<T, UPD_CH>(q, Bcoef + S.cblk_coef[s] + en.q0, nq, ld, Acoef + S.cblk_coef[s] + en.p0, np, ld, K,
                                sb, tid);
         if (wr < nq && wc < np) {
-            UQFOR({
+            quad_sub(q, lane, [&](int qrow, int qcol, bool &ok) -> T * {
                 const int qj = wr + qrow, pi = wc + qcol;
-                if (qj < nq && pi < np) {
-                    const bool keep = (MODE == 0) ? (rblk[pi] >= qblk[qj]) : (rblk[pi] > qblk[qj]);
-                    if (keep) C[rmap[pi] + (int64_t)cmap[qj] * stf] -= q.c[m_][n_][r_];
-                }
-            })
+                ok = qj < nq && pi < np && ((MODE == 0) ? (rblk[pi] >= qblk[qj]) : (rblk[pi] > qblk[qj]));
+                return ok ? C + rmap[pi] + (int64_t)cmap[qj] * stf : C;
+            });
         }
     }
 }
