@@ -125,10 +125,22 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     S_.cblk_btile = upload(*this, P.cblk_btile);
 
     lv_cblk_ptr_ = P.lv_cblk_ptr;
-    lv_fact_cnt_ = P.lv_fact_cnt;
     schurfcol_ = (P.schur_cblk < cblknbr_) ? s.cblk_fcol[P.schur_cblk] : n_;
-    d_fact_cblks_ = upload(*this, P.fact_cblks);
-    n_fact_ = (int)P.fact_cblks.size();
+    lv_sq_ptr_.clear();
+    if (factotype == 2) {
+        std::vector<PanelItem> sq;
+        lv_sq_ptr_.push_back(0);
+        for (int32_t lv = 0; lv < P.nlevels; lv++) {
+            for (int32_t k = P.lv_cblk_ptr[lv]; k < P.lv_cblk_ptr[lv] + P.lv_fact_cnt[lv]; k++) {
+                const int32_t c = P.lv_cblks[k], K = (int32_t)(s.cblk_fcol[c + 1] - s.cblk_fcol[c]);
+                for (int32_t c0 = 0; c0 < K; c0 += 64)
+                    for (int32_t r0 = c0; r0 < K; r0 += 64) sq.push_back(PanelItem{c, r0, c0, 0});
+            }
+            lv_sq_ptr_.push_back((int32_t)sq.size());
+        }
+        d_sq_ = upload(*this, sq);
+        if (!d_sq_) return -1;
+    }
     // leaf region of LL^t factorisations
     leaf_ = LeafDev{};
     leaf_levels_ = 0;
@@ -164,7 +176,6 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     lv_wt_next_ = P.lv_wt_next;
     slv_fwd_ptr_ = P.slv_fwd_ptr;
     slv_bwd_ptr_ = P.slv_bwd_ptr;
-    d_lv_cblks_ = upload(*this, P.lv_cblks);
     lv_step_ptr_ = P.lv_step_ptr;
     step_cb_ptr_ = P.step_cb_ptr;
     step_trsm_ptr_ = P.step_trsm_ptr;
@@ -395,11 +406,10 @@ template <typename T> int Engine::factorize_t(double thr) {
     for (size_t lv = lv_first; lv < nl; lv++) {
         cur_lv_ = (int)lv;
         int pk = prof_begin(stream_);
-        if (facto_ == 2) {
-            // the level's factored cblks (the Schur ones keep their sums)
-            const int c0 = lv_cblk_ptr_[lv], nc = lv_fact_cnt_[lv];
-            launch_lu_square_merge<T>(S_, d_lv_cblks_ + c0, nc, L, U, stream_);
-        }
+        // the level's factored cblks (the Schur ones keep their sums); level
+        // 0 has received no update
+        if (facto_ == 2 && lv > 0)
+            launch_lu_square_merge<T>(S_, d_sq_ + lv_sq_ptr_[lv], lv_sq_ptr_[lv + 1] - lv_sq_ptr_[lv], L, U, stream_);
         // blocked panel: 64-column steps, each over every cblk of the level
         for (int s = lv_step_ptr_[lv]; s < lv_step_ptr_[lv + 1]; s++) {
             const int kb = s - lv_step_ptr_[lv];
@@ -508,7 +518,7 @@ template <typename T> int Engine::factorize_t(double thr) {
         HIPCHK(hipStreamWaitEvent(stream_, ev_winv_, 0));
     }
     // LU: the squares in the reference layout once every inverse is formed
-    if (facto_ == 2) launch_lu_square_layout<T>(S_, d_fact_cblks_, n_fact_, L, U, stream_);
+    if (facto_ == 2) launch_lu_square_layout<T>(S_, d_sq_, lv_sq_ptr_.back(), L, U, stream_);
     HIPCHK(hipGetLastError());
     return 0;
 }

@@ -202,15 +202,16 @@ class Engine {
     // solve levels: widest node (diagonal kernels), widest cblk (products)
     std::vector<int> slv_maxw_, slv_maxcw_;
     int64_t schurfcol_ = 0;
-    std::vector<int32_t> lv_fact_cnt_;
-    int32_t *d_fact_cblks_ = nullptr;
-    int n_fact_ = 0;
+    // LU: 64x64 tiles on and below the diagonal of the factored cblks'
+    // squares, level L's at [lv_sq_ptr_[L], lv_sq_ptr_[L + 1])
+    PanelItem *d_sq_ = nullptr;
+    std::vector<int32_t> lv_sq_ptr_;
     DevSymbol S_{};
     // host copies of the level pointers
     std::vector<int32_t> lv_cblk_ptr_, lv_upd_ptr_, lv_upd_split_, slv_fwd_ptr_, slv_bwd_ptr_;
     std::vector<int32_t> lv_upd_dnext_, lv_upd_mnext_, lv_wt_next_;
     // device plan
-    int32_t *d_lv_cblks_ = nullptr, *d_shift_ = nullptr;
+    int32_t *d_shift_ = nullptr;
     YSlices ys_{};  // update-buffer slices
     int32_t *d_ydst_ = nullptr;
     int64_t nyrows_ = 0;

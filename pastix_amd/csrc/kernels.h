@@ -49,9 +49,9 @@ template <typename T>
 void launch_getrf64(const DevSymbol &S, const int32_t *cblks, int n, int kb, T *lcoef, T *ucoef, T *w1, T *w2, T *wb,
                     double thr, int *stat, hipStream_t st);
 template <typename T>
-void launch_lu_square_merge(const DevSymbol &S, const int32_t *cblks, int n, T *lcoef, T *ucoef, hipStream_t st);
+void launch_lu_square_merge(const DevSymbol &S, const PanelItem *items, int n, T *lcoef, T *ucoef, hipStream_t st);
 template <typename T>
-void launch_lu_square_layout(const DevSymbol &S, const int32_t *cblks, int n, T *lcoef, T *ucoef, hipStream_t st);
+void launch_lu_square_layout(const DevSymbol &S, const PanelItem *items, int n, T *lcoef, T *ucoef, hipStream_t st);
 // Inverses of the solve nodes' diagonal blocks from the 64-column inverses
 // the diagonal-block kernels leave in w (and wt): the leaves of nodes of
 // several cblks copied into the nodes' inverses, then nrounds merge rounds,

@@ -778,48 +778,97 @@ __global__ __launch_bounds__(256) void k_getrf64(DevSymbol S, const int32_t *__r
     }
 }
 
+// The square parts of the LU panels, by 64x64 tiles on and below the
+// diagonal (item: rows [r0, r0+64), columns [c0, c0+64) of cblk c's square,
+// r0 >= c0) and their mirror images above it.  Bound by memory: each tile
+// crosses LDS so that both the tile and its mirror are walked down columns.
+// One workgroup per cblk with the transposed side read across columns took
+// 135 us per level and 353 us for the layout on the 48^3 27-point operator
+// (FP64, beside the updates of the second stream); these take 21 and 71 us.
+
 // Before the LU panel of a cblk: the square part's upper triangle arrives
 // split between the L panel (same-block Schur contributions, written above
 // the diagonal as the reference does) and the U panel (transposed): the
 // reference adds them (core_zgeadd, kernels/core_zgetrfsp.c:240-242); here
 // the sum goes to the U panel and the L panel keeps the lower triangle only.
 template <typename T>
-__global__ __launch_bounds__(256) void k_lu_square_merge(DevSymbol S, const int32_t *__restrict__ cblks,
+__global__ __launch_bounds__(256) void k_lu_square_merge(DevSymbol S, const PanelItem *__restrict__ items,
                                                          T *__restrict__ lcoef, T *__restrict__ ucoef) {
-    const int c = cblks[blockIdx.x];
-    const int K = S.cblk_fcol[c + 1] - S.cblk_fcol[c];
-    const int64_t ld = S.cblk_stride[c];
-    T *PL = lcoef + S.cblk_coef[c];
-    T *PU = ucoef + S.cblk_coef[c];
-    for (int64_t e = threadIdx.x; e < (int64_t)K * K; e += 256) {
-        const int r = (int)(e % K), cc = (int)(e / K);
-        if (r < cc) {
-            PU[cc + (int64_t)r * ld] += PL[r + (int64_t)cc * ld];
-            PL[r + (int64_t)cc * ld] = (T)0;
-        }
+    __shared__ T tile[64][65];
+    const PanelItem it = items[blockIdx.x];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int K = S.cblk_fcol[it.c + 1] - S.cblk_fcol[it.c];
+    const int64_t ld = S.cblk_stride[it.c];
+    T *PL = lcoef + S.cblk_coef[it.c], *PU = ucoef + S.cblk_coef[it.c];
+    // L(r, cc), r < cc: rows r = c0 + lane of columns cc = r0 + j
+    const int r = it.c0 + lane;
+    T v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int cc = it.r0 + w + 4 * u;
+        v[u] = (r < cc && cc < K) ? PL[r + (int64_t)cc * ld] : (T)0;
+    }
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int cc = it.r0 + w + 4 * u;
+        if (r < cc && cc < K) PL[r + (int64_t)cc * ld] = (T)0;
+        tile[w + 4 * u][lane] = v[u];
+    }
+    __syncthreads();
+    // added to U^T(cc, r): rows cc = r0 + lane of columns r = c0 + i
+    const int cc = it.r0 + lane;
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int q = it.c0 + w + 4 * u;
+        v[u] = (q < cc && cc < K) ? PU[cc + (int64_t)q * ld] : (T)0;
+    }
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int q = it.c0 + w + 4 * u;
+        if (q < cc && cc < K) PU[cc + (int64_t)q * ld] = v[u] + tile[lane][w + 4 * u];
     }
 }
 
 // Final layout of the LU diagonal blocks (reference core_zgetrfsp.c:240-251):
 // the L panel's square receives the whole LU (strict upper part from the U
 // panel, where it was kept transposed) and the U panel's square its
-// transpose (core_zgetmo).  One workgroup per cblk.
+// transpose (core_zgetmo).  The lower triangles stay, so every entry moves
+// once: L(j, i) = U^T(i, j) and U^T(j, i) = L(i, j) for i > j, and the
+// diagonal of U^T is L's.
 template <typename T>
-__global__ __launch_bounds__(256) void k_lu_square_layout(DevSymbol S, const int32_t *__restrict__ cblks,
+__global__ __launch_bounds__(256) void k_lu_square_layout(DevSymbol S, const PanelItem *__restrict__ items,
                                                           T *__restrict__ lcoef, T *__restrict__ ucoef) {
-    const int c = cblks[blockIdx.x];
-    const int K = S.cblk_fcol[c + 1] - S.cblk_fcol[c];
-    const int64_t ld = S.cblk_stride[c];
-    T *PL = lcoef + S.cblk_coef[c];
-    T *PU = ucoef + S.cblk_coef[c];
-    for (int64_t e = threadIdx.x; e < (int64_t)K * K; e += 256) {
-        const int r = (int)(e % K), cc = (int)(e / K);
-        if (r < cc) PL[r + (int64_t)cc * ld] = PU[cc + (int64_t)r * ld];
+    __shared__ T tl[64][65], tu[64][65];
+    const PanelItem it = items[blockIdx.x];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int K = S.cblk_fcol[it.c + 1] - S.cblk_fcol[it.c];
+    const int64_t ld = S.cblk_stride[it.c];
+    T *PL = lcoef + S.cblk_coef[it.c], *PU = ucoef + S.cblk_coef[it.c];
+    // the lower tile: rows i = r0 + lane of columns j
+    const int i = it.r0 + lane;
+    T a[16], b[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int j = it.c0 + w + 4 * u;
+        const bool ok = i < K && j <= i;
+        a[u] = ok ? PL[i + (int64_t)j * ld] : (T)0;
+        b[u] = ok ? PU[i + (int64_t)j * ld] : (T)0;
+    }
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        tl[w + 4 * u][lane] = a[u];
+        tu[w + 4 * u][lane] = b[u];
     }
     __syncthreads();
-    for (int64_t e = threadIdx.x; e < (int64_t)K * K; e += 256) {
-        const int r = (int)(e % K), cc = (int)(e / K);
-        PU[r + (int64_t)cc * ld] = PL[cc + (int64_t)r * ld];
+    // its mirror: rows j = c0 + lane of columns i
+    const int j = it.c0 + lane;
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int q = it.r0 + w + 4 * u;
+        if (q < K && j <= q) {
+            PU[j + (int64_t)q * ld] = tl[lane][w + 4 * u];
+            if (j < q) PL[j + (int64_t)q * ld] = tu[lane][w + 4 * u];
+        }
     }
 }
 
@@ -954,14 +1003,14 @@ void launch_getrf64(const DevSymbol &S, const int32_t *cblks, int n, int kb, T *
     hipLaunchKernelGGL(k_getrf64<T>, dim3(n), dim3(256), 0, st, S, cblks, kb, lcoef, ucoef, w1, w2, wb, thr, stat);
 }
 template <typename T>
-void launch_lu_square_merge(const DevSymbol &S, const int32_t *cblks, int n, T *lcoef, T *ucoef, hipStream_t st) {
+void launch_lu_square_merge(const DevSymbol &S, const PanelItem *items, int n, T *lcoef, T *ucoef, hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_lu_square_merge<T>, dim3(n), dim3(256), 0, st, S, cblks, lcoef, ucoef);
+    hipLaunchKernelGGL(k_lu_square_merge<T>, dim3(n), dim3(256), 0, st, S, items, lcoef, ucoef);
 }
 template <typename T>
-void launch_lu_square_layout(const DevSymbol &S, const int32_t *cblks, int n, T *lcoef, T *ucoef, hipStream_t st) {
+void launch_lu_square_layout(const DevSymbol &S, const PanelItem *items, int n, T *lcoef, T *ucoef, hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_lu_square_layout<T>, dim3(n), dim3(256), 0, st, S, cblks, lcoef, ucoef);
+    hipLaunchKernelGGL(k_lu_square_layout<T>, dim3(n), dim3(256), 0, st, S, items, lcoef, ucoef);
 }
 template <typename T>
 void launch_panel_trsm(const DevSymbol &S, const PanelItem *items, int n, int kb, T *coef, const T *winv,
@@ -1029,8 +1078,8 @@ void launch_leaf_tasks(const DevSymbol &S, const LeafDev &LP, const UpdEntry *en
                                        hipStream_t);                                                               \
     template void launch_getrf64<T>(const DevSymbol &, const int32_t *, int, int, T *, T *, T *, T *, T *, double, \
                                     int *, hipStream_t);                                                           \
-    template void launch_lu_square_layout<T>(const DevSymbol &, const int32_t *, int, T *, T *, hipStream_t);      \
-    template void launch_lu_square_merge<T>(const DevSymbol &, const int32_t *, int, T *, T *, hipStream_t);       \
+    template void launch_lu_square_layout<T>(const DevSymbol &, const PanelItem *, int, T *, T *, hipStream_t);      \
+    template void launch_lu_square_merge<T>(const DevSymbol &, const PanelItem *, int, T *, T *, hipStream_t);       \
     template void launch_potrf64<T>(const DevSymbol &, const int32_t *, int, int, T *, T *, T *, double, int *,    \
                                     hipStream_t);                                                                  \
     template void launch_panel_trsm<T>(const DevSymbol &, const PanelItem *, int, int, T *, const T *, hipStream_t); \

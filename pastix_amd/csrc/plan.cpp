@@ -83,7 +83,6 @@ Plan build_plan(const Symbol &s, const Layout &L, int64_t schur_cblk, const Plan
             P.lv_fact_cnt[L.cblk_level[c]]++;
         }
         for (int64_t c = sc; c < cb; c++) P.lv_cblks[pos[L.cblk_level[c]]++] = (int32_t)c;
-        for (int64_t c = 0; c < sc; c++) P.fact_cblks.push_back((int32_t)c);
     }
     auto width = [&](int64_t c) { return s.cblk_fcol[c + 1] - s.cblk_fcol[c]; };
     auto rows = [&](int64_t b) { return s.blok_lrow[b] - s.blok_frow[b] + 1; };

@@ -29,7 +29,6 @@ struct Plan {
     // come after the factored cblks, of which there are lv_fact_cnt[lv]
     int32_t schur_cblk = 0;
     std::vector<int32_t> lv_fact_cnt;
-    std::vector<int32_t> fact_cblks;  // every factored cblk
     // blocked panel steps: level L owns steps [lv_step_ptr[L], lv_step_ptr[L+1]),
     // step s is column block kb = s - lv_step_ptr[L] of the level's cblks
     std::vector<int32_t> lv_step_ptr;
