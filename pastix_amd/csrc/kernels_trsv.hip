@@ -24,8 +24,9 @@
 // The diagonal inverses are stored whole (zeros in the other triangle), so
 // the triangular products run over full 64-column blocks.  Every output
 // element is produced in a fixed order by one workgroup: no atomics,
-// bitwise-reproducible solves.  NR is the compile-time bound on the
-// right-hand sides of one launch (1 or 8); NW the waves of a workgroup.
+// bitwise-reproducible solves.  NW: waves of a workgroup.  Several
+// right-hand sides take the kernels on the matrix cores (k_*_m,
+// k_diag_gemm16), one takes the vector kernels.
 #include <algorithm>
 
 #include "dev_common.h"
@@ -44,37 +45,17 @@ constexpr int SOLVE_TINY = 16;
 // before the diagonal kernels (k_fwd_gather, k_bwd_reduce)
 constexpr int SOLVE_SPLIT = 512;
 
-// Loads and stores of the data one solve task hands to another (update
-// buffer, forward result, solution rows, backward partials).  CO: device-
-// coherent accesses for the single-launch solve, where the producer and the
-// consumer may sit on different dies; plain accesses between level kernels.
-template <bool CO, typename T> __device__ __forceinline__ T ld_co(const T *p) {
-    if constexpr (CO) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else return *p;
-}
-template <bool CO, typename T> __device__ __forceinline__ void st_co(T *p, T v) {
-    if constexpr (CO) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else *p = v;
-}
-
-// red holds NW x 64 x NR partial sums; the sum over waves is taken in wave
-// order by the threads of wave 0.
-template <bool CO, typename T, int NR, int NW>
-__device__ __forceinline__ void wave_sum_store(T (&acc)[NR], T *red, int r, int q, bool ok, int nrhs, T *out,
-                                               int64_t ldo, const T *sub, int64_t lds) {
-#pragma unroll
-    for (int u = 0; u < NR; u++) red[(q * 64 + r) * NR + u] = acc[u];
+// red holds NW x 64 partial sums; the sum over waves is taken in wave order
+// by the threads of wave 0.
+template <typename T, int NW>
+__device__ __forceinline__ void wave_sum_store(T acc, T *red, int r, int q, bool ok, T *out) {
+    red[q * 64 + r] = acc;
     __syncthreads();
     if (q == 0 && ok) {
+        T v = red[r];
 #pragma unroll
-        for (int u = 0; u < NR; u++) {
-            if (u < nrhs) {
-                T v = red[r * NR + u];
-#pragma unroll
-                for (int w = 1; w < NW; w++) v += red[(w * 64 + r) * NR + u];
-                st_co<CO>(out + u * ldo, sub ? ld_co<CO>(sub + u * lds) - v : v);
-            }
-        }
+        for (int w = 1; w < NW; w++) v += red[w * 64 + r];
+        *out = v;
     }
 }
 
@@ -82,46 +63,40 @@ __device__ __forceinline__ void wave_sum_store(T (&acc)[NR], T *red, int r, int 
 // wave q holds rows E*(l % (64/E)) + i of columns l / (64/E); the E lanes of a
 // row group combine with lane shuffles, then the waves as above (row r =
 // the calling lane).
-template <bool CO, typename T, int NR, int NW, int E>
-__device__ __forceinline__ void wave_sum_store_rows(T (&acc)[E][NR], T *red, int r, int q, bool ok, int nrhs,
-                                                    T *out, int64_t ldo) {
+template <typename T, int NW, int E>
+__device__ __forceinline__ void wave_sum_store_rows(T (&acc)[E], T *red, int r, int q, bool ok, T *out) {
     constexpr int G = 64 / E;
 #pragma unroll
     for (int off = G; off < 64; off *= 2)
 #pragma unroll
-        for (int i = 0; i < E; i++)
-#pragma unroll
-            for (int u = 0; u < NR; u++) acc[i][u] += __shfl_xor(acc[i][u], off);
+        for (int i = 0; i < E; i++) acc[i] += __shfl_xor(acc[i], off);
     if (r < G) {
 #pragma unroll
-        for (int i = 0; i < E; i++)
-#pragma unroll
-            for (int u = 0; u < NR; u++) red[(q * 64 + E * r + i) * NR + u] = acc[i][u];
+        for (int i = 0; i < E; i++) red[q * 64 + E * r + i] = acc[i];
     }
     __syncthreads();
     if (q == 0 && ok) {
+        T v = red[r];
 #pragma unroll
-        for (int u = 0; u < NR; u++) {
-            if (u < nrhs) {
-                T v = red[r * NR + u];
-#pragma unroll
-                for (int w = 1; w < NW; w++) v += red[(w * 64 + r) * NR + u];
-                st_co<CO>(out + u * ldo, v);
-            }
-        }
+        for (int w = 1; w < NW; w++) v += red[w * 64 + r];
+        *out = v;
     }
 }
 
-// ---------------------------------------------------------------------------
-// Task bodies, each run by one whole workgroup of NW waves (the level
-// kernels below and the dependency-driven solve share them).
-// ---------------------------------------------------------------------------
-template <bool CO, typename T, int NR, int NW, bool PRE = false>
-__device__ __forceinline__ void fwd_diag_body(const DevSymbol &S, const DiagItem it,
-                                              const YSlices ys, const T *__restrict__ ybuf,
-                                              int64_t ldy, const T *__restrict__ b, int64_t ldb, T *__restrict__ z,
-                                              int64_t ldz, int nrhs, const T *__restrict__ w1,
-                                              const T *__restrict__ w1t, T *y, T *red) {
+// ------------------- one right-hand side: level kernels ---------------------
+template <typename T, int NW>
+__global__ __launch_bounds__(NW * 64) void k_fwd_diag(DevSymbol S, const DiagItem *__restrict__ items, int nitems,
+                                                      const YSlices ys, const T *__restrict__ ybuf,
+                                                      const T *__restrict__ b, T *__restrict__ z,
+                                                      const T *__restrict__ w1, const T *__restrict__ w1t) {
+    extern __shared__ char smem_raw[];
+    T *y = reinterpret_cast<T *>(smem_raw);
+    __shared__ T red[NW * 64];
+    // the blocks with the most rows to gather and columns to read (the last
+    // ones of a node) take the lowest workgroup ids, so that they start first
+    const int id = (int)gridDim.x - 1 - xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const DiagItem it = items[id];
     const int tid = threadIdx.x, r = tid & 63, q = tid >> 6;
     const int nd = it.nd, r0 = it.ib * 64;
     const int fc = S.cblk_fcol[S.node_cblk[nd]];
@@ -134,10 +109,9 @@ __device__ __forceinline__ void fwd_diag_body(const DevSymbol &S, const DiagItem
     // the lanes' sums combined by xor shuffles in a fixed order.  With one
     // lane per row, consecutive lanes read consecutive rows' entries, which
     // the sliced update buffer keeps side by side.
-    const int tasks = nrow * nrhs;
     const int ne = ys.cnt[fc];
     int gl = 1;
-    while (gl < 64 && gl * 2 <= ne && tasks * gl * 2 <= NW * 64) gl *= 2;
+    while (gl < 64 && gl * 2 <= ne && nrow * gl * 2 <= NW * 64) gl *= 2;
     // rows of the inverse: E consecutive per lane (16-byte loads); the first
     // PF column groups are fetched before the gather, so that their latency
     // overlaps it
@@ -145,9 +119,9 @@ __device__ __forceinline__ void fwd_diag_body(const DevSymbol &S, const DiagItem
     const int rr = E * (r % G), kc = r / G;
     const bool mrow = r0 + rr < Kc;
     const T *M = w1 + S.node_winv[nd] + r0 + rr;
-    // one right-hand side with W^T at hand (LL^t): row i of W is read as
-    // column i of W^T (contiguous), NW lanes per row (row r0 + jt, lane lt)
-    const bool tw = NR == 1 && w1t != nullptr;
+    // with W^T at hand (LL^t): row i of W is read as column i of W^T
+    // (contiguous), NW lanes per row (row r0 + jt, lane lt)
+    const bool tw = w1t != nullptr;
     const int jt = tid / NW, lt = tid % NW, it_row = r0 + jt;
     const T *MT = tw ? w1t + S.node_winv[nd] + (int64_t)it_row * Kc : nullptr;
     T mpre[PF][E];
@@ -162,30 +136,22 @@ __device__ __forceinline__ void fwd_diag_body(const DevSymbol &S, const DiagItem
         }
     }
     constexpr int UL = 16;
-    if constexpr (PRE) {
-        // the rows' pending products were subtracted in b already (k_fwd_gather)
-        for (int t = tid; t < tasks; t += NW * 64) {
-            const int i = t % nrow, u = t / nrow;
-            y[i + u * Kc] = b[fc + i + u * ldb];
-        }
-    } else
-    for (int base = 0; base < tasks * gl; base += NW * 64) {
-        const int t = base + tid, task = t / gl, j = t % gl;
-        const int i = task % nrow, u = task / nrow;
+    for (int base = 0; base < nrow * gl; base += NW * 64) {
+        const int t = base + tid, i = t / gl, j = t % gl;
         T v = 0;
-        if (task < tasks) {
+        if (i < nrow) {
             const int g = fc + i, ne_i = ys.cnt[g];
-            const T *yb = ybuf + u * ldy + ys.base[g >> 6] + (g & 63);
+            const T *yb = ybuf + ys.base[g >> 6] + (g & 63);
             for (int e = j; e < ne_i; e += UL * gl) {
                 T a[UL];
 #pragma unroll
-                for (int k = 0; k < UL; k++) a[k] = (e + k * gl < ne_i) ? ld_co<CO>(yb + (int64_t)(e + k * gl) * 64) : (T)0;
+                for (int k = 0; k < UL; k++) a[k] = (e + k * gl < ne_i) ? yb[(int64_t)(e + k * gl) * 64] : (T)0;
 #pragma unroll
                 for (int k = 0; k < UL; k++) v += a[k];
             }
         }
         for (int o = gl >> 1; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-        if (task < tasks && j == 0) y[i + u * Kc] = b[fc + i + u * ldb] - v;
+        if (i < nrow && j == 0) y[i] = b[fc + i] - v;
     }
     __syncthreads();
     if (tw) {
@@ -215,28 +181,20 @@ __device__ __forceinline__ void fwd_diag_body(const DevSymbol &S, const DiagItem
         for (int e = 0; e < E; e++) v += a2[e];
 #pragma unroll
         for (int o = NW / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, NW);
-        if (lt == 0 && it_row < Kc) st_co<CO>(z + fc + it_row, v);
+        if (lt == 0 && it_row < Kc) z[fc + it_row] = v;
         return;  // uniform: tw is the same for the whole workgroup
     }
     const int i = r0 + r;
-    T acc[E][NR];
+    T acc[E];
 #pragma unroll
-    for (int e = 0; e < E; e++)
-#pragma unroll
-        for (int u = 0; u < NR; u++) acc[e][u] = 0;
+    for (int e = 0; e < E; e++) acc[e] = 0;
     if (mrow) {
 #pragma unroll
         for (int f = 0; f < PF; f++) {
             const int k = q * E + kc + f * NW * E;
             if (k < nrow) {
 #pragma unroll
-                for (int u = 0; u < NR; u++) {
-                    if (u < nrhs) {
-                        const T yv = y[k + u * Kc];
-#pragma unroll
-                        for (int e = 0; e < E; e++) acc[e][u] += mpre[f][e] * yv;
-                    }
-                }
+                for (int e = 0; e < E; e++) acc[e] += mpre[f][e] * y[k];
             }
         }
 #pragma unroll 4
@@ -244,40 +202,37 @@ __device__ __forceinline__ void fwd_diag_body(const DevSymbol &S, const DiagItem
             T m[E];
             ld_rows(M + (int64_t)k * Kc, rr, Kc - r0, m);
 #pragma unroll
-            for (int u = 0; u < NR; u++) {
-                if (u < nrhs) {
-                    const T yv = y[k + u * Kc];
-#pragma unroll
-                    for (int e = 0; e < E; e++) acc[e][u] += m[e] * yv;
-                }
-            }
+            for (int e = 0; e < E; e++) acc[e] += m[e] * y[k];
         }
     }
-    wave_sum_store_rows<CO, T, NR, NW, E>(acc, red, r, q, i < Kc, nrhs, z + fc + i, ldz);
+    wave_sum_store_rows<T, NW, E>(acc, red, r, q, i < Kc, z + fc + i);
 }
 
-template <bool CO, typename T, int NR, int NW>
-__device__ __forceinline__ void fwd_prod_body(const DevSymbol &S, const FwdItem it, const T *__restrict__ coef,
-                                              const T *__restrict__ z, int64_t ldz, int nrhs,
-                                              const int32_t *__restrict__ ydst, T *__restrict__ ybuf, int64_t ldy,
-                                              T *xs, T *red) {
+template <typename T, int NW>
+__global__ __launch_bounds__(NW * 64) void k_fwd_prod(DevSymbol S, const FwdItem *__restrict__ items, int nitems,
+                                                      const T *__restrict__ coef, const T *__restrict__ z,
+                                                      const int32_t *__restrict__ ydst, T *__restrict__ ybuf) {
+    extern __shared__ char smem_raw[];
+    T *xs = reinterpret_cast<T *>(smem_raw);
+    __shared__ T red[NW * 64];
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const FwdItem it = items[id];
     const int tid = threadIdx.x, r = tid & 63, q = tid >> 6;
     const int c = it.c;
     const int fc = S.cblk_fcol[c];
     const int Kc = S.cblk_fcol[c + 1] - fc;
     const int64_t ld = S.cblk_stride[c];
-    for (int t = tid; t < Kc * nrhs; t += NW * 64) xs[t] = ld_co<CO>(z + fc + (t % Kc) + (int64_t)(t / Kc) * ldz);
+    for (int t = tid; t < Kc; t += NW * 64) xs[t] = z[fc + t];
     __syncthreads();
     const int nr = it.r1 - it.r0;
     // E consecutive rows per lane (one 16-byte load), E columns per wave
     // instruction
     constexpr int E = Vec<T>::E, G = 64 / E;
     const int rr = E * (r % G), kc = r / G;
-    T acc[E][NR];
+    T acc[E];
 #pragma unroll
-    for (int i = 0; i < E; i++)
-#pragma unroll
-        for (int u = 0; u < NR; u++) acc[i][u] = 0;
+    for (int i = 0; i < E; i++) acc[i] = 0;
     if (rr < nr) {
         const T *rows = coef + S.cblk_coef[c] + it.r0 + rr;
 #pragma unroll 2
@@ -285,40 +240,39 @@ __device__ __forceinline__ void fwd_prod_body(const DevSymbol &S, const FwdItem 
             T a[E];
             ld_rows(rows + (int64_t)k * ld, rr, nr, a);
 #pragma unroll
-            for (int u = 0; u < NR; u++) {
-                if (u < nrhs) {
-                    const T xv = xs[k + u * Kc];
-#pragma unroll
-                    for (int i = 0; i < E; i++) acc[i][u] += a[i] * xv;
-                }
-            }
+            for (int i = 0; i < E; i++) acc[i] += a[i] * xs[k];
         }
     }
     const int dst = (r < nr) ? ydst[it.slot + r] : 0;
-    wave_sum_store_rows<CO, T, NR, NW, E>(acc, red, r, q, r < nr, nrhs, ybuf + dst, ldy);
+    wave_sum_store_rows<T, NW, E>(acc, red, r, q, r < nr, ybuf + dst);
 }
 
 // one strip (panel rows [r0, r1), any multiple of 64 of them, column block
-// k0/64) of the backward products, 4 waves: partial[j] = sum over the strip's
-// rows of L[r, k0+j] x[row(r)], 64 rows at a time, the next chunk's loads in
-// flight while the current one is summed.  nrhs right-hand sides starting at
-// column u0 of the partials (laid out for nrhs_tot columns); x points at
-// column u0 already
-template <bool CO, typename T, int NR>
-__device__ __forceinline__ void bwd_prod_body(const DevSymbol &S, const BwdItem it, int k0,
-                                              const T *__restrict__ coef, const T *__restrict__ x, int64_t ldx,
-                                              int nrhs, int nrhs_tot, int u0, T *__restrict__ part, T (*tile)[65],
-                                              T *xr, T *red) {
-    const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
+// blockIdx.y) of the backward products, 4 waves: partial[j] = sum over the
+// strip's rows of L[r, k0+j] x[row(r)], 64 rows at a time, the next chunk's
+// loads in flight while the current one is summed
+template <typename T>
+__global__ __launch_bounds__(256) void k_bwd_prod(DevSymbol S, const BwdItem *__restrict__ items, int nitems,
+                                                  const T *__restrict__ coef, const T *__restrict__ x,
+                                                  T *__restrict__ part) {
+    __shared__ T tile[64][65];
+    __shared__ T xr[64];
+    __shared__ T red[256];
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const BwdItem it = items[id];
+    const int k0 = blockIdx.y * 64;
     const int c = it.c;
     const int Kc = S.cblk_fcol[c + 1] - S.cblk_fcol[c];
+    if (k0 >= Kc) return;
+    const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
     const int64_t ld = S.cblk_stride[c];
     const int64_t rb = S.cblk_rowbase[c];
     // E consecutive rows per lane (one 16-byte load), 4E columns per pass
     constexpr int E = Vec<T>::E, G = 64 / E, NP = 64 / (4 * E);
     const int rr = E * (lane % G), kc = lane / G;
     const T *P = coef + S.cblk_coef[c];
-    T a[NP][E], xv[NR];
+    T a[NP][E], xv = 0;
     auto gload = [&](int r0) {
         const int nr = min(64, it.r1 - r0);
 #pragma unroll
@@ -326,15 +280,9 @@ __device__ __forceinline__ void bwd_prod_body(const DevSymbol &S, const BwdItem 
             const int cc = q * E + kc + 4 * E * u;
             ld_rows(P + r0 + rr + (int64_t)(k0 + cc) * ld, rr, (k0 + cc < Kc) ? nr : 0, a[u]);
         }
-        if (tid < 64) {
-#pragma unroll
-            for (int v = 0; v < NR; v++)
-                xv[v] = (tid < nr && v < nrhs) ? ld_co<CO>(x + S.panel_grow[rb + r0 + tid] + v * ldx) : (T)0;
-        }
+        if (tid < 64) xv = (tid < nr) ? x[S.panel_grow[rb + r0 + tid]] : (T)0;
     };
-    T acc[NR];
-#pragma unroll
-    for (int u = 0; u < NR; u++) acc[u] = 0;
+    T acc = 0;
     gload(it.r0);
     for (int r0 = it.r0; r0 < it.r1; r0 += 64) {
         // the chunk in registers goes to LDS, the next one is fetched
@@ -344,130 +292,63 @@ __device__ __forceinline__ void bwd_prod_body(const DevSymbol &S, const BwdItem 
 #pragma unroll
             for (int i = 0; i < E; i++) tile[rr + i][cc] = a[u][i];
         }
-        if (tid < 64) {
-#pragma unroll
-            for (int v = 0; v < NR; v++) xr[tid + v * 64] = xv[v];
-        }
+        if (tid < 64) xr[tid] = xv;
         __syncthreads();
         if (r0 + 64 < it.r1) gload(r0 + 64);
 #pragma unroll 4
-        for (int row = q * 16; row < q * 16 + 16; row++) {
-            const T t = tile[row][lane];
-#pragma unroll
-            for (int u = 0; u < NR; u++) acc[u] += t * xr[row + u * 64];
-        }
+        for (int row = q * 16; row < q * 16 + 16; row++) acc += tile[row][lane] * xr[row];
         __syncthreads();
     }
-    T *out = part + (int64_t)it.slot * nrhs_tot + (int64_t)u0 * Kc + k0 + lane;
-    wave_sum_store<CO, T, NR, 4>(acc, red, lane, q, k0 + lane < Kc, nrhs, out, Kc, (const T *)nullptr, 0);
+    wave_sum_store<T, 4>(acc, red, lane, q, k0 + lane < Kc, part + (int64_t)it.slot + k0 + lane);
 }
 
-// nrhs right-hand sides starting at column u0 of the partials, which are laid
-// out for nrhs_tot columns (z and x point at column u0 already)
-template <bool CO, typename T, int NR, int NW, bool PRE = false>
-__device__ __forceinline__ void bwd_diag_body(const DevSymbol &S, const DiagItem it,
-                                              const BwdItem *__restrict__ bitems, const T *__restrict__ z,
-                                              int64_t ldz, T *__restrict__ x, int64_t ldx, int nrhs, int nrhs_tot,
-                                              int u0, const T *__restrict__ part, const T *__restrict__ wb, T *y,
-                                              T *red) {
+template <typename T, int NW>
+__global__ __launch_bounds__(NW * 64) void k_bwd_diag(DevSymbol S, const DiagItem *__restrict__ items, int nitems,
+                                                      const BwdItem *__restrict__ bitems, const T *__restrict__ z,
+                                                      T *__restrict__ x, const T *__restrict__ part,
+                                                      const T *__restrict__ wb) {
+    extern __shared__ char smem_raw[];
+    T *y = reinterpret_cast<T *>(smem_raw);
+    __shared__ T red[NW * 64];
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const DiagItem it = items[id];
     const int tid = threadIdx.x, r = tid & 63, q = tid >> 6;
     const int nd = it.nd, r0 = it.ib * 64;
     const int cb0 = S.node_cblk[nd], cb1 = S.node_cblk[nd + 1];
     const int fc = S.cblk_fcol[cb0];
     const int Kc = S.cblk_fcol[cb1] - fc;
+    // y = z_c - the strips' partials for columns [r0, Kc): all columns at
+    // once (cpp per pass), each summed over every L-th strip by L threads,
+    // whose sums are then added in thread order; one barrier pair per pass.
     // Column k of the node belongs to member cblk m (column k - o of it, o
     // = fcol[m] - fc); m's strips [tb, te) own consecutive partial slots, w
-    // apart, the first at bitems[tb].slot.  pcol returns the address of the
-    // partial of right-hand side 0 in m's first strip; the strips follow at
-    // stride w * nrhs_tot.
-    auto pcol = [&](int k, int &tb, int &te, int64_t &stride) -> const T * {
-        int lo = cb0, hi = cb1 - 1;  // the last member whose first column is <= k
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (S.cblk_fcol[mid] - fc <= k) lo = mid;
-            else hi = mid - 1;
-        }
-        const int o = S.cblk_fcol[lo] - fc, w = S.cblk_fcol[lo + 1] - S.cblk_fcol[lo];
-        tb = S.cblk_btile[2 * lo];
-        te = S.cblk_btile[2 * lo + 1];
-        stride = (int64_t)w * nrhs_tot;
-        const int64_t s0 = (te > tb) ? (int64_t)bitems[tb].slot : 0;
-        return part + s0 * nrhs_tot + (int64_t)u0 * w + (k - o);
-    };
-    if constexpr (PRE) {
-        // the partials were subtracted from z already (k_bwd_reduce)
-        for (int t = tid; t < (Kc - r0) * nrhs; t += NW * 64) {
-            const int k = r0 + t % (Kc - r0), u = t / (Kc - r0);
-            y[k + u * Kc] = z[fc + k + u * ldz];
-        }
-        __syncthreads();
-    }
-    // y = z_c - the tiles' partials for columns [r0, Kc).  Several
-    // right-hand sides: 64 columns at a time, the waves splitting the tiles.
-    if constexpr (NR > 1 && !PRE) {
-        for (int kc = r0; kc < Kc; kc += 64) {
-            const int k = kc + r;
-            T acc[NR];
-#pragma unroll
-            for (int u = 0; u < NR; u++) acc[u] = 0;
-            if (k < Kc) {
-                int tb, te;
-                int64_t stride;
-                const T *p0 = pcol(k, tb, te, stride);
-                const int w = (int)(stride / nrhs_tot);
-#pragma unroll 4
-                for (int j = tb + q; j < te; j += NW) {
-                    const T *pp = p0 + (int64_t)(j - tb) * stride;
-#pragma unroll
-                    for (int u = 0; u < NR; u++)
-                        if (u < nrhs) acc[u] += ld_co<CO>(pp + u * w);
-                }
-            }
-            // y lives in LDS: a plain store; z comes from other tasks
-            wave_sum_store<CO, T, NR, NW>(acc, red, r, q, k < Kc, nrhs, y + k, Kc, z + fc + k, ldz);
-            __syncthreads();
-        }
-    }
-    // One right-hand side: all columns at once (cpp per pass), each summed
-    // over every L-th tile by L threads, whose sums are then added in thread
-    // order; one barrier pair per pass instead of one per 64 columns.
-    const int ncol = (NR > 1 || PRE) ? 0 : Kc - r0;
+    // apart, the first at bitems[tb].slot.
+    const int ncol = Kc - r0;
     const int cpp = max(1, min(ncol, NW * 64)), L = (NW * 64) / cpp;
     for (int c0 = 0; c0 < ncol; c0 += cpp) {
         const int cc = tid % cpp, h = tid / cpp;
         const int k = r0 + c0 + cc;
-        const bool live = h < L && c0 + cc < ncol;
-        T acc[NR];
-#pragma unroll
-        for (int u = 0; u < NR; u++) acc[u] = 0;
-        if (live) {
-            int tb, te;
-            int64_t stride;
-            const T *p0 = pcol(k, tb, te, stride);
-            const int w = (int)(stride / nrhs_tot);
-#pragma unroll 4
-            for (int j = tb + h; j < te; j += L) {
-                const T *pp = p0 + (int64_t)(j - tb) * stride;
-#pragma unroll
-                for (int u = 0; u < NR; u++)
-                    if (u < nrhs) acc[u] += ld_co<CO>(pp + u * w);
+        T acc = 0;
+        if (h < L && c0 + cc < ncol) {
+            int lo = cb0, hi = cb1 - 1;  // the last member whose first column is <= k
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (S.cblk_fcol[mid] - fc <= k) lo = mid;
+                else hi = mid - 1;
             }
+            const int o = S.cblk_fcol[lo] - fc, w = S.cblk_fcol[lo + 1] - S.cblk_fcol[lo];
+            const int tb = S.cblk_btile[2 * lo], te = S.cblk_btile[2 * lo + 1];
+            const T *p0 = part + ((te > tb) ? (int64_t)bitems[tb].slot : 0) + (k - o);
+#pragma unroll 4
+            for (int j = tb + h; j < te; j += L) acc += p0[(int64_t)(j - tb) * w];
         }
-        if (h < L) {
-#pragma unroll
-            for (int u = 0; u < NR; u++) red[(h * cpp + cc) * NR + u] = acc[u];
-        }
+        if (h < L) red[h * cpp + cc] = acc;
         __syncthreads();
         if (h == 0 && c0 + cc < ncol) {
-#pragma unroll
-            for (int u = 0; u < NR; u++) {
-                if (u < nrhs) {
-                    T v = red[cc * NR + u];
-                    for (int w = 1; w < L; w++) v += red[(w * cpp + cc) * NR + u];
-                    // y lives in LDS: a plain store; z comes from other tasks
-                    y[k + u * Kc] = ld_co<CO>(z + fc + k + u * ldz) - v;
-                }
-            }
+            T v = red[cc];
+            for (int w = 1; w < L; w++) v += red[w * cpp + cc];
+            y[k] = z[fc + k] - v;
         }
         __syncthreads();
     }
@@ -475,11 +356,9 @@ __device__ __forceinline__ void bwd_diag_body(const DevSymbol &S, const DiagItem
     // rows of the inverse: E consecutive per lane (16-byte loads)
     constexpr int E = Vec<T>::E, G = 64 / E;
     const int rr = E * (r % G), kc = r / G;
-    T acc2[E][NR];
+    T acc2[E];
 #pragma unroll
-    for (int e = 0; e < E; e++)
-#pragma unroll
-        for (int u = 0; u < NR; u++) acc2[e][u] = 0;
+    for (int e = 0; e < E; e++) acc2[e] = 0;
     if (r0 + rr < Kc) {
         // wb holds inv(L_cc)^T (or inv(U_cc)) column-major: upper triangular
         const T *M = wb + S.node_winv[nd] + r0 + rr;
@@ -488,68 +367,10 @@ __device__ __forceinline__ void bwd_diag_body(const DevSymbol &S, const DiagItem
             T m[E];
             ld_rows(M + (int64_t)k * Kc, rr, Kc - r0, m);
 #pragma unroll
-            for (int u = 0; u < NR; u++) {
-                if (u < nrhs) {
-                    const T yv = y[k + u * Kc];
-#pragma unroll
-                    for (int e = 0; e < E; e++) acc2[e][u] += m[e] * yv;
-                }
-            }
+            for (int e = 0; e < E; e++) acc2[e] += m[e] * y[k];
         }
     }
-    wave_sum_store_rows<CO, T, NR, NW, E>(acc2, red, r, q, i < Kc, nrhs, x + fc + i, ldx);
-}
-
-// ------------------------------ level kernels -------------------------------
-template <typename T, int NR, int NW, bool PRE = false>
-__global__ __launch_bounds__(NW * 64) void k_fwd_diag(DevSymbol S, const DiagItem *__restrict__ items, int nitems,
-                                                      const YSlices ys, const T *__restrict__ ybuf, int64_t ldy,
-                                                      const T *__restrict__ b, int64_t ldb, T *__restrict__ z,
-                                                      int64_t ldz, int nrhs, const T *__restrict__ w1,
-                                                      const T *__restrict__ w1t) {
-    extern __shared__ char smem_raw[];
-    __shared__ T red[NW * 64 * NR];
-    // the blocks with the most rows to gather and columns to read (the last
-    // ones of a node) take the lowest workgroup ids, so that they start first
-    const int id = (int)gridDim.x - 1 - xcd_remap(blockIdx.x, gridDim.x);
-    if (id >= nitems) return;
-    // right-hand sides [NR*blockIdx.y, NR*blockIdx.y + NR)
-    const int u0 = NR * blockIdx.y;
-    fwd_diag_body<false, T, NR, NW, PRE>(S, items[id], ys, ybuf + u0 * ldy, ldy, b + u0 * ldb, ldb, z + u0 * ldz,
-                                    ldz, min(NR, nrhs - u0), w1, w1t, reinterpret_cast<T *>(smem_raw), red);
-}
-
-template <typename T, int NR, int NW>
-__global__ __launch_bounds__(NW * 64) void k_fwd_prod(DevSymbol S, const FwdItem *__restrict__ items, int nitems,
-                                                      const T *__restrict__ coef, const T *__restrict__ z,
-                                                      int64_t ldz, int nrhs, const int32_t *__restrict__ ydst,
-                                                      T *__restrict__ ybuf, int64_t ldy) {
-    extern __shared__ char smem_raw[];
-    __shared__ T red[NW * 64 * NR];
-    const int id = xcd_remap(blockIdx.x, gridDim.x);
-    if (id >= nitems) return;
-    // right-hand sides [NR*blockIdx.y, NR*blockIdx.y + NR)
-    const int u0 = NR * blockIdx.y;
-    fwd_prod_body<false, T, NR, NW>(S, items[id], coef, z + u0 * ldz, ldz, min(NR, nrhs - u0), ydst, ybuf + u0 * ldy,
-                                    ldy, reinterpret_cast<T *>(smem_raw), red);
-}
-
-template <typename T, int NR>
-__global__ __launch_bounds__(256) void k_bwd_prod(DevSymbol S, const BwdItem *__restrict__ items, int nitems,
-                                                  const T *__restrict__ coef, const T *__restrict__ x, int64_t ldx,
-                                                  int nrhs, T *__restrict__ part) {
-    __shared__ T tile[64][65];
-    __shared__ T xr[64 * NR];
-    __shared__ T red[256 * NR];
-    const int id = xcd_remap(blockIdx.x, gridDim.x);
-    if (id >= nitems) return;
-    const BwdItem it = items[id];
-    const int k0 = blockIdx.y * 64;
-    if (k0 >= S.cblk_fcol[it.c + 1] - S.cblk_fcol[it.c]) return;
-    // right-hand sides [NR*blockIdx.z, NR*blockIdx.z + NR)
-    const int u0 = NR * blockIdx.z;
-    bwd_prod_body<false, T, NR>(S, it, k0, coef, x + u0 * ldx, ldx, min(NR, nrhs - u0), nrhs, u0, part, tile, xr,
-                                red);
+    wave_sum_store_rows<T, NW, E>(acc2, red, r, q, i < Kc, x + fc + i);
 }
 
 // Backward strips of narrow cblks (at most C columns), one right-hand side:
@@ -591,22 +412,6 @@ __global__ __launch_bounds__(64) void k_bwd_prod_narrow(DevSymbol S, const BwdIt
     for (int k = 0; k < C; k++)
         if ((k & 15) == l && k < Kc) part[(int64_t)it.slot + k] = acc[k];
 }
-
-template <typename T, int NR, int NW, bool PRE = false>
-__global__ __launch_bounds__(NW * 64) void k_bwd_diag(DevSymbol S, const DiagItem *__restrict__ items, int nitems,
-                                                      const BwdItem *__restrict__ bitems, const T *__restrict__ z,
-                                                      int64_t ldz, T *__restrict__ x, int64_t ldx, int nrhs,
-                                                      const T *__restrict__ part, const T *__restrict__ wb) {
-    extern __shared__ char smem_raw[];
-    __shared__ T red[NW * 64 * NR];
-    const int id = xcd_remap(blockIdx.x, gridDim.x);
-    if (id >= nitems) return;
-    // right-hand sides [NR*blockIdx.y, NR*blockIdx.y + NR)
-    const int u0 = NR * blockIdx.y;
-    bwd_diag_body<false, T, NR, NW, PRE>(S, items[id], bitems, z + u0 * ldz, ldz, x + u0 * ldx, ldx, min(NR, nrhs - u0),
-                                    nrhs, u0, part, wb, reinterpret_cast<T *>(smem_raw), red);
-}
-
 
 // Levels of wide nodes (more than SOLVE_SPLIT columns): the gathers run once
 // per 64-row block in a launch of their own instead of in every diagonal
@@ -876,122 +681,536 @@ __global__ __launch_bounds__(64) void k_bwd_diag_tiny(DevSymbol S, const DiagIte
     if (col) x[fc + k] = acc;
 }
 
+// ---------------------------------------------------------------------------
+// Several right-hand sides: the same sweeps as products on the matrix cores,
+// sixteen right-hand sides to an MFMA block and NB blocks to a workgroup, so
+// that the factor crosses once for up to 16 NB of them.  Bound by the levels'
+// memory latency (a 53x47x50 factor is 0.46 GB).  The vector kernels these
+// replace took two (diagonal steps) or eight columns at a time and read the
+// factor again for the next ones: 53x47x50 FP64, 2 columns 1165 -> 847 us, 8
+// 1484 -> 917, 32 3212 -> 1305; FP32 867 -> 601, 1154 -> 655, 2477 -> 904.
+// Products are formed
+// transposed, D(u, row) = sum_k Y(k, u) M(row, k): a lane's results of one
+// MFMA register belong to one right-hand side, so sixteen lanes store
+// consecutive rows.  Rows and right-hand sides that do not exist repeat an
+// existing one (their results are not stored); inner indices beyond the last
+// count as zero on both operands.
+// ---------------------------------------------------------------------------
+
+// Forward products: 64 panel rows x K columns of cblk c times z_c.  Lanes
+// read E consecutive rows of a column (16 bytes); a wave covers 16 E rows,
+// the remaining split of the four waves goes over the columns (KS ways,
+// combined through LDS in a fixed order).  z_c is staged KC columns at a time.
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_fwd_prod_m(DevSymbol S, const FwdItem *__restrict__ items, int nitems,
+                                                    const T *__restrict__ coef, const T *__restrict__ z, int64_t ldz,
+                                                    int nrhs, const int32_t *__restrict__ ydst,
+                                                    T *__restrict__ ybuf, int64_t ldy) {
+    constexpr int E = Vec<T>::E, WR = 4 / E, KS = 4 / WR, KC = 128, NC = 16 * NB, ZP = KC + 2;
+    constexpr int ZN = NC * ZP, RN = KS * NC * 64;
+    __shared__ T lds[ZN > RN ? ZN : RN];
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const FwdItem it = items[id];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, kq = lane >> 4, wr = wave % WR, ks = wave / WR;
+    const int u0 = NC * blockIdx.y, nu = min(NC, nrhs - u0);
+    const int fc = S.cblk_fcol[it.c], K = S.cblk_fcol[it.c + 1] - fc;
+    const int64_t ld = S.cblk_stride[it.c];
+    const int nr = it.r1 - it.r0, row = 16 * E * wr + E * i;
+    const T *P = coef + S.cblk_coef[it.c] + it.r0 + (row < nr ? row : 0);
+    typename Mfma<T>::v4 acc[E][NB];
+#pragma unroll
+    for (int e = 0; e < E; e++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[e][b] = {0, 0, 0, 0};
+    // thread (k, group) stages right-hand sides group, group + 2, ... of
+    // column k of the chunk; the next chunk's are in flight during the MFMAs
+    const int zk = tid & (KC - 1), zu = tid / KC;
+    T v[NC / 2];
+    auto zload = [&](int kc) {
+        const T *q = z + fc + min(kc + zk, K - 1) + (int64_t)u0 * ldz;
+#pragma unroll
+        for (int t = 0; t < NC / 2; t++) v[t] = q[(int64_t)min(zu + 2 * t, nu - 1) * ldz];
+    };
+    zload(0);
+    for (int kc = 0; kc < K; kc += KC) {
+        const int kn = min(KC, K - kc);
+        if (kc > 0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < NC / 2; t++) lds[(zu + 2 * t) * ZP + zk] = (zk < kn) ? v[t] : (T)0;
+        __syncthreads();
+        if (kc + KC < K) zload(kc + KC);
+        // four steps' factor loads together, then their MFMAs
+        for (int s0 = 4 * ks; s0 < kn; s0 += 16 * KS) {
+            T m[4][E];
+#pragma unroll
+            for (int j = 0; j < 4; j++) ld_vec(P + (int64_t)(kc + min(s0 + 4 * KS * j + kq, kn - 1)) * ld, m[j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int s = s0 + 4 * KS * j, k = s + kq;
+                if (s >= kn) break;  // uniform
+#pragma unroll
+                for (int e = 0; e < E; e++) m[j][e] = (k < kn) ? m[j][e] : (T)0;
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    const T a = lds[(16 * b + i) * ZP + k];
+#pragma unroll
+                    for (int e = 0; e < E; e++) acc[e][b] = Mfma<T>::mma(a, m[j][e], acc[e][b]);
+                }
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; e++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                lds[(ks * NC + 16 * b + Mfma<T>::drow(lane, r)) * 64 + row + e] = acc[e][b][r];
+    __syncthreads();
+    const int rl = tid & 63;
+    if (rl < nr) {
+        T *out = ybuf + ydst[it.slot + rl] + (int64_t)u0 * ldy;
+        for (int u = tid >> 6; u < nu; u += 4) {
+            T v = lds[u * 64 + rl];
+#pragma unroll
+            for (int q = 1; q < KS; q++) v += lds[(q * NC + u) * 64 + rl];
+            out[(int64_t)u * ldy] = v;
+        }
+    }
+}
+
+// Backward products: columns [k0, k0 + 16 WC) of cblk c, panel rows of one
+// strip: partial(u, j) = sum_r L(r, j) x(row(r), u).  A lane reads E
+// consecutive rows of its column (16 bytes, four lanes to a column); a wave
+// takes 16 columns, the waves left over (4 / WC ways, levels of narrow cblks)
+// split the rows and combine through LDS in a fixed order.  x is gathered 64
+// rows at a time.
+template <typename T, int NB, int WC>
+__global__ __launch_bounds__(256) void k_bwd_prod_m(DevSymbol S, const BwdItem *__restrict__ items, int nitems,
+                                                    const T *__restrict__ coef, const T *__restrict__ x, int64_t ldx,
+                                                    int nrhs, T *__restrict__ part) {
+    constexpr int E = Vec<T>::E, RS = 4 / WC, NC = 16 * NB, XP = 64 + E, RR = 64 / RS, NG = RR / (4 * E);
+    constexpr int XN = NC * XP, RN = RS > 1 ? RS * WC * 16 * NC : 0;
+    __shared__ T lds[XN > RN ? XN : RN];
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const BwdItem it = items[id];
+    const int fc = S.cblk_fcol[it.c], K = S.cblk_fcol[it.c + 1] - fc;
+    const int k0 = blockIdx.y * 16 * WC;
+    if (k0 >= K) return;  // uniform: the whole workgroup leaves
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, kq = lane >> 4, wc = wave % WC, rs = wave / WC;
+    const int u0 = NC * blockIdx.z, nu = min(NC, nrhs - u0);
+    const int64_t ld = S.cblk_stride[it.c];
+    const int32_t *grow = S.panel_grow + S.cblk_rowbase[it.c];
+    const bool live = k0 + 16 * wc < K;
+    const int col = k0 + 16 * wc + i;
+    const T *P = coef + S.cblk_coef[it.c] + (int64_t)min(col, K - 1) * ld;
+    typename Mfma<T>::v4 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[b] = {0, 0, 0, 0};
+    // thread (row, group) gathers right-hand sides group, group + 4, ... of
+    // its row of the chunk; the next chunk's are in flight during the MFMAs
+    const int xr = tid & 63, xu = tid >> 6;
+    T v[NC / 4];
+    int gr = grow[min(it.r0 + xr, it.r1 - 1)];
+    auto xload = [&]() {
+        const T *xg = x + gr + (int64_t)u0 * ldx;
+#pragma unroll
+        for (int t = 0; t < NC / 4; t++) v[t] = xg[(int64_t)min(xu + 4 * t, nu - 1) * ldx];
+    };
+    xload();
+    for (int r0 = it.r0; r0 < it.r1; r0 += 64) {
+        const int rn = min(64, it.r1 - r0);
+        const bool more = r0 + 64 < it.r1;
+        if (more) gr = grow[min(r0 + 64 + xr, it.r1 - 1)];
+        T m[NG][E];
+        if (live) {
+#pragma unroll
+            for (int g = 0; g < NG; g++) {
+                const int r = RR * rs + 4 * E * g + E * kq;
+                ld_vec(P + r0 + (r < rn ? r : 0), m[g]);
+            }
+        }
+        if (r0 > it.r0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < NC / 4; t++) lds[(xu + 4 * t) * XP + xr] = (xr < rn) ? v[t] : (T)0;
+        __syncthreads();
+        if (more) xload();
+        if (live) {
+#pragma unroll
+            for (int g = 0; g < NG; g++) {
+#pragma unroll
+                for (int e = 0; e < E; e++) m[g][e] = (RR * rs + 4 * E * g + E * kq + e < rn) ? m[g][e] : (T)0;
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    const T *a = &lds[(16 * b + i) * XP + RR * rs + 4 * E * g + E * kq];
+#pragma unroll
+                    for (int e = 0; e < E; e++) acc[b] = Mfma<T>::mma(a[e], m[g][e], acc[b]);
+                }
+            }
+        }
+    }
+    T *out = part + (int64_t)it.slot * nrhs + (int64_t)u0 * K;
+    if constexpr (RS == 1) {
+        if (col < K) {
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int u = 16 * b + Mfma<T>::drow(lane, r);
+                    if (u < nu) out[(int64_t)u * K + col] = acc[b][r];
+                }
+        }
+    } else {
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                lds[(rs * NC + 16 * b + Mfma<T>::drow(lane, r)) * (16 * WC) + 16 * wc + i] = acc[b][r];
+        __syncthreads();
+        for (int t = tid; t < 16 * WC * NC; t += 256) {
+            const int j = t % (16 * WC), u = t / (16 * WC);
+            if (k0 + j < K && u < nu) {
+                T w = lds[t];
+#pragma unroll
+                for (int q = 1; q < RS; q++) w += lds[q * NC * 16 * WC + t];
+                out[(int64_t)u * K + k0 + j] = w;
+            }
+        }
+    }
+}
+
+// Diagonal steps of nodes of at most 16 W columns: one workgroup of W waves
+// per node, 16 rows of the node's inverse to a wave (read into registers
+// before the gather), Y staged in LDS.  Forward (UPPER false): Y = b minus the
+// rows' update-buffer entries, z = W Y; backward: Y = z minus the strips'
+// partials, x = WB Y.
+template <typename T, int NB, int W, bool UPPER>
+__global__ __launch_bounds__(64 * W) void k_diag_narrow_m(DevSymbol S, const DiagItem *__restrict__ items, int nitems,
+                                                          const YSlices ys, const BwdItem *__restrict__ bitems,
+                                                          const T *__restrict__ pend, int64_t ldp,
+                                                          const T *__restrict__ src, int64_t lds_, T *__restrict__ dst,
+                                                          int64_t ldd, int nrhs, const T *__restrict__ inv) {
+    constexpr int NC = 16 * NB, KM = 16 * W, YP = KM + 2;
+    __shared__ T y[NC][YP];
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, kq = lane >> 4;
+    const int u0 = NC * blockIdx.y, nu = min(NC, nrhs - u0);
+    const int nd = items[id].nd, cb0 = S.node_cblk[nd], cb1 = S.node_cblk[nd + 1];
+    const int fc = S.cblk_fcol[cb0], K = S.cblk_fcol[cb1] - fc;
+    // this wave's rows of the inverse, the nonzero side of the diagonal
+    const int ro = 16 * wave;
+    const int s0 = UPPER ? 4 * wave : 0, s1 = UPPER ? 4 * W : 4 * wave + 4;
+    const T *M = inv + S.node_winv[nd] + min(ro + i, K - 1);
+    T m[4 * W];
+#pragma unroll
+    for (int s = 0; s < 4 * W; s++) {
+        const int k = 4 * s + kq;
+        m[s] = (s >= s0 && s < s1 && k < K) ? M[(int64_t)k * K] : (T)0;
+    }
+    // Y: thread (row, group) takes right-hand sides group, group + 4, ...
+    const int row = tid % KM, ug = tid / KM;
+    T v[NC / 4];
+#pragma unroll
+    for (int t = 0; t < NC / 4; t++) v[t] = 0;
+    if (row < K) {
+        int ne;
+        int64_t step, ldu;
+        const T *p;
+        if constexpr (!UPPER) {
+            const int g = fc + row;
+            ne = ys.cnt[g];
+            step = 64;
+            ldu = ldp;
+            p = pend + ys.base[g >> 6] + (g & 63) + (int64_t)u0 * ldp;
+        } else {
+            // member of the column, its strips' partials
+            int c = cb0;
+            while (c + 1 < cb1 && S.cblk_fcol[c + 1] - fc <= row) c++;
+            const int o = S.cblk_fcol[c] - fc, w = S.cblk_fcol[c + 1] - S.cblk_fcol[c];
+            const int tb = S.cblk_btile[2 * c];
+            ne = S.cblk_btile[2 * c + 1] - tb;
+            step = (int64_t)w * nrhs;
+            ldu = w;
+            p = pend + (ne > 0 ? (int64_t)bitems[tb].slot * nrhs : 0) + (int64_t)u0 * w + (row - o);
+        }
+        const T *q = src + fc + row + (int64_t)u0 * lds_;
+        T b[NC / 4];
+#pragma unroll
+        for (int t = 0; t < NC / 4; t++) b[t] = (ug + 4 * t < nu) ? q[(int64_t)(ug + 4 * t) * lds_] : (T)0;
+        // two entries' loads together, added in order (a right-hand side
+        // beyond the last repeats it: its sum is not used)
+        for (int e = 0; e < ne; e += 2) {
+            T a0[NC / 4], a1[NC / 4];
+            const T *p0 = p + (int64_t)e * step, *p1 = p + (int64_t)min(e + 1, ne - 1) * step;
+#pragma unroll
+            for (int t = 0; t < NC / 4; t++) {
+                const int64_t uo = (int64_t)min(ug + 4 * t, nu - 1) * ldu;
+                a0[t] = p0[uo];
+                a1[t] = p1[uo];
+            }
+#pragma unroll
+            for (int t = 0; t < NC / 4; t++) {
+                v[t] += a0[t];
+                v[t] += (e + 1 < ne) ? a1[t] : (T)0;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < NC / 4; t++) v[t] = (ug + 4 * t < nu) ? b[t] - v[t] : (T)0;
+    }
+#pragma unroll
+    for (int t = 0; t < NC / 4; t++) y[ug + 4 * t][row] = v[t];
+    __syncthreads();
+    if (ro >= K) return;
+    typename Mfma<T>::v4 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[b] = {0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4 * W; s++) {
+        if (s >= s0 && s < s1) {  // uniform in the wave
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[b] = Mfma<T>::mma(y[16 * b + i][4 * s + kq], m[s], acc[b]);
+        }
+    }
+    if (ro + i < K) {
+        T *out = dst + fc + ro + i + (int64_t)u0 * ldd;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int u = 16 * b + Mfma<T>::drow(lane, r);
+                if (u < nu) out[(int64_t)u * ldd] = acc[b][r];
+            }
+    }
+}
+
+// Diagonal steps of wider nodes, after the gathers (k_fwd_gather,
+// k_bwd_reduce): 16 rows x 16 right-hand sides to a workgroup (four per
+// 64-row item), the waves splitting the inner index and combining through
+// LDS in wave order.  Forward: z = W y over columns [0, r + 16); backward
+// (UPPER): x = WB y over [r, K).  TR: the matrix is given transposed (row i
+// at w[i*K ...], one contiguous run), else column-major.
+template <typename T, bool UPPER, bool TR>
+__global__ __launch_bounds__(256) void k_diag_gemm16(DevSymbol S, const DiagItem *__restrict__ items, int nitems,
+                                                     const T *__restrict__ src, int64_t lds_, T *__restrict__ dst,
+                                                     int64_t ldd, int nrhs, const T *__restrict__ w) {
+    constexpr int E = Vec<T>::E, G = 4 * E;
+    __shared__ T red[4][16][17];
+    // forward: the blocks with the most columns (the last rows of a node)
+    // take the lowest workgroup ids, so that they start first
+    const int g0 = xcd_remap(blockIdx.x, gridDim.x);
+    const int gid = UPPER ? g0 : (int)gridDim.x - 1 - g0;
+    const int id = gid >> 2, sub = gid & 3;
+    if (id >= nitems) return;
+    const DiagItem it = items[id];
+    const int fc = S.cblk_fcol[S.node_cblk[it.nd]];
+    const int K = S.cblk_fcol[S.node_cblk[it.nd + 1]] - fc;
+    const int r = it.ib * 64 + sub * 16;
+    if (r >= K) return;  // uniform: the whole workgroup leaves
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, kq = lane >> 4;
+    const int u0 = 16 * blockIdx.y, nu = min(16, nrhs - u0);
+    const int k0 = UPPER ? r : 0, k1 = UPPER ? K : min(K, r + 16);
+    const T *Y = src + fc + (int64_t)(u0 + min(i, nu - 1)) * lds_;
+    const int64_t mi = min(r + i, K - 1);
+    const T *M = w + S.node_winv[it.nd] + (TR ? mi * K : mi);
+    typename Mfma<T>::v4 acc = {0, 0, 0, 0};
+    constexpr int U = 4;  // groups of G inner indices whose loads go out together
+    for (int kb0 = k0 + G * wave; kb0 < k1; kb0 += 4 * U * G) {
+        T a[U][E], m[U][E];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int kb = kb0 + 4 * G * j, k = kb + E * kq;
+            if (kb >= k1) break;  // uniform
+            if (kb + G <= k1) {
+                ld_vec(Y + k, a[j]);
+                if constexpr (TR) ld_vec(M + k, m[j]);
+                else {
+#pragma unroll
+                    for (int e = 0; e < E; e++) m[j][e] = M[(int64_t)(k + e) * K];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    const bool ok = k + e < k1;
+                    const int64_t ke = min(k + e, k1 - 1);
+                    const T av = Y[ke], mv = M[TR ? ke : ke * K];
+                    a[j][e] = ok ? av : (T)0;
+                    m[j][e] = ok ? mv : (T)0;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            if (kb0 + 4 * G * j >= k1) break;  // uniform
+#pragma unroll
+            for (int e = 0; e < E; e++) acc = Mfma<T>::mma(a[j][e], m[j][e], acc);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) red[wave][Mfma<T>::drow(lane, q)][i] = acc[q];
+    __syncthreads();
+    const int u = tid >> 4, row = tid & 15;
+    if (u < nu && r + row < K)
+        dst[fc + r + row + (int64_t)(u0 + u) * ldd] =
+            ((red[0][u][row] + red[1][u][row]) + red[2][u][row]) + red[3][u][row];
+}
+
 // ------------------------------- launchers ---------------------------------
+// NB of the several-right-hand-side kernels: 16 or 32 columns at a time
+#define PXA_NB(nrhs, CALL)        \
+    do {                          \
+        if ((nrhs) <= 16) {       \
+            constexpr int NB = 1; \
+            CALL;                 \
+        } else {                  \
+            constexpr int NB = 2; \
+            CALL;                 \
+        }                         \
+    } while (0)
+
+template <typename T, bool UPPER>
+static void launch_diag_narrow_m(const DevSymbol &S, const DiagItem *items, int n, const YSlices &ys,
+                                 const BwdItem *bitems, const T *pend, int64_t ldp, const T *src, int64_t lds,
+                                 T *dst, int64_t ldd, int nrhs, const T *inv, int maxwidth, hipStream_t st) {
+    PXA_NB(nrhs, {
+        const dim3 g(grid8(n), (nrhs + 16 * NB - 1) / (16 * NB));
+        if (maxwidth <= 16)
+            hipLaunchKernelGGL((k_diag_narrow_m<T, NB, 1, UPPER>), g, dim3(64), 0, st, S, items, n, ys, bitems, pend,
+                               ldp, src, lds, dst, ldd, nrhs, inv);
+        else if (maxwidth <= 32)
+            hipLaunchKernelGGL((k_diag_narrow_m<T, NB, 2, UPPER>), g, dim3(128), 0, st, S, items, n, ys, bitems, pend,
+                               ldp, src, lds, dst, ldd, nrhs, inv);
+        else
+            hipLaunchKernelGGL((k_diag_narrow_m<T, NB, 4, UPPER>), g, dim3(256), 0, st, S, items, n, ys, bitems, pend,
+                               ldp, src, lds, dst, ldd, nrhs, inv);
+    });
+}
+
 template <typename T>
 void launch_fwd_diag(const DevSymbol &S, const DiagItem *items, int n, const YSlices &ys, const T *ybuf,
                      int64_t ldy, T *b, int64_t ldb, T *z, int64_t ldz, int nrhs, const T *w1, const T *w1t,
                      int maxwidth, hipStream_t st) {
     if (n <= 0) return;
-    if (maxwidth > SOLVE_SPLIT) {
+    if (nrhs > 1) {
+        if (maxwidth <= SOLVE_NARROW) {
+            launch_diag_narrow_m<T, false>(S, items, n, ys, nullptr, ybuf, ldy, b, ldb, z, ldz, nrhs, w1, maxwidth, st);
+            return;
+        }
         hipLaunchKernelGGL(k_fwd_gather<T>, dim3(grid8(n), nrhs), dim3(256), 0, st, S, items, n, ys, ybuf, ldy, b, ldb);
-        if (nrhs == 1 && w1t)
-            hipLaunchKernelGGL(k_fwd_gemv16t<T>, dim3(grid8(4 * n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S,
-                               items, n, (const T *)b, z, w1t);
-        else if (nrhs == 1)
-            hipLaunchKernelGGL((k_diag_gemv16<T, false>), dim3(grid8(4 * n)), dim3(256), (size_t)maxwidth * sizeof(T),
-                               st, S, items, n, (const T *)b, z, w1);
+        const dim3 g(grid8(4 * n), (nrhs + 15) / 16);
+        if (w1t)
+            hipLaunchKernelGGL((k_diag_gemm16<T, false, true>), g, dim3(256), 0, st, S, items, n, (const T *)b, ldb, z,
+                               ldz, nrhs, w1t);
         else
-            hipLaunchKernelGGL((k_fwd_diag<T, 2, 16, true>), dim3(grid8(n), (nrhs + 1) / 2), dim3(1024),
-                               (size_t)maxwidth * 2 * sizeof(T), st, S, items, n, ys, ybuf, ldy, b, ldb, z, ldz,
-                               nrhs, w1, (const T *)nullptr);
+            hipLaunchKernelGGL((k_diag_gemm16<T, false, false>), g, dim3(256), 0, st, S, items, n, (const T *)b, ldb,
+                               z, ldz, nrhs, w1);
         return;
     }
-    // several right-hand sides: pairs of columns on the grid's y dimension,
-    // so that the few diagonal blocks of the top levels use more of the chip;
-    // levels of narrow cblks (maxwidth = the level's widest) take 4-wave
-    // workgroups
-    const bool narrow = maxwidth <= SOLVE_NARROW;
-    if (nrhs == 1) {
-        if (maxwidth <= SOLVE_TINY)
-            hipLaunchKernelGGL(k_fwd_diag_tiny<T>, dim3(grid8((n + 3) / 4)), dim3(64), 0, st, S, items, n, ys, ybuf, b,
-                               z, w1);
-        else if (narrow)
-            hipLaunchKernelGGL((k_fwd_diag<T, 1, 4>), dim3(grid8(n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S,
-                               items, n, ys, ybuf, ldy, b, ldb, z, ldz, nrhs, w1, w1t);
+    if (maxwidth > SOLVE_SPLIT) {
+        hipLaunchKernelGGL(k_fwd_gather<T>, dim3(grid8(n), 1), dim3(256), 0, st, S, items, n, ys, ybuf, ldy, b, ldb);
+        if (w1t)
+            hipLaunchKernelGGL(k_fwd_gemv16t<T>, dim3(grid8(4 * n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S,
+                               items, n, (const T *)b, z, w1t);
         else
-            hipLaunchKernelGGL((k_fwd_diag<T, 1, 16>), dim3(grid8(n)), dim3(1024), (size_t)maxwidth * sizeof(T), st,
-                               S, items, n, ys, ybuf, ldy, b, ldb, z, ldz, nrhs, w1, w1t);
-    } else {
-        if (narrow)
-            hipLaunchKernelGGL((k_fwd_diag<T, 2, 4>), dim3(grid8(n), (nrhs + 1) / 2), dim3(256),
-                               (size_t)maxwidth * 2 * sizeof(T), st, S, items, n, ys, ybuf, ldy, b, ldb, z, ldz,
-                               nrhs, w1, (const T *)nullptr);
-        else
-            hipLaunchKernelGGL((k_fwd_diag<T, 2, 16>), dim3(grid8(n), (nrhs + 1) / 2), dim3(1024),
-                               (size_t)maxwidth * 2 * sizeof(T), st, S, items, n, ys, ybuf, ldy, b, ldb, z, ldz,
-                               nrhs, w1, (const T *)nullptr);
+            hipLaunchKernelGGL((k_diag_gemv16<T, false>), dim3(grid8(4 * n)), dim3(256), (size_t)maxwidth * sizeof(T),
+                               st, S, items, n, (const T *)b, z, w1);
+        return;
     }
+    // levels of narrow cblks (maxwidth = the level's widest) take 4-wave workgroups
+    if (maxwidth <= SOLVE_TINY)
+        hipLaunchKernelGGL(k_fwd_diag_tiny<T>, dim3(grid8((n + 3) / 4)), dim3(64), 0, st, S, items, n, ys, ybuf, b, z,
+                           w1);
+    else if (maxwidth <= SOLVE_NARROW)
+        hipLaunchKernelGGL((k_fwd_diag<T, 4>), dim3(grid8(n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S, items,
+                           n, ys, ybuf, b, z, w1, w1t);
+    else
+        hipLaunchKernelGGL((k_fwd_diag<T, 16>), dim3(grid8(n)), dim3(1024), (size_t)maxwidth * sizeof(T), st, S,
+                           items, n, ys, ybuf, b, z, w1, w1t);
 }
 template <typename T>
 void launch_fwd_prod(const DevSymbol &S, const FwdItem *items, int n, const T *coef, const T *z, int64_t ldz,
                      int nrhs, const int32_t *ydst, T *ybuf, int64_t ldy, int maxwidth, hipStream_t st) {
     if (n <= 0) return;
-    if (nrhs == 1 && maxwidth <= SOLVE_TINY)
-        hipLaunchKernelGGL((k_fwd_prod<T, 1, 1>), dim3(grid8(n)), dim3(64), (size_t)maxwidth * sizeof(T), st, S,
-                           items, n, coef, z, ldz, nrhs, ydst, ybuf, ldy);
-    else if (nrhs == 1 && maxwidth <= SOLVE_NARROW)
-        hipLaunchKernelGGL((k_fwd_prod<T, 1, 4>), dim3(grid8(n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S,
-                           items, n, coef, z, ldz, nrhs, ydst, ybuf, ldy);
-    else if (nrhs == 1)
-        hipLaunchKernelGGL((k_fwd_prod<T, 1, 16>), dim3(grid8(n)), dim3(1024), (size_t)maxwidth * sizeof(T), st, S,
-                           items, n, coef, z, ldz, nrhs, ydst, ybuf, ldy);
+    if (nrhs > 1)
+        PXA_NB(nrhs, hipLaunchKernelGGL((k_fwd_prod_m<T, NB>), dim3(grid8(n), (nrhs + 16 * NB - 1) / (16 * NB)),
+                                        dim3(256), 0, st, S, items, n, coef, z, ldz, nrhs, ydst, ybuf, ldy));
+    else if (maxwidth <= SOLVE_TINY)
+        hipLaunchKernelGGL((k_fwd_prod<T, 1>), dim3(grid8(n)), dim3(64), (size_t)maxwidth * sizeof(T), st, S, items,
+                           n, coef, z, ydst, ybuf);
+    else if (maxwidth <= SOLVE_NARROW)
+        hipLaunchKernelGGL((k_fwd_prod<T, 4>), dim3(grid8(n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S, items,
+                           n, coef, z, ydst, ybuf);
     else
-        hipLaunchKernelGGL((k_fwd_prod<T, 8, 8>), dim3(grid8(n), (nrhs + 7) / 8), dim3(512),
-                           (size_t)maxwidth * 8 * sizeof(T), st, S, items, n, coef, z, ldz, nrhs, ydst, ybuf, ldy);
+        hipLaunchKernelGGL((k_fwd_prod<T, 16>), dim3(grid8(n)), dim3(1024), (size_t)maxwidth * sizeof(T), st, S, items,
+                           n, coef, z, ydst, ybuf);
 }
 template <typename T>
 void launch_bwd_prod(const DevSymbol &S, const BwdItem *items, int n, const T *coef, const T *x, int64_t ldx,
                      int nrhs, T *part, int maxwidth, hipStream_t st) {
     if (n <= 0) return;
-    if (nrhs == 1 && maxwidth <= SOLVE_TINY) {
+    if (nrhs > 1) {
+        PXA_NB(nrhs, {
+            const int gz = (nrhs + 16 * NB - 1) / (16 * NB);
+            if (maxwidth <= 16)
+                hipLaunchKernelGGL((k_bwd_prod_m<T, NB, 1>), dim3(grid8(n), 1, gz), dim3(256), 0, st, S, items, n,
+                                   coef, x, ldx, nrhs, part);
+            else if (maxwidth <= 32)
+                hipLaunchKernelGGL((k_bwd_prod_m<T, NB, 2>), dim3(grid8(n), 1, gz), dim3(256), 0, st, S, items, n,
+                                   coef, x, ldx, nrhs, part);
+            else
+                hipLaunchKernelGGL((k_bwd_prod_m<T, NB, 4>), dim3(grid8(n), (maxwidth + 63) / 64, gz), dim3(256), 0,
+                                   st, S, items, n, coef, x, ldx, nrhs, part);
+        });
+        return;
+    }
+    if (maxwidth <= SOLVE_TINY) {
         hipLaunchKernelGGL((k_bwd_prod_narrow<T, SOLVE_TINY>), dim3(grid8((n + 3) / 4)), dim3(64), 0, st, S, items, n,
                            coef, x, part);
         return;
     }
-    const dim3 g(grid8(n), (maxwidth + 63) / 64, nrhs == 1 ? 1 : (nrhs + 7) / 8);
-    if (nrhs == 1)
-        hipLaunchKernelGGL((k_bwd_prod<T, 1>), g, dim3(256), 0, st, S, items, n, coef, x, ldx, nrhs, part);
-    else
-        hipLaunchKernelGGL((k_bwd_prod<T, 8>), g, dim3(256), 0, st, S, items, n, coef, x, ldx, nrhs, part);
+    hipLaunchKernelGGL(k_bwd_prod<T>, dim3(grid8(n), (maxwidth + 63) / 64), dim3(256), 0, st, S, items, n, coef, x,
+                       part);
 }
 template <typename T>
 void launch_bwd_diag(const DevSymbol &S, const DiagItem *items, int n, const BwdItem *bitems, T *z,
                      int64_t ldz, T *x, int64_t ldx, int nrhs, const T *part, const T *wb, int maxwidth,
                      hipStream_t st) {
     if (n <= 0) return;
-    if (maxwidth > SOLVE_SPLIT) {
+    if (nrhs > 1) {
+        if (maxwidth <= SOLVE_NARROW) {
+            launch_diag_narrow_m<T, true>(S, items, n, YSlices{}, bitems, part, 0, z, ldz, x, ldx, nrhs, wb, maxwidth,
+                                          st);
+            return;
+        }
         hipLaunchKernelGGL(k_bwd_reduce<T>, dim3(grid8(n), nrhs), dim3(256), 0, st, S, items, n, bitems, z, ldz, part,
                            nrhs);
-        if (nrhs == 1)
-            hipLaunchKernelGGL((k_diag_gemv16<T, true>), dim3(grid8(4 * n)), dim3(256), (size_t)maxwidth * sizeof(T),
-                               st, S, items, n, (const T *)z, x, wb);
-        else
-            hipLaunchKernelGGL((k_bwd_diag<T, 2, 16, true>), dim3(grid8(n), (nrhs + 1) / 2), dim3(1024),
-                               (size_t)maxwidth * 2 * sizeof(T), st, S, items, n, bitems, z, ldz, x, ldx, nrhs, part,
-                               wb);
+        hipLaunchKernelGGL((k_diag_gemm16<T, true, false>), dim3(grid8(4 * n), (nrhs + 15) / 16), dim3(256), 0, st, S,
+                           items, n, (const T *)z, ldz, x, ldx, nrhs, wb);
         return;
     }
-    const bool narrow = maxwidth <= SOLVE_NARROW;
-    if (nrhs == 1) {
-        if (maxwidth <= SOLVE_TINY)
-            hipLaunchKernelGGL(k_bwd_diag_tiny<T>, dim3(grid8((n + 3) / 4)), dim3(64), 0, st, S, items, n, bitems, z, x,
-                               part, wb);
-        else if (narrow)
-            hipLaunchKernelGGL((k_bwd_diag<T, 1, 4>), dim3(grid8(n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S,
-                               items, n, bitems, z, ldz, x, ldx, nrhs, part, wb);
-        else
-            hipLaunchKernelGGL((k_bwd_diag<T, 1, 16>), dim3(grid8(n)), dim3(1024), (size_t)maxwidth * sizeof(T), st,
-                               S, items, n, bitems, z, ldz, x, ldx, nrhs, part, wb);
-    } else {
-        if (narrow)
-            hipLaunchKernelGGL((k_bwd_diag<T, 2, 4>), dim3(grid8(n), (nrhs + 1) / 2), dim3(256),
-                               (size_t)maxwidth * 2 * sizeof(T), st, S, items, n, bitems, z, ldz, x, ldx, nrhs, part,
-                               wb);
-        else
-            hipLaunchKernelGGL((k_bwd_diag<T, 2, 16>), dim3(grid8(n), (nrhs + 1) / 2), dim3(1024),
-                               (size_t)maxwidth * 2 * sizeof(T), st, S, items, n, bitems, z, ldz, x, ldx, nrhs, part,
-                               wb);
+    if (maxwidth > SOLVE_SPLIT) {
+        hipLaunchKernelGGL(k_bwd_reduce<T>, dim3(grid8(n), 1), dim3(256), 0, st, S, items, n, bitems, z, ldz, part, 1);
+        hipLaunchKernelGGL((k_diag_gemv16<T, true>), dim3(grid8(4 * n)), dim3(256), (size_t)maxwidth * sizeof(T), st,
+                           S, items, n, (const T *)z, x, wb);
+        return;
     }
+    if (maxwidth <= SOLVE_TINY)
+        hipLaunchKernelGGL(k_bwd_diag_tiny<T>, dim3(grid8((n + 3) / 4)), dim3(64), 0, st, S, items, n, bitems, z, x,
+                           part, wb);
+    else if (maxwidth <= SOLVE_NARROW)
+        hipLaunchKernelGGL((k_bwd_diag<T, 4>), dim3(grid8(n)), dim3(256), (size_t)maxwidth * sizeof(T), st, S, items,
+                           n, bitems, z, x, part, wb);
+    else
+        hipLaunchKernelGGL((k_bwd_diag<T, 16>), dim3(grid8(n)), dim3(1024), (size_t)maxwidth * sizeof(T), st, S, items,
+                           n, bitems, z, x, part, wb);
 }
 
 
