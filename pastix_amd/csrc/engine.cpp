@@ -1049,9 +1049,13 @@ int64_t Engine::work_bytes(int R) const {
     return 8 * (2 * nr + 4 * nr) + (prec_ == 2 ? fsz * nr : 0) + 8 * 8 * (int64_t)R + 8 * nchunk * R;
 }
 
-int Engine::precond_block(double *zb, int R) {
-    if (prec_ == 3) return solve_t<double>(zb, n_, R);
+// zb = M^{-1} rb, R columns
+int Engine::precond_block(const double *rb, double *zb, int R) {
     const int64_t nr = n_ * (int64_t)R;
+    if (prec_ == 3) {
+        launch_copy(nr, rb, zb, stream_);
+        return solve_t<double>(zb, n_, R);
+    }
     if (bsvec_cap_ < nr) {
         release(d_bsvec_);
         bsvec_cap_ = nr;
@@ -1061,7 +1065,7 @@ int Engine::precond_block(double *zb, int R) {
             return -1;
         }
     }
-    launch_d2s(nr, zb, d_bsvec_, stream_);
+    launch_d2s(nr, rb, d_bsvec_, stream_);
     const int rc = solve_t<float>(d_bsvec_, n_, R);
     if (rc) return rc;
     launch_s2d(nr, d_bsvec_, zb, stream_);
@@ -1158,10 +1162,8 @@ int Engine::refine_cg_batch(double *X, const double *B, int R, const std::vector
     };
     if (segdot(B, B, normb.data())) return -1;
     for (int64_t k = 0; k < ns; k++) normb[k] = std::sqrt(normb[k]);
-    for (int c = 0; c < R; c++) {
-        launch_copy(n_, B + c * n_, Rv + c * n_, stream_);
-        spmv(-1.0, X + c * n_, 1.0, Rv + c * n_);
-    }
+    if (!have_matrix_) return fail("matrix not uploaded");
+    launch_spmv_cols(n_, R, d_rowptr_, d_cols_, d_vals_, -1.0, X, 1.0, B, Rv, stream_);
     auto residuals = [&]() -> double {
         double worst = 0;
         for (int64_t k = 0; k < ns; k++) {
@@ -1175,14 +1177,13 @@ int Engine::refine_cg_batch(double *X, const double *B, int R, const std::vector
     double worst = residuals();
     int it = 0;
     if (worst > eps && it < itermax) {
-        launch_copy(nr, Rv, Z, stream_);
-        if (precond_block(Z, R)) return -1;
+        if (precond_block(Rv, Z, R)) return -1;
         launch_copy(nr, Z, P, stream_);
     }
     std::vector<double> pap(ns), rz2(ns);
     while (worst > eps && it < itermax) {
         it++;
-        for (int c = 0; c < R; c++) spmv(1.0, P + c * n_, 0.0, AP + c * n_);
+        launch_spmv_cols(n_, R, d_rowptr_, d_cols_, d_vals_, 1.0, P, 0.0, AP, AP, stream_);
         if (segdot(Rv, Z, rz.data()) || segdot(AP, P, pap.data())) return -1;
         for (int64_t k = 0; k < ns; k++) a[k] = (rb[k] > eps && pap[k] != 0.0) ? rz[k] / pap[k] : 0.0;
         if (upload(a)) return -1;
@@ -1193,8 +1194,7 @@ int Engine::refine_cg_batch(double *X, const double *B, int R, const std::vector
         if (segdot(Rv, Rv, h.data())) return -1;
         worst = residuals();
         if (!(worst > eps && it < itermax)) break;
-        launch_copy(nr, Rv, Z, stream_);
-        if (precond_block(Z, R)) return -1;
+        if (precond_block(Rv, Z, R)) return -1;
         if (segdot(Rv, Z, rz2.data())) return -1;
         for (int64_t k = 0; k < ns; k++) a[k] = (rz[k] != 0.0) ? rz2[k] / rz[k] : 0.0;
         if (upload(a)) return -1;
@@ -1233,8 +1233,7 @@ int Engine::refine_user(const double *Bu, int64_t ldb, double *Xu, int64_t ldx, 
     };
     in(Bu, ldb, PB);
     if (initial_solve) {
-        launch_copy(nr, PB, PX, stream_);
-        if (precond_block(PX, R)) return -1;
+        if (precond_block(PB, PX, R)) return -1;
     } else {
         in(Xu, ldx, PX);
     }

