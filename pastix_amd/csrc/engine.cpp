@@ -126,6 +126,13 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
 
     lv_cblk_ptr_ = P.lv_cblk_ptr;
     schurfcol_ = (P.schur_cblk < cblknbr_) ? s.cblk_fcol[P.schur_cblk] : n_;
+    // widest factored cblk of each level
+    lv_maxw_.assign(P.nlevels, 0);
+    for (int32_t lv = 0; lv < P.nlevels; lv++)
+        for (int32_t k = P.lv_cblk_ptr[lv]; k < P.lv_cblk_ptr[lv] + P.lv_fact_cnt[lv]; k++) {
+            const int32_t c = P.lv_cblks[k];
+            lv_maxw_[lv] = std::max<int>(lv_maxw_[lv], (int)(s.cblk_fcol[c + 1] - s.cblk_fcol[c]));
+        }
     lv_sq_ptr_.clear();
     if (factotype == 2) {
         std::vector<PanelItem> sq;
@@ -435,13 +442,13 @@ template <typename T> int Engine::factorize_t(double thr) {
                 // here: it reserves the factorisation's LDS for every update
                 // workgroup, which the second stream's updates then lack)
                 launch_panel_upd<T>(S_, d_pupd_ + q0, nq, kb, false, L, L, L, false, stream_);
-                launch_potrf64<T>(S_, d_step_cblks_ + b0, nb, kb, L, W1, (T *)d_WB_, thr, d_stat_, stream_);
+                launch_potrf64<T>(S_, d_step_cblks_ + b0, nb, kb, lv_maxw_[lv], L, W1, (T *)d_WB_, thr, d_stat_, stream_);
                 launch_panel_trsm<T>(S_, d_ptrsm_ + p0, np, kb, L, W1, stream_);
             } else {
                 // right-looking: the step's update and the next step's
                 // diagonal factorisations share one launch
                 if (kb == 0)
-                    launch_potrf64<T>(S_, d_step_cblks_ + b0, nb, kb, L, W1, (T *)d_WB_, thr, d_stat_, stream_);
+                    launch_potrf64<T>(S_, d_step_cblks_ + b0, nb, kb, lv_maxw_[lv], L, W1, (T *)d_WB_, thr, d_stat_, stream_);
                 launch_panel_trsm<T>(S_, d_ptrsm_ + p0, np, kb, L, W1, stream_);
                 if (s + 1 < lv_step_ptr_[lv + 1]) {
                     const int b1 = step_cb_ptr_[s + 1], nb1 = step_cb_ptr_[s + 2] - b1;

@@ -202,6 +202,7 @@ class Engine {
     // solve levels: widest node (diagonal kernels), widest cblk (products)
     std::vector<int> slv_maxw_, slv_maxcw_;
     int64_t schurfcol_ = 0;
+    std::vector<int> lv_maxw_;  // widest factored cblk of each level
     // LU: 64x64 tiles on and below the diagonal of the factored cblks'
     // squares, level L's at [lv_sq_ptr_[L], lv_sq_ptr_[L + 1])
     PanelItem *d_sq_ = nullptr;

@@ -21,7 +21,7 @@ void launch_update_gather(const DevSymbol &S, int mode, const UpdItem *items, in
 
 // Blocked panel factorisation (64-column steps).
 template <typename T>
-void launch_potrf64(const DevSymbol &S, const int32_t *cblks, int n, int kb, T *coef, T *winv, T *winvt, double thr,
+void launch_potrf64(const DevSymbol &S, const int32_t *cblks, int n, int kb, int maxwidth, T *coef, T *winv, T *winvt, double thr,
                     int *stat, hipStream_t st);
 template <typename T>
 void launch_panel_trsm(const DevSymbol &S, const PanelItem *items, int n, int kb, T *coef, const T *winv,

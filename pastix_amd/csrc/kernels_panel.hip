@@ -16,6 +16,7 @@
 // once the panels are factored.  Inverses are stored twice: W (lower,
 // column-major) for the forward sweep and WT = W^T for the backward sweep.
 #include <algorithm>
+#include <type_traits>
 
 #include "dev_common.h"
 #include "dev_types.h"
@@ -343,6 +344,118 @@ __global__ __launch_bounds__(256) void k_potrf64(DevSymbol S, const int32_t *__r
     __builtin_amdgcn_s_setprio(3);  // panel steps lead the critical path
     __shared__ PotrfLds<T> lds;
     potrf64_block<T>(S, cblks[blockIdx.x], kb, coef, winv, winvt, thr, stat, lds);
+}
+
+// Narrow supernodes.  k_potrf64 gives each one a 256-thread workgroup and 42 KB
+// of LDS whatever its width: a leaf level of thousands of supernodes of 4 to
+// 10 columns was three workgroups to a compute unit, each padding to 64 rows
+// (701x653 grid, FP64: 16,384 of at most 5 columns 523 us; 80^3: 21,293 of at
+// most 8).  Below, a row is a lane with its columns in registers, the pivot
+// column crosses lanes without LDS, and nothing waits on a barrier.  The
+// elimination is k_potrf64's, operation for operation; the inverse comes from
+// forward substitution, lane c solving for column c.
+
+// f(integral_constant<int, I>) for I = B .. E - 1
+template <int B, int E, class F> __device__ __forceinline__ void static_for(F f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
+}
+
+// v of lane N of the calling lane's row of sixteen
+template <int N> __device__ __forceinline__ int row16(int v) {
+    return __builtin_amdgcn_mov_dpp(v, 0x150 + N, 0xf, 0xf, true);  // row_newbcast:N
+}
+template <int N> __device__ __forceinline__ float row16(float v) {
+    return __builtin_bit_cast(float, row16<N>(__builtin_bit_cast(int, v)));
+}
+template <int N> __device__ __forceinline__ double row16(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)row16<N>((int)(unsigned)u), hi = (unsigned)row16<N>((int)(unsigned)(u >> 32));
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Lane exchange of one supernode of at most KM columns: sixteen lanes and
+// four supernodes to a wave (KM = 16), or the whole wave (KM = 32, uniform
+// reads of one lane).
+template <typename T, int KM, int N> __device__ __forceinline__ T from_row(T v) {
+    if constexpr (KM == 16) return row16<N>(v);
+    else return rlane(v, N);
+}
+
+template <typename T, int KM>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KM == 16 ? 4 : 3))) void k_potrf_narrow(DevSymbol S, const int32_t *__restrict__ cblks, int n,
+                                                     T *__restrict__ coef, T *__restrict__ winv,
+                                                     T *__restrict__ winvt, double thr, int *stat) {
+    __builtin_amdgcn_s_setprio(3);
+    constexpr int PW = KM == 16 ? 4 : 1;  // supernodes of a wave
+    const int lane = threadIdx.x, i = KM == 16 ? (lane & 15) : lane;
+    const int id = blockIdx.x * PW + (KM == 16 ? (lane >> 4) : 0);
+    int K = 0;
+    int64_t ld = 0, wo = 0;
+    T *P = coef;
+    if (id < n) {
+        const int c = cblks[id];
+        K = S.cblk_fcol[c + 1] - S.cblk_fcol[c];
+        ld = S.cblk_stride[c];
+        P = coef + S.cblk_coef[c];
+        wo = S.cblk_winv[c];
+    }
+    T a[KM];
+#pragma unroll
+    for (int j = 0; j < KM; j++) a[j] = (i < K && j <= i) ? P[i + (int64_t)j * ld] : (i == j) ? (T)1 : (T)0;
+    // columns of the wave's widest supernode: the padding after them is skipped
+    int km = __builtin_amdgcn_readfirstlane(K);
+    if constexpr (KM == 16)
+        for (int g = 1; g < 4; g++) km = max(km, __builtin_amdgcn_readlane(K, 16 * g));
+    const T crit = (T)thr;
+    int npiv = 0, neg = 0;
+    T dia = (T)1;  // this row's diagonal entry
+    static_for<0, KM>([&](auto kk) {
+        constexpr int k = kk;
+        if (k >= km) return;  // uniform
+        const T d = from_row<T, KM, k>(a[k]);
+        int np = 0, ng = 0;
+        T L, r;
+        sqrt_rsqrt(piv_max(d, crit, np, ng), L, r);
+        npiv += (k < K) ? np : 0;
+        neg |= (k < K) ? ng : 0;
+        if (i == k) dia = L;
+        a[k] = (i == k) ? L : a[k] * r;
+        static_for<k + 1, KM>([&](auto jj) {
+            constexpr int j = jj;
+            a[j] = fma_(-a[k], from_row<T, KM, j>(a[k]), a[j]);
+        });
+    });
+#pragma unroll
+    for (int j = 0; j < KM; j++)
+        if (i < K && j <= i) P[i + (int64_t)j * ld] = a[j];
+    if (i == 0) {
+        if (npiv) atomicAdd(&stat[0], npiv);
+        if (neg) atomicOr(&stat[1], 1);
+    }
+    const T di = recip(dia);
+    T x[KM];
+    static_for<0, KM>([&](auto rr) {
+        constexpr int r = rr;
+        if (r >= km) return;  // uniform
+        T v = (i == r) ? (T)1 : (T)0;
+        static_for<0, r>([&](auto kk) {
+            constexpr int k = kk;
+            v = fma_(-from_row<T, KM, r>(a[k]), x[k], v);
+        });
+        x[r] = v * from_row<T, KM, r>(di);
+    });
+    if (i < K) {
+        T *W = winv + wo, *WT = winvt + wo;
+#pragma unroll
+        for (int r = 0; r < KM; r++)
+            if (r < K) {
+                W[r + (int64_t)i * K] = x[r];
+                WT[i + (int64_t)r * K] = x[r];
+            }
+    }
 }
 
 // rows [r0, r0+64) of cblk c below the diagonal sub-block kb: X = A * W_kk^T
@@ -991,9 +1104,23 @@ __global__ __launch_bounds__(256) void k_leaf_tasks(DevSymbol S, LeafDev LP, con
 static inline int grid8(int n) { return ((n + 7) / 8) * 8; }
 
 template <typename T>
-void launch_potrf64(const DevSymbol &S, const int32_t *cblks, int n, int kb, T *coef, T *winv, T *winvt, double thr,
-                    int *stat, hipStream_t st) {
+void launch_potrf64(const DevSymbol &S, const int32_t *cblks, int n, int kb, int maxwidth, T *coef, T *winv, T *winvt,
+                    double thr, int *stat, hipStream_t st) {
     if (n <= 0) return;
+    // at most 16 columns: 8 to 40 us (16,384 supernodes), k_potrf64 17 to 523
+    if (kb == 0 && maxwidth <= 16) {
+        hipLaunchKernelGGL((k_potrf_narrow<T, 16>), dim3((n + 3) / 4), dim3(64), 0, st, S, cblks, n, coef, winv, winvt,
+                           thr, stat);
+        return;
+    }
+    // up to 32 columns the whole wave takes one: 30 us however few there are
+    // (its 32 pivots follow each other), where k_potrf64 takes 20 us for up to
+    // some 500 supernodes and 40 us more for every 1024 (FP64)
+    if (kb == 0 && maxwidth <= 32 && n >= 1024) {
+        hipLaunchKernelGGL((k_potrf_narrow<T, 32>), dim3(n), dim3(64), 0, st, S, cblks, n, coef, winv, winvt, thr,
+                           stat);
+        return;
+    }
     hipLaunchKernelGGL(k_potrf64<T>, dim3(n), dim3(256), 0, st, S, cblks, kb, coef, winv, winvt, thr, stat);
 }
 template <typename T>
@@ -1080,7 +1207,7 @@ void launch_leaf_tasks(const DevSymbol &S, const LeafDev &LP, const UpdEntry *en
                                     int *, hipStream_t);                                                           \
     template void launch_lu_square_layout<T>(const DevSymbol &, const PanelItem *, int, T *, T *, hipStream_t);      \
     template void launch_lu_square_merge<T>(const DevSymbol &, const PanelItem *, int, T *, T *, hipStream_t);       \
-    template void launch_potrf64<T>(const DevSymbol &, const int32_t *, int, int, T *, T *, T *, double, int *,    \
+    template void launch_potrf64<T>(const DevSymbol &, const int32_t *, int, int, int, T *, T *, T *, double, int *,    \
                                     hipStream_t);                                                                  \
     template void launch_panel_trsm<T>(const DevSymbol &, const PanelItem *, int, int, T *, const T *, hipStream_t); \
     template void launch_panel_trsm2<T>(const DevSymbol &, const PanelItem *, int, int, T *, const T *, T *,         \
