@@ -35,10 +35,8 @@ template <typename T> struct Quad {
             for (int n = 0; n < 2; n++)
                 for (int r = 0; r < 4; r++) c[m][n][r] = (T)0;
     }
-    // Block m takes the rows of parity m, block n the columns of parity n (a
-    // lane's two operand rows are then adjacent in LDS: one read for both).
     // Element of block (m,n), register r, owned by `lane`:
-    //   row = 2*Mfma<T>::drow(lane, r) + m, col = 2*(lane&15) + n
+    //   row = m*16 + Mfma<T>::drow(lane, r), col = n*16 + (lane&15)
 };
 
 // Operand staging moves 16 bytes per lane: E = 16 / sizeof(T) consecutive
@@ -106,25 +104,25 @@ template <typename T, int CH = 16> struct StageBuf {
     T ys[CH][68];
 };
 
-// an MFMA operand pair of one lane: rows 2i and 2i+1 of a 32-row fragment
-template <typename T> struct Frag { typedef T v __attribute__((ext_vector_type(2))); };
-
 // one chunk's MFMAs of a 32x32 quadrant, X fragments at xs[.][xr], Y at
-// ys[.][yr]; left columns of the chunk (and later) exist.  The steps stay
-// behind the test of left: without it (straight-line code) the direct update
-// ran 22.4 instead of 21.9 ms.
+// ys[.][yr]; left columns of the chunk (and later) exist.  A rolled loop:
+// unrolled four times the direct update ran 21.7 instead of 20.9 ms,
+// straight through 22.4.  Rows i and i + 16 to a lane, so that a lane group
+// stores sixteen rows side by side; rows 2i and 2i + 1 would come in one LDS
+// read but store every other row (21.4 ms).
 template <typename T, int CH, int PX, int PY>
 __device__ __forceinline__ void quad_chunk(Quad<T> &q, const T (*xs)[PX], const T (*ys)[PY], int xr, int yr, int left,
                                            int kq) {
-#pragma unroll
-    for (int s = 0; s < CH / 4; s++) {
-        if (4 * s >= left) break;  // uniform
-        const typename Frag<T>::v x = *reinterpret_cast<const typename Frag<T>::v *>(&xs[4 * s + kq][xr]);
-        const typename Frag<T>::v y = *reinterpret_cast<const typename Frag<T>::v *>(&ys[4 * s + kq][yr]);
-        q.c[0][0] = Mfma<T>::mma(x[0], y[0], q.c[0][0]);
-        q.c[0][1] = Mfma<T>::mma(x[0], y[1], q.c[0][1]);
-        q.c[1][0] = Mfma<T>::mma(x[1], y[0], q.c[1][0]);
-        q.c[1][1] = Mfma<T>::mma(x[1], y[1], q.c[1][1]);
+    const int ns = (min(CH, left) + 3) / 4;
+#pragma unroll 1
+    for (int s = 0; s < ns; s++) {
+        const int kr = 4 * s + kq;
+        const T x0 = xs[kr][xr], x1 = xs[kr][xr + 16];
+        const T y0 = ys[kr][yr], y1 = ys[kr][yr + 16];
+        q.c[0][0] = Mfma<T>::mma(x0, y0, q.c[0][0]);
+        q.c[0][1] = Mfma<T>::mma(x0, y1, q.c[0][1]);
+        q.c[1][0] = Mfma<T>::mma(x1, y0, q.c[1][0]);
+        q.c[1][1] = Mfma<T>::mma(x1, y1, q.c[1][1]);
     }
 }
 
@@ -175,35 +173,52 @@ template <typename T, int R, int CH> struct Stager {
     }
 };
 
+template <typename T, int CH> struct GemmLds {
+    Stager<T, 64, CH> gx, gy;
+    int mx, my, K;
+    // the first chunk's loads go out
+    __device__ __forceinline__ void start(const T *X, int mx_, int64_t ldx, const T *Y, int my_, int64_t ldy, int K_,
+                                          int tid) {
+        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        mx = mx_;
+        my = my_;
+        K = K_;
+        gx.init(X, mx, ldx, lane, wave);
+        gy.init(Y, my, ldy, lane, wave);
+        gx.load(0, K);
+        gy.load(0, K);
+    }
+    __device__ __forceinline__ void run(Quad<T> &q, StageBuf<T, CH> &sb, int tid) {
+        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+        const int i = lane & 15, kq = lane >> 4;
+        const bool active = (wr < mx) && (wc < my);
+        gx.store(sb.xs, 0, K);
+        gy.store(sb.ys, 0, K);
+        __syncthreads();
+        for (int k0 = 0; k0 < K; k0 += CH) {
+            const bool more = k0 + CH < K;
+            if (more) {
+                gx.load(k0 + CH, K);
+                gy.load(k0 + CH, K);
+            }
+            if (active) quad_chunk<T, CH>(q, sb.xs, sb.ys, wr + i, wc + i, K - k0, kq);
+            __syncthreads();
+            if (more) {
+                gx.store(sb.xs, k0 + CH, K);
+                gy.store(sb.ys, k0 + CH, K);
+            }
+            __syncthreads();
+        }
+    }
+};
+
 template <typename T, int CH>
 __device__ __forceinline__ void wg_gemm_lds(Quad<T> &q, const T *X, int mx, int64_t ldx, const T *Y, int my,
                                             int64_t ldy, int K, StageBuf<T, CH> &sb, int tid) {
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    const int i = 2 * (lane & 15), kq = lane >> 4;
-    Stager<T, 64, CH> gx, gy;
-    gx.init(X, mx, ldx, lane, wave);
-    gy.init(Y, my, ldy, lane, wave);
-    const bool active = (wr < mx) && (wc < my);
-    gx.load(0, K);
-    gy.load(0, K);
-    gx.store(sb.xs, 0, K);
-    gy.store(sb.ys, 0, K);
-    __syncthreads();
-    for (int k0 = 0; k0 < K; k0 += CH) {
-        const bool more = k0 + CH < K;
-        if (more) {
-            gx.load(k0 + CH, K);
-            gy.load(k0 + CH, K);
-        }
-        if (active) quad_chunk<T, CH>(q, sb.xs, sb.ys, wr + i, wc + i, K - k0, kq);
-        __syncthreads();
-        if (more) {
-            gx.store(sb.xs, k0 + CH, K);
-            gy.store(sb.ys, k0 + CH, K);
-        }
-        __syncthreads();
-    }
+    GemmLds<T, CH> g;
+    g.start(X, mx, ldx, Y, my, ldy, K, tid);
+    g.run(q, sb, tid);
 }
 
 // The same product for a 64 x 128 tile: q0, q1 += X[0:64, 0:K] * Y[0:128,
@@ -221,7 +236,7 @@ __device__ __forceinline__ void wg_gemm_lds_64x128(Quad<T> &q0, Quad<T> &q1, con
                                                    int tid) {
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = (wave >> 1) * 32, wc = (wave & 1) * 64;
-    const int i = 2 * (lane & 15), kq = lane >> 4;
+    const int i = lane & 15, kq = lane >> 4;
     Stager<T, 64, CH> gx;
     Stager<T, 128, CH> gy;
     gx.init(X, mx, ldx, lane, wave);
@@ -242,14 +257,14 @@ __device__ __forceinline__ void wg_gemm_lds_64x128(Quad<T> &q0, Quad<T> &q1, con
 #pragma unroll
             for (int s = 0; s < CH / 4; s++) {
                 if (k0 + 4 * s < K) {
-                    const typename Frag<T>::v x = *reinterpret_cast<const typename Frag<T>::v *>(&sb.xs[4 * s + kq][wr + i]);
-                    const typename Frag<T>::v y = *reinterpret_cast<const typename Frag<T>::v *>(&sb.ys[4 * s + kq][wc + i]);
+                    const T x[2] = {sb.xs[4 * s + kq][wr + i], sb.xs[4 * s + kq][wr + 16 + i]};
+                    const T y[2] = {sb.ys[4 * s + kq][wc + i], sb.ys[4 * s + kq][wc + 16 + i]};
                     q0.c[0][0] = Mfma<T>::mma(x[0], y[0], q0.c[0][0]);
                     q0.c[0][1] = Mfma<T>::mma(x[0], y[1], q0.c[0][1]);
                     q0.c[1][0] = Mfma<T>::mma(x[1], y[0], q0.c[1][0]);
                     q0.c[1][1] = Mfma<T>::mma(x[1], y[1], q0.c[1][1]);
                     if (act1) {
-                        const typename Frag<T>::v z = *reinterpret_cast<const typename Frag<T>::v *>(&sb.ys[4 * s + kq][wc + 32 + i]);
+                        const T z[2] = {sb.ys[4 * s + kq][wc + 32 + i], sb.ys[4 * s + kq][wc + 48 + i]};
                         q1.c[0][0] = Mfma<T>::mma(x[0], z[0], q1.c[0][0]);
                         q1.c[0][1] = Mfma<T>::mma(x[0], z[1], q1.c[0][1]);
                         q1.c[1][0] = Mfma<T>::mma(x[1], z[0], q1.c[1][0]);
@@ -281,7 +296,7 @@ template <typename T, class At> __device__ __forceinline__ void quad_sub(const Q
         for (int n = 0; n < 2; n++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                p[n][r] = at(2 * Mfma<T>::drow(lane, r) + m, 2 * (lane & 15) + n, ok[n][r]);
+                p[n][r] = at(m * 16 + Mfma<T>::drow(lane, r), n * 16 + (lane & 15), ok[n][r]);
                 v[n][r] = *p[n][r];
             }
 #pragma unroll

@@ -48,6 +48,18 @@ struct UpdEntry {
     int32_t s, p0, p1, q0, q1, sb, ib0, grp;
 };
 
+// The same contribution as the one-pass update kernels read it: every field
+// they need in one 64-byte line, so that a tile's operand and map loads start
+// one memory round trip after its launch instead of three or four.
+struct alignas(64) UpdX {
+    int64_t a;     // coefficient index of source row p0 (row q0: a + dq)
+    int64_t c;     // coefficient index of the target panel
+    int64_t rb;    // row-map index of source row p0 (row q0: rb + dq)
+    int32_t K, ld, stf, np, nq, dq;
+    int32_t sbi;   // source row p lands on row panel_grow + shift[sbi + panel_blk]
+    int32_t fcol;  // first column of the target
+};
+
 // Product group of a source s and the run of its blocks facing one target
 // (first block ib0): the dense product P(p, q) = A(p, :) . B(q, :)^T over the
 // source panel rows p in [roff(ib0), stride) and q in [roff(ib0), roff(ib0)+nq),

@@ -12,8 +12,8 @@ namespace pxa {
     for (int m_ = 0; m_ < 2; m_++)                                       \
         for (int n_ = 0; n_ < 2; n_++)                                   \
             for (int r_ = 0; r_ < 4; r_++) {                             \
-                const int qrow = 2 * Mfma<T>::drow(lane, r_) + m_;        \
-                const int qcol = 2 * (lane & 15) + n_;                    \
+                const int qrow = m_ * 16 + Mfma<T>::drow(lane, r_);       \
+                const int qcol = n_ * 16 + (lane & 15);                   \
                 __VA_ARGS__                                              \
             }
 

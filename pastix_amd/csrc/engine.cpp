@@ -169,7 +169,6 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
         d_leaf_ctr_ = (int32_t *)alloc(std::max<int64_t>(cblknbr_, 1) * sizeof(int32_t));
         d_leaf_queue_ = (int32_t *)alloc(std::max<int32_t>(P.leaf_n, 1) * sizeof(int32_t));
         d_leaf_sync_ = (int32_t *)alloc(4 * sizeof(int32_t));
-        d_leaf_out_ = upload(*this, P.leaf_out);
         n_leaf_out_ = (int32_t)P.leaf_out.size();
         leaf_out_split_ = P.leaf_out_split;
         if (!leaf_.in_ptr || !leaf_.tgt_ptr || !leaf_.ctr0 || !leaf_.init || !d_leaf_ctr_ || !d_leaf_queue_ ||
@@ -203,7 +202,6 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     d_ydst_ = upload(*this, P.ydst);
     nyrows_ = P.nyrows;
     d_shift_ = upload(*this, P.shift);
-    d_upd_ = upload(*this, P.upd);
     d_ents_ = upload(*this, P.ents);
     d_fwd_ = upload(*this, P.fwd);
     d_diag_ = upload(*this, P.diag);
@@ -221,8 +219,6 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     d_wgrp_ = upload(*this, P.wgrp);
     d_wtiles_ = upload(*this, P.wtiles);
     lv_wt_ptr_ = P.lv_wt_ptr;
-    lv_wsize_ = P.lv_wsize;
-    lv_single_pass_ = P.lv_single_pass;
 
     const size_t fsz = (prec_ == 2) ? sizeof(float) : sizeof(double);
     // level workspace of the two-phase update: the largest level's products,
@@ -237,6 +233,54 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
             d_wspace_ = alloc((size_t)wcap_ * fsz);
             if (!d_wspace_) return -1;
         }
+    }
+    {
+        // the one-pass kernels' entries in one line each, in item order: item
+        // t's first at upd_x_[t] (single-entry items of a range side by side);
+        // the multi-entry items among them point at theirs.  Two-phase items
+        // keep the plan's entries.
+        std::vector<UpdX> xs;
+        std::vector<UpdItem> items = P.upd;
+        auto entry = [&](const UpdItem &it, const UpdEntry &en) {
+            const int32_t f = it.f, ss = en.s;
+            UpdX x{};
+            x.a = L.cblk_coef[ss] + en.p0;
+            x.c = L.cblk_coef[f];
+            x.rb = P.rowbase[ss] + en.p0;
+            x.K = (int32_t)(s.cblk_fcol[ss + 1] - s.cblk_fcol[ss]);
+            x.ld = (int32_t)L.cblk_stride[ss];
+            x.stf = (int32_t)L.cblk_stride[f];
+            x.np = en.p1 - en.p0;
+            x.nq = en.q1 - en.q0;
+            x.dq = en.q0 - en.p0;
+            x.sbi = en.sb - en.ib0;
+            x.fcol = (int32_t)s.cblk_fcol[f];
+            xs.push_back(x);
+        };
+        auto take = [&](UpdItem &it) -> int32_t {
+            const int32_t x0 = (int32_t)xs.size();
+            for (int32_t e = it.e0; e < it.e1; e++) entry(it, P.ents[e]);
+            it.e0 = x0;
+            it.e1 = (int32_t)xs.size();
+            return x0;
+        };
+        upd_x_.assign(items.size() + 1, 0);
+        lv_two_phase_.assign(P.nlevels, 0);
+        for (int32_t lv = 0; lv < P.nlevels; lv++) {
+            // two-phase levels: their products fit the workspace
+            lv_two_phase_[lv] = P.lv_upd_ptr[lv + 1] > P.lv_upd_split[lv] && !P.lv_single_pass[lv] &&
+                                P.lv_wsize[lv] <= wcap_;
+            const int32_t end = lv_two_phase_[lv] ? P.lv_upd_split[lv] : P.lv_upd_ptr[lv + 1];
+            for (int32_t t = P.lv_upd_ptr[lv]; t < end; t++) upd_x_[t] = take(items[t]);
+        }
+        std::vector<UpdItem> leaf_out = P.leaf_out;
+        leaf_out_x_ = (int32_t)xs.size();
+        if (leaf_levels_ > 0)
+            for (UpdItem &it : leaf_out) take(it);
+        d_upd_ = upload(*this, items);
+        d_updx_ = upload(*this, xs);
+        if (leaf_levels_ > 0) d_leaf_out_ = upload(*this, leaf_out);
+        if (!d_upd_ || !d_updx_) return -1;
     }
     d_L_ = alloc(coefnbr_ * fsz);
     d_W1_ = alloc(winvnbr_ * fsz);
@@ -398,13 +442,13 @@ template <typename T> int Engine::factorize_t(double thr) {
         prof_end(KC_LEAF, pk, stream_);
         if (leaf_out_split_ > 0) {
             pk = prof_begin(stream_);
-            launch_update<T>(S_, 0, true, d_leaf_out_, leaf_out_split_, d_ents_, d_shift_, L, L, L, stream_);
+            launch_update_direct<T>(S_, 0, d_updx_ + leaf_out_x_, leaf_out_split_, d_shift_, L, L, L, stream_);
             prof_end(KC_DIRECT, pk, stream_);
         }
         if (n_leaf_out_ > leaf_out_split_) {
             pk = prof_begin(stream_);
-            launch_update<T>(S_, 0, false, d_leaf_out_ + leaf_out_split_, n_leaf_out_ - leaf_out_split_, d_ents_,
-                             d_shift_, L, L, L, stream_);
+            launch_update_seq<T>(S_, 0, d_leaf_out_ + leaf_out_split_, n_leaf_out_ - leaf_out_split_, d_updx_,
+                                 d_shift_, L, L, L, stream_);
             prof_end(KC_ACC, pk, stream_);
         }
         lv_first = (size_t)leaf_levels_;
@@ -460,7 +504,7 @@ template <typename T> int Engine::factorize_t(double thr) {
         prof_end(KC_PANEL, pk, stream_);
         const int u0 = lv_upd_ptr_[lv], us = lv_upd_split_[lv], u1 = lv_upd_ptr_[lv + 1];
         const int w0 = lv_wt_ptr_[lv], w1 = lv_wt_ptr_[lv + 1];
-        const bool two_phase = u1 > us && !lv_single_pass_[lv] && lv_wsize_[lv] <= wcap_;
+        const bool two_phase = lv_two_phase_[lv] != 0;
         T *Wk = (T *)d_wspace_;
         // one side of an update range: direct tiles [da, db), multi-source
         // tiles [ma, mb) with their product tiles [wa, wb); (A, B) are the
@@ -470,7 +514,7 @@ template <typename T> int Engine::factorize_t(double thr) {
             int k;
             if (db > da) {
                 k = prof_begin(st);
-                launch_update<T>(S_, mode, true, d_upd_ + da, db - da, d_ents_, d_shift_, A, B, C, st);
+                launch_update_direct<T>(S_, mode, d_updx_ + upd_x_[da], db - da, d_shift_, A, B, C, st);
                 prof_end(KC_DIRECT, k, st);
             }
             if (mb == ma) return;
@@ -485,7 +529,7 @@ template <typename T> int Engine::factorize_t(double thr) {
                 prof_end(KC_GATHER, k, st);
             } else {
                 k = prof_begin(st);
-                launch_update<T>(S_, mode, false, d_upd_ + ma, mb - ma, d_ents_, d_shift_, A, B, C, st);
+                launch_update_seq<T>(S_, mode, d_upd_ + ma, mb - ma, d_updx_, d_shift_, A, B, C, st);
                 prof_end(KC_ACC, k, st);
             }
         };

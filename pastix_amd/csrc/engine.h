@@ -230,12 +230,13 @@ class Engine {
     PanelItem *d_ptrsm_ = nullptr, *d_pupd_ = nullptr;
     UpdItem *d_upd_ = nullptr;
     UpdEntry *d_ents_ = nullptr;
+    UpdX *d_updx_ = nullptr;        // one-pass entries, item t's first at upd_x_[t]
+    std::vector<int32_t> upd_x_;
+    std::vector<uint8_t> lv_two_phase_;
     // two-phase multi-source update: product groups, tiles, level workspace
     WGroup *d_wgrp_ = nullptr;
     WTile *d_wtiles_ = nullptr;
     std::vector<int32_t> lv_wt_ptr_;
-    std::vector<int64_t> lv_wsize_;
-    std::vector<uint8_t> lv_single_pass_;
     void *d_wspace_ = nullptr;
     int64_t wcap_ = 0;  // workspace entries
     // leaf region (LL^t): task lists, counters, ready queue, the updates it
@@ -245,6 +246,7 @@ class Engine {
     long long leaf_maxwait_ = 0;  // wall-clock ticks of one wait in that launch (two seconds)
     int32_t *d_leaf_ctr_ = nullptr, *d_leaf_queue_ = nullptr, *d_leaf_sync_ = nullptr;
     UpdItem *d_leaf_out_ = nullptr;
+    int32_t leaf_out_x_ = 0;  // their entries in d_updx_
     int32_t n_leaf_out_ = 0, leaf_out_split_ = 0;
     FwdItem *d_fwd_ = nullptr;
     DiagItem *d_diag_ = nullptr;

@@ -29,8 +29,8 @@ namespace pxa {
     for (int m_ = 0; m_ < 2; m_++)                                       \
         for (int n_ = 0; n_ < 2; n_++)                                   \
             for (int r_ = 0; r_ < 4; r_++) {                             \
-                const int qrow = 2 * Mfma<T>::drow(lane, r_) + m_;        \
-                const int qcol = 2 * (lane & 15) + n_;                    \
+                const int qrow = m_ * 16 + Mfma<T>::drow(lane, r_);       \
+                const int qcol = n_ * 16 + (lane & 15);                   \
                 __VA_ARGS__                                              \
             }
 
@@ -606,7 +606,7 @@ __device__ __forceinline__ void wg_gemm_lds_xcol_yt(Quad<T> &q, XCol &xcol, int 
                                                     int K, StageBuf<T, CH> &sb, int tid) {
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    const int i = 2 * (lane & 15), kq = lane >> 4;
+    const int i = lane & 15, kq = lane >> 4;
     constexpr int E = Vec<T>::E, NP = CH / (4 * E), NY = CH / 4;
     const int re = E * (tid % (64 / E)), ke = tid / (64 / E);
     // Y: thread (row yr, k group yk) fetches NY consecutive k of its row

@@ -8,11 +8,8 @@
 //   k_update_direct : tiles fed by a single source: the product is kept in
 //                     registers (computed transposed so that stores walk down
 //                     target columns) and subtracted straight into C;
-//   k_update_seq    : tiles fed by several sources (FP64): each entry's
-//                     product as in k_update_direct, subtracted into C in
-//                     entry order;
-//   k_update_acc    : tiles fed by several sources (FP32): contributions are
-//                     summed in an LDS tile, written once at the end.
+//   k_update_seq    : tiles fed by several sources: each entry's product as
+//                     in k_update_direct, subtracted into C in entry order.
 // MODE 0 (LL^t and the L side of LU) keeps pairs with block(p) >= block(q),
 // MODE 1 (U side of LU) keeps block(p) > block(q), as the reference's
 // iterblok >= blok / iterblok > blok loops.
@@ -29,42 +26,70 @@ namespace pxa {
 // two of 16 slower, 24.0 against 21.9 ms).
 constexpr int UPD_CH = 16;
 
+// One entry's product minus from the target: up to 64 source rows p x 64
+// source columns q, computed transposed, D(j, i) = B(q_j) . A(p_i), so that
+// stores walk down target columns.  The row and column maps are fetched
+// before the product and published after it: their loads (two deep) run
+// under the first chunks.  Bound by the matrix cores (65 to 80 % busy) with
+// the rest in the tiles' first and last memory round trips: 80^3 Laplacian,
+// FP64, one stream, k_update_direct 20.9 ms (47 TFLOP/s; 21.9 with the maps
+// before the product and the descriptors behind three loads), k_update_seq
+// 14.0 ms (47 TFLOP/s); FP32 on 61x57x66 2.75 and 1.87 ms (the sum in an LDS
+// tile, one write of C for all entries, took 2.07).  Fire-and-forget atomic
+// subtraction instead of the load was slower.
+template <typename T> struct UpdLds {
+    StageBuf<T, UPD_CH> sb;
+    int rmap[64], cmap[64], rblk[64], qblk[64];
+};
+template <typename T, int MODE>
+__device__ __forceinline__ void update_entry(const DevSymbol &S, const UpdX &x, const int32_t *__restrict__ shift,
+                                             const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
+                                             T *__restrict__ Ccoef, UpdLds<T> &l, int tid) {
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+    int mrow = 0, mblk = 0;
+    if (tid < 128) {
+        const int64_t r = x.rb + (tid < 64 ? min(lane, x.np - 1) : x.dq + min(lane, x.nq - 1));
+        mblk = S.panel_blk[r];
+        mrow = S.panel_grow[r];
+    }
+    GemmLds<T, UPD_CH> g;
+    g.start(Bcoef + x.a + x.dq, x.nq, x.ld, Acoef + x.a, x.np, x.ld, x.K, tid);
+    if (tid < 64) mrow += shift[x.sbi + mblk];
+    else mrow -= x.fcol;
+    Quad<T> q;
+    q.zero();
+    g.run(q, l.sb, tid);
+    if (tid < 64) {
+        l.rmap[lane] = mrow;
+        l.rblk[lane] = mblk;
+    } else if (tid < 128) {
+        l.cmap[lane] = mrow;
+        l.qblk[lane] = mblk;
+    }
+    __syncthreads();
+    if (wr < x.nq && wc < x.np) {
+        const int64_t stf = x.stf;
+        T *C = Ccoef + x.c;
+        quad_sub(q, lane, [&](int qrow, int qcol, bool &ok) -> T * {
+            const int qj = wr + qrow, pi = wc + qcol;
+            ok = qj < x.nq && pi < x.np && ((MODE == 0) ? (l.rblk[pi] >= l.qblk[qj]) : (l.rblk[pi] > l.qblk[qj]));
+            return ok ? C + l.rmap[pi] + (int64_t)l.cmap[qj] * stf : C;
+        });
+    }
+}
+
 // register budget held to seven waves per SIMD (72 registers in FP64, no
 // spills; the compiler's own choice, 80, allows six): 54.4 -> 53.9 ms FP64
 // numfact on the 80^3 Laplacian
 template <typename T, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_update_direct(DevSymbol S, const UpdItem *__restrict__ items, int nitems,
-                                                       const UpdEntry *__restrict__ ents,
-                                                       const int32_t *__restrict__ shift, const T *__restrict__ Acoef,
-                                                       const T *__restrict__ Bcoef, T *__restrict__ Ccoef) {
-    __shared__ StageBuf<T, UPD_CH> sb;
-    __shared__ int rmap[64], cmap[64], rblk[64], qblk[64];
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_update_direct(
+    DevSymbol S, const UpdX *__restrict__ xs, int nitems, const int32_t *__restrict__ shift,
+    const T *__restrict__ Acoef, const T *__restrict__ Bcoef, T *__restrict__ Ccoef) {
+    __shared__ UpdLds<T> lds;
     const int id = xcd_remap(blockIdx.x, gridDim.x);
     if (id >= nitems) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    const UpdItem it = items[id];
-    const int f = it.f, r0 = it.r0, c0 = it.c0;
-    const int fcol = S.cblk_fcol[f];
-    const UpdEntry en = ents[it.e0];
-    update_maps(S, en, shift, r0, fcol + c0, rmap, cmap, rblk, qblk, tid);
-    const int s = en.s;
-    const int np = en.p1 - en.p0, nq = en.q1 - en.q0;
-    const int K = S.cblk_fcol[s + 1] - S.cblk_fcol[s];
-    const int64_t ld = S.cblk_stride[s];
-    Quad<T> q;
-    q.zero();
-    // D(j, i) = B(q_j) . A(p_i): quadrant rows index columns of the target
-    wg_gemm_lds<T, UPD_CH>(q, Bcoef + S.cblk_coef[s] + en.q0, nq, ld, Acoef + S.cblk_coef[s] + en.p0, np, ld, K, sb, tid);
-    const int64_t stf = S.cblk_stride[f];
-    T *C = Ccoef + S.cblk_coef[f] + r0 + (int64_t)c0 * stf;
-    if (wr < nq && wc < np) {
-        quad_sub(q, lane, [&](int qrow, int qcol, bool &ok) -> T * {
-            const int qj = wr + qrow, pi = wc + qcol;
-            ok = qj < nq && pi < np && ((MODE == 0) ? (rblk[pi] >= qblk[qj]) : (rblk[pi] > qblk[qj]));
-            return ok ? C + rmap[pi] + (int64_t)cmap[qj] * stf : C;
-        });
-    }
+    update_entry<T, MODE>(S, xs[id], shift, Acoef, Bcoef, Ccoef, lds, threadIdx.x);
 }
 
 // Tiles fed by several sources: the entries in order, each one's product
@@ -74,54 +99,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
 // element another wave wrote sees it.  The direct kernel's LDS footprint
 // (no 64x64 accumulator), so six waves per SIMD instead of three.
 template <typename T, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_update_seq(DevSymbol S, const UpdItem *__restrict__ items, int nitems,
-                                                    const UpdEntry *__restrict__ ents, const int32_t *__restrict__ shift,
-                                                    const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
-                                                    T *__restrict__ Ccoef) {
-    __shared__ StageBuf<T, UPD_CH> sb;
-    __shared__ int rmap[64], cmap[64], rblk[64], qblk[64];
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_update_seq(
+    DevSymbol S, const UpdItem *__restrict__ items, int nitems, const UpdX *__restrict__ xs,
+    const int32_t *__restrict__ shift, const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
+    T *__restrict__ Ccoef) {
+    __shared__ UpdLds<T> lds;
     const int id = xcd_remap(blockIdx.x, gridDim.x);
     if (id >= nitems) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    const UpdItem it = items[id];
-    const int f = it.f, r0 = it.r0, c0 = it.c0;
-    const int fcol = S.cblk_fcol[f];
-    const int64_t stf = S.cblk_stride[f];
-    T *C = Ccoef + S.cblk_coef[f] + r0 + (int64_t)c0 * stf;
-    for (int e = it.e0; e < it.e1; e++) {
+    const int e0 = items[id].e0, e1 = items[id].e1;
+    for (int e = e0; e < e1; e++) {
         // the previous entry's stores and map reads are done by every wave
-        if (e > it.e0) __syncthreads();
-        const UpdEntry en = ents[e];
-        update_maps(S, en, shift, r0, fcol + c0, rmap, cmap, rblk, qblk, tid);
-        const int s = en.s;
-        const int np = en.p1 - en.p0, nq = en.q1 - en.q0;
-        const int K = S.cblk_fcol[s + 1] - S.cblk_fcol[s];
-        const int64_t ld = S.cblk_stride[s];
-        Quad<T> q;
-        q.zero();
-        // D(j, i) = B(q_j) . A(p_i): quadrant rows index columns of the target
-        wg_gemm_lds<T, UPD_CH>(q, Bcoef + S.cblk_coef[s] + en.q0, nq, ld, Acoef + S.cblk_coef[s] + en.p0, np, ld, K,
-                               sb, tid);
-        if (wr < nq && wc < np) {
-            quad_sub(q, lane, [&](int qrow, int qcol, bool &ok) -> T * {
-                const int qj = wr + qrow, pi = wc + qcol;
-                ok = qj < nq && pi < np && ((MODE == 0) ? (rblk[pi] >= qblk[qj]) : (rblk[pi] > qblk[qj]));
-                return ok ? C + rmap[pi] + (int64_t)cmap[qj] * stf : C;
-            });
-        }
+        if (e > e0) __syncthreads();
+        update_entry<T, MODE>(S, xs[e], shift, Acoef, Bcoef, Ccoef, lds, threadIdx.x);
     }
-}
-
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) void k_update_acc(DevSymbol S, const UpdItem *__restrict__ items, int nitems,
-                                                    const UpdEntry *__restrict__ ents, const int32_t *__restrict__ shift,
-                                                    const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
-                                                    T *__restrict__ Ccoef) {
-    __shared__ UpdAccLds<T> lds;
-    const int id = xcd_remap(blockIdx.x, gridDim.x);
-    if (id >= nitems) return;
-    update_acc_tile<T, MODE>(S, items[id], ents, shift, Acoef, Bcoef, Ccoef, lds);
 }
 
 // Phase 1 of the multi-source tiles: dense 128 (p) x 64 (q) tile of a
@@ -303,26 +293,21 @@ __global__ __launch_bounds__(256) void k_update_gather(DevSymbol S, const UpdIte
 static inline int grid8(int n) { return ((n + 7) / 8) * 8; }
 
 template <typename T>
-void launch_update(const DevSymbol &S, int mode, bool direct, const UpdItem *items, int n, const UpdEntry *ents,
-                   const int32_t *shift, const T *A, const T *B, T *C, hipStream_t st) {
+void launch_update_direct(const DevSymbol &S, int mode, const UpdX *xs, int n, const int32_t *shift, const T *A,
+                          const T *B, T *C, hipStream_t st) {
     if (n <= 0) return;
     const dim3 g(grid8(n)), b(256);
-    if (direct) {
-        if (mode == 0) hipLaunchKernelGGL((k_update_direct<T, 0>), g, b, 0, st, S, items, n, ents, shift, A, B, C);
-        else hipLaunchKernelGGL((k_update_direct<T, 1>), g, b, 0, st, S, items, n, ents, shift, A, B, C);
-    } else {
-        // FP64: entries subtracted in turn (six waves per SIMD; the LDS
-        // accumulator's 52 KB allow three): 56.0 -> 54.3 ms numfact on the
-        // 80^3 Laplacian.  FP32: the accumulator (26 KB, six waves already)
-        // saves the extra read-modify-writes of C: 33.1 against 33.5 ms.
-        if constexpr (sizeof(T) == 8) {
-            if (mode == 0) hipLaunchKernelGGL((k_update_seq<T, 0>), g, b, 0, st, S, items, n, ents, shift, A, B, C);
-            else hipLaunchKernelGGL((k_update_seq<T, 1>), g, b, 0, st, S, items, n, ents, shift, A, B, C);
-        } else {
-            if (mode == 0) hipLaunchKernelGGL((k_update_acc<T, 0>), g, b, 0, st, S, items, n, ents, shift, A, B, C);
-            else hipLaunchKernelGGL((k_update_acc<T, 1>), g, b, 0, st, S, items, n, ents, shift, A, B, C);
-        }
-    }
+    if (mode == 0) hipLaunchKernelGGL((k_update_direct<T, 0>), g, b, 0, st, S, xs, n, shift, A, B, C);
+    else hipLaunchKernelGGL((k_update_direct<T, 1>), g, b, 0, st, S, xs, n, shift, A, B, C);
+}
+
+template <typename T>
+void launch_update_seq(const DevSymbol &S, int mode, const UpdItem *items, int n, const UpdX *xs,
+                       const int32_t *shift, const T *A, const T *B, T *C, hipStream_t st) {
+    if (n <= 0) return;
+    const dim3 g(grid8(n)), b(256);
+    if (mode == 0) hipLaunchKernelGGL((k_update_seq<T, 0>), g, b, 0, st, S, items, n, xs, shift, A, B, C);
+    else hipLaunchKernelGGL((k_update_seq<T, 1>), g, b, 0, st, S, items, n, xs, shift, A, B, C);
 }
 
 template <typename T>
@@ -341,8 +326,10 @@ void launch_update_gather(const DevSymbol &S, int mode, const UpdItem *items, in
 }
 
 #define PXA_UPD_INST(T)                                                                                           \
-    template void launch_update<T>(const DevSymbol &, int, bool, const UpdItem *, int, const UpdEntry *,          \
-                                   const int32_t *, const T *, const T *, T *, hipStream_t);                      \
+    template void launch_update_direct<T>(const DevSymbol &, int, const UpdX *, int, const int32_t *, const T *,  \
+                                          const T *, T *, hipStream_t);                                           \
+    template void launch_update_seq<T>(const DevSymbol &, int, const UpdItem *, int, const UpdX *,                \
+                                       const int32_t *, const T *, const T *, T *, hipStream_t);                  \
     template void launch_update_wgemm<T>(const DevSymbol &, const WTile *, int, const T *, const T *, T *,        \
                                          hipStream_t);                                                            \
     template void launch_update_gather<T>(const DevSymbol &, int, const UpdItem *, int, const UpdEntry *,         \
