@@ -442,13 +442,13 @@ template <typename T> int Engine::factorize_t(double thr) {
         prof_end(KC_LEAF, pk, stream_);
         if (leaf_out_split_ > 0) {
             pk = prof_begin(stream_);
-            launch_update_direct<T>(S_, 0, d_updx_ + leaf_out_x_, leaf_out_split_, d_shift_, L, L, L, stream_);
+            launch_update_direct<T>(S_, 0, d_updx_ + leaf_out_x_, leaf_out_split_, d_shift_, L, L, L, false, stream_);
             prof_end(KC_DIRECT, pk, stream_);
         }
         if (n_leaf_out_ > leaf_out_split_) {
             pk = prof_begin(stream_);
             launch_update_seq<T>(S_, 0, d_leaf_out_ + leaf_out_split_, n_leaf_out_ - leaf_out_split_, d_updx_,
-                                 d_shift_, L, L, L, stream_);
+                                 d_shift_, L, L, L, false, stream_);
             prof_end(KC_ACC, pk, stream_);
         }
         lv_first = (size_t)leaf_levels_;
@@ -514,7 +514,7 @@ template <typename T> int Engine::factorize_t(double thr) {
             int k;
             if (db > da) {
                 k = prof_begin(st);
-                launch_update_direct<T>(S_, mode, d_updx_ + upd_x_[da], db - da, d_shift_, A, B, C, st);
+                launch_update_direct<T>(S_, mode, d_updx_ + upd_x_[da], db - da, d_shift_, A, B, C, st == side_, st);
                 prof_end(KC_DIRECT, k, st);
             }
             if (mb == ma) return;
@@ -529,7 +529,7 @@ template <typename T> int Engine::factorize_t(double thr) {
                 prof_end(KC_GATHER, k, st);
             } else {
                 k = prof_begin(st);
-                launch_update_seq<T>(S_, mode, d_upd_ + ma, mb - ma, d_updx_, d_shift_, A, B, C, st);
+                launch_update_seq<T>(S_, mode, d_upd_ + ma, mb - ma, d_updx_, d_shift_, A, B, C, st == side_, st);
                 prof_end(KC_ACC, k, st);
             }
         };

@@ -10,10 +10,10 @@ namespace pxa {
 // direct: every item has exactly one entry (no LDS accumulation).
 template <typename T>
 void launch_update_direct(const DevSymbol &S, int mode, const UpdX *xs, int n, const int32_t *shift, const T *A,
-                          const T *B, T *C, hipStream_t st);
+                          const T *B, T *C, bool beside, hipStream_t st);
 template <typename T>
 void launch_update_seq(const DevSymbol &S, int mode, const UpdItem *items, int n, const UpdX *xs,
-                       const int32_t *shift, const T *A, const T *B, T *C, hipStream_t st);
+                       const int32_t *shift, const T *A, const T *B, T *C, bool beside, hipStream_t st);
 // Two-phase update of the multi-source tiles: dense product tiles into the
 // level workspace W, then the per-target-tile ordered sum.
 template <typename T>

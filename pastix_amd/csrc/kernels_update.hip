@@ -292,22 +292,35 @@ __global__ __launch_bounds__(256) void k_update_gather(DevSymbol S, const UpdIte
 
 static inline int grid8(int n) { return ((n + 7) / 8) * 8; }
 
+// LDS of an update workgroup that runs beside the panel kernels (`beside`,
+// the second stream): unused space rounds it up so that five of them fill a
+// CU.  At the seven that the registers allow, a panel kernel of a few
+// workgroups (a diagonal block takes 42 KB and a wave of 124 registers on
+// every SIMD) waits for a CU to drain: k_potrf64 took 90-186 us beside the
+// updates, 22 us alone, and the level's other panels wait for it.
+// Factorisation of an 80^3 Laplacian with 7 / 6 / 5 / 3 workgroups per CU:
+// 49.9 / 49.1 / 48.4 / 50.0 ms; in FP32 (61x57x66), with 8 / 6 / 5: 10.05 /
+// 9.88 / 9.69 ms; LU of 48^3 13.7 ms with either.
+constexpr size_t BESIDE_LDS = 32768;
+
 template <typename T>
 void launch_update_direct(const DevSymbol &S, int mode, const UpdX *xs, int n, const int32_t *shift, const T *A,
-                          const T *B, T *C, hipStream_t st) {
+                          const T *B, T *C, bool beside, hipStream_t st) {
     if (n <= 0) return;
     const dim3 g(grid8(n)), b(256);
-    if (mode == 0) hipLaunchKernelGGL((k_update_direct<T, 0>), g, b, 0, st, S, xs, n, shift, A, B, C);
-    else hipLaunchKernelGGL((k_update_direct<T, 1>), g, b, 0, st, S, xs, n, shift, A, B, C);
+    const size_t lds = beside ? BESIDE_LDS - sizeof(UpdLds<T>) : 0;
+    if (mode == 0) hipLaunchKernelGGL((k_update_direct<T, 0>), g, b, lds, st, S, xs, n, shift, A, B, C);
+    else hipLaunchKernelGGL((k_update_direct<T, 1>), g, b, lds, st, S, xs, n, shift, A, B, C);
 }
 
 template <typename T>
 void launch_update_seq(const DevSymbol &S, int mode, const UpdItem *items, int n, const UpdX *xs,
-                       const int32_t *shift, const T *A, const T *B, T *C, hipStream_t st) {
+                       const int32_t *shift, const T *A, const T *B, T *C, bool beside, hipStream_t st) {
     if (n <= 0) return;
     const dim3 g(grid8(n)), b(256);
-    if (mode == 0) hipLaunchKernelGGL((k_update_seq<T, 0>), g, b, 0, st, S, items, n, xs, shift, A, B, C);
-    else hipLaunchKernelGGL((k_update_seq<T, 1>), g, b, 0, st, S, items, n, xs, shift, A, B, C);
+    const size_t lds = beside ? BESIDE_LDS - sizeof(UpdLds<T>) : 0;
+    if (mode == 0) hipLaunchKernelGGL((k_update_seq<T, 0>), g, b, lds, st, S, items, n, xs, shift, A, B, C);
+    else hipLaunchKernelGGL((k_update_seq<T, 1>), g, b, lds, st, S, items, n, xs, shift, A, B, C);
 }
 
 template <typename T>
@@ -327,9 +340,9 @@ void launch_update_gather(const DevSymbol &S, int mode, const UpdItem *items, in
 
 #define PXA_UPD_INST(T)                                                                                           \
     template void launch_update_direct<T>(const DevSymbol &, int, const UpdX *, int, const int32_t *, const T *,  \
-                                          const T *, T *, hipStream_t);                                           \
+                                          const T *, T *, bool, hipStream_t);                                     \
     template void launch_update_seq<T>(const DevSymbol &, int, const UpdItem *, int, const UpdX *,                \
-                                       const int32_t *, const T *, const T *, T *, hipStream_t);                  \
+                                       const int32_t *, const T *, const T *, T *, bool, hipStream_t);            \
     template void launch_update_wgemm<T>(const DevSymbol &, const WTile *, int, const T *, const T *, T *,        \
                                          hipStream_t);                                                            \
     template void launch_update_gather<T>(const DevSymbol &, int, const UpdItem *, int, const UpdEntry *,         \
