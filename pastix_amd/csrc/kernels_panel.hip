@@ -98,16 +98,14 @@ __device__ __forceinline__ float rlane(float v, int lane) {
 // One joining level of the recursive-doubling inverse below, on the vector
 // units: for every pair of inverted diagonal blocks of size B (X11 at
 // [base, base+B), X22 at [base+B, base+2B)), X21 = -X22 (M21 X11).
-template <typename T, int B, bool TRANS>
-__device__ __forceinline__ void inv_join_valu(T (*Ls)[65], T (*Xs)[65], T *Ts, int tid) {
+template <typename T, int B> __device__ __forceinline__ void inv_join_valu(T (*Xs)[65], T *Ts, int tid) {
     constexpr int NO = 32 * B;  // outputs of the level: 64/(2B) pairs of B x B
-    auto M = [&](int r, int k) -> T { return TRANS ? Ls[k][r] : Ls[r][k]; };
     const int o = tid;
     const int p = o / (B * B), rem = o % (B * B), r = rem / B, cc = rem % B, base = 2 * B * p;
     if (o < NO) {
         T s = (T)0;
 #pragma unroll
-        for (int m = 0; m < B; m++) s = fma_(M(base + B + r, base + m), Xs[base + m][base + cc], s);
+        for (int m = 0; m < B; m++) s = fma_(Xs[base + B + r][base + m], Xs[base + m][base + cc], s);
         Ts[o] = s;
     }
     __syncthreads();
@@ -121,10 +119,8 @@ __device__ __forceinline__ void inv_join_valu(T (*Ls)[65], T (*Xs)[65], T *Ts, i
 }
 
 // The same on the matrix cores for B = 16, 32: one 16x16 tile per wave.
-template <typename T, int B, bool TRANS>
-__device__ __forceinline__ void inv_join_mfma(T (*Ls)[65], T (*Xs)[65], T *Ts, int lane, int w) {
+template <typename T, int B> __device__ __forceinline__ void inv_join_mfma(T (*Xs)[65], T *Ts, int lane, int w) {
     constexpr int TPP = (B / 16) * (B / 16), NT = (64 / (2 * B)) * TPP;
-    auto M = [&](int r, int k) -> T { return TRANS ? Ls[k][r] : Ls[r][k]; };
     const int i = lane & 15, kq = lane >> 4;
     const int p = w / TPP, ti = (w % TPP) / (B / 16), tj = w % (B / 16), base = 2 * B * p;
     if (w < NT) {
@@ -132,7 +128,7 @@ __device__ __forceinline__ void inv_join_mfma(T (*Ls)[65], T (*Xs)[65], T *Ts, i
 #pragma unroll
         for (int s = 0; s < B / 4; s++) {
             const int k = 4 * s + kq;
-            acc = Mfma<T>::mma(M(base + B + ti * 16 + i, base + k), Xs[base + k][base + tj * 16 + i], acc);
+            acc = Mfma<T>::mma(Xs[base + B + ti * 16 + i][base + k], Xs[base + k][base + tj * 16 + i], acc);
         }
 #pragma unroll
         for (int r = 0; r < 4; r++) Ts[p * B * B + (ti * 16 + Mfma<T>::drow(lane, r)) * B + tj * 16 + i] = acc[r];
@@ -151,35 +147,25 @@ __device__ __forceinline__ void inv_join_mfma(T (*Ls)[65], T (*Xs)[65], T *Ts, i
     __syncthreads();
 }
 
-// X = inv(M) for the lower-triangular 64x64 M held in Ls (M(r, k) = Ls[r][k],
-// or Ls[k][r] when TRANS; unit diagonal when UNIT, else 1/M(r, r) = dinv[r])
-// by recursive doubling: the sixteen 4x4 diagonal blocks are inverted
-// directly, then pairs of inverted blocks of size 4, 8, 16 and 32 are joined
+// X = inv(M) in place for the lower-triangular 64x64 M held in Xs, zeros
+// above the diagonal (1/M(r, r) = dinv[r]), by recursive doubling: the
+// sixteen 4x4 diagonal blocks are inverted directly, then pairs of inverted
+// blocks of size 4, 8, 16 and 32 are joined
 // (inv([M11 0; M21 M22]) = [X11 0; -X22 M21 X11 X22]): 4 levels of small
-// products instead of a 64-step substitution.  Xs receives X with zeros above
-// the diagonal; Ts (1024 entries) is scratch.  With INPLACE (not TRANS), Xs
-// is Ls, whose upper triangle the caller has zeroed: every join overwrites
-// the block M21 it has consumed, and only M21 blocks are read from M after
-// the 4x4 blocks.  Only X[0:nb, 0:nb] is complete: levels that would join
-// blocks of the identity padding only are skipped.  All 256 threads (nb
-// uniform), barriers inside; Ls and dinv must be visible to all threads on
-// entry.
-template <typename T, bool UNIT, bool TRANS, bool INPLACE>
-__device__ __forceinline__ void lower_inverse(T (*Ls)[65], T (*Xs)[65], T *Ts, const T *dinv, int nb, int tid,
-                                              int w) {
-    static_assert(!(INPLACE && TRANS), "in place only from the lower triangle");
-    auto M = [&](int r, int k) -> T { return TRANS ? Ls[k][r] : Ls[r][k]; };
-    if (!INPLACE) {
-        for (int e = tid; e < 64 * 64; e += 256) Xs[e >> 6][e & 63] = (T)0;
-        __syncthreads();
-    }
+// products instead of a 64-step substitution.  Every join overwrites the
+// block M21 it has consumed, and only M21 blocks are read from M after the
+// 4x4 blocks.  Ts (1024 entries) is scratch.  Only X[0:nb, 0:nb] is complete:
+// levels that would join blocks of the identity padding only are skipped.
+// All 256 threads (nb uniform), barriers inside; Xs and dinv must be visible
+// to all threads on entry.
+template <typename T>
+__device__ __forceinline__ void lower_inverse(T (*Xs)[65], T *Ts, const T *dinv, int nb, int tid, int w) {
     if (tid < 64) {
         // one wave; the block's strict lower entries are read before any write
         const int b0 = 4 * (tid >> 2), cc = tid & 3;
-        const T m10 = M(b0 + 1, b0), m20 = M(b0 + 2, b0), m21 = M(b0 + 2, b0 + 1);
-        const T m30 = M(b0 + 3, b0), m31 = M(b0 + 3, b0 + 1), m32 = M(b0 + 3, b0 + 2);
-        const T d0 = UNIT ? (T)1 : dinv[b0], d1 = UNIT ? (T)1 : dinv[b0 + 1];
-        const T d2 = UNIT ? (T)1 : dinv[b0 + 2], d3 = UNIT ? (T)1 : dinv[b0 + 3];
+        auto M = [&](int r, int k) -> T { return Xs[b0 + r][b0 + k]; };
+        const T m10 = M(1, 0), m20 = M(2, 0), m21 = M(2, 1), m30 = M(3, 0), m31 = M(3, 1), m32 = M(3, 2);
+        const T d0 = dinv[b0], d1 = dinv[b0 + 1], d2 = dinv[b0 + 2], d3 = dinv[b0 + 3];
         const T x0 = (cc == 0) ? d0 : (T)0;
         const T x1 = (cc > 1) ? (T)0 : (cc == 1) ? d1 : -(m10 * x0) * d1;
         const T x2 = (cc > 2) ? (T)0 : (cc == 2) ? d2 : -fma_(m21, x1, m20 * x0) * d2;
@@ -191,10 +177,10 @@ __device__ __forceinline__ void lower_inverse(T (*Ls)[65], T (*Xs)[65], T *Ts, c
     }
     __syncthreads();
     // a level whose joined blocks start at or beyond nb only builds padding
-    if (nb > 4) inv_join_valu<T, 4, TRANS>(Ls, Xs, Ts, tid);
-    if (nb > 8) inv_join_valu<T, 8, TRANS>(Ls, Xs, Ts, tid);
-    if (nb > 16) inv_join_mfma<T, 16, TRANS>(Ls, Xs, Ts, tid & 63, w);
-    if (nb > 32) inv_join_mfma<T, 32, TRANS>(Ls, Xs, Ts, tid & 63, w);
+    if (nb > 4) inv_join_valu<T, 4>(Xs, Ts, tid);
+    if (nb > 8) inv_join_valu<T, 8>(Xs, Ts, tid);
+    if (nb > 16) inv_join_mfma<T, 16>(Xs, Ts, tid & 63, w);
+    if (nb > 32) inv_join_mfma<T, 32>(Xs, Ts, tid & 63, w);
 }
 
 // Cholesky and inverse of one 64-column diagonal sub-block.
@@ -325,7 +311,7 @@ __device__ __forceinline__ void potrf64_block(const DevSymbol &S, const int c, i
     __syncthreads();
     if (tid < 64) dinv[tid] = recip(Ls[tid][tid]);
     __syncthreads();
-    lower_inverse<T, false, false, true>(Ls, Ls, Ts, dinv, nb, tid, w);
+    lower_inverse<T>(Ls, Ts, dinv, nb, tid, w);
     T *W = winv + S.cblk_winv[c] + k0 + (int64_t)k0 * K;
     T *WT = winvt + S.cblk_winv[c] + k0 + (int64_t)k0 * K;
     for (int e = tid; e < 64 * 64; e += 256) {
@@ -740,6 +726,122 @@ __global__ __launch_bounds__(256) void k_winv_merge(DevSymbol S, const WinvTile 
     }
 }
 
+// Entry (r, c) of a lower-triangular matrix of the LU pair packed in X: the
+// unit lower L (strictly below the diagonal), or with UT the transpose of U
+// (U on and above the diagonal).
+template <typename T, bool UT> __device__ __forceinline__ T &lu_at(T (*X)[65], int r, int c) {
+    return UT ? X[c][r] : X[r][c];
+}
+template <typename T, bool UT> __device__ __forceinline__ T lu_tri(T (*X)[65], int r, int c) {
+    const T v = lu_at<T, UT>(X, r, c);
+    return r > c ? v : r < c ? (T)0 : UT ? v : (T)1;
+}
+
+// One joining level for one of the two matrices (see lower_inverse):
+// PHASE 1: Ts = M21 X11, PHASE 2: X21 = -X22 Ts; output o of 32 B on the
+// vector units, 16x16 tile t on the matrix cores.
+template <typename T, bool UT, int B, int PHASE>
+__device__ __forceinline__ void lu_join_valu(T (*X)[65], T *Ts, int o) {
+    const int p = o / (B * B), rem = o % (B * B), r = rem / B, cc = rem % B, base = 2 * B * p;
+    T s = (T)0;
+#pragma unroll
+    for (int m = 0; m < B; m++) {
+        if (PHASE == 1) s = fma_(lu_at<T, UT>(X, base + B + r, base + m), lu_tri<T, UT>(X, base + m, base + cc), s);
+        else s = fma_(lu_tri<T, UT>(X, base + B + r, base + B + m), Ts[p * B * B + m * B + cc], s);
+    }
+    if (PHASE == 1) Ts[o] = s;
+    else lu_at<T, UT>(X, base + B + r, base + cc) = -s;
+}
+template <typename T, bool UT, int B, int PHASE>
+__device__ __forceinline__ void lu_join_mfma(T (*X)[65], T *Ts, int lane, int t) {
+    constexpr int TPP = (B / 16) * (B / 16);
+    const int i = lane & 15, kq = lane >> 4;
+    const int p = t / TPP, ti = (t % TPP) / (B / 16) * 16, tj = t % (B / 16) * 16, base = 2 * B * p;
+    typename Mfma<T>::v4 acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < B / 4; s++) {
+        const int k = 4 * s + kq;
+        if (PHASE == 1)
+            acc = Mfma<T>::mma(lu_at<T, UT>(X, base + B + ti + i, base + k), lu_tri<T, UT>(X, base + k, base + tj + i),
+                               acc);
+        else
+            acc = Mfma<T>::mma(lu_tri<T, UT>(X, base + B + ti + i, base + B + k), Ts[p * B * B + k * B + tj + i], acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int row = ti + Mfma<T>::drow(lane, r);
+        if (PHASE == 1) Ts[p * B * B + row * B + tj + i] = acc[r];
+        else lu_at<T, UT>(X, base + B + row, base + tj + i) = -acc[r];
+    }
+}
+
+// The 4x4 diagonal blocks of one of the two (lane: 4 columns of 16 blocks).
+template <typename T, bool UT> __device__ __forceinline__ void lu_inv4(T (*X)[65], const T *dinv, int lane) {
+    const int b0 = 4 * (lane >> 2), cc = lane & 3;
+    auto M = [&](int r, int c) -> T { return lu_at<T, UT>(X, b0 + r, b0 + c); };
+    const T m10 = M(1, 0), m20 = M(2, 0), m21 = M(2, 1), m30 = M(3, 0), m31 = M(3, 1), m32 = M(3, 2);
+    const T d0 = UT ? dinv[b0] : (T)1, d1 = UT ? dinv[b0 + 1] : (T)1;
+    const T d2 = UT ? dinv[b0 + 2] : (T)1, d3 = UT ? dinv[b0 + 3] : (T)1;
+    const T x0 = (cc == 0) ? d0 : (T)0;
+    const T x1 = (cc > 1) ? (T)0 : (cc == 1) ? d1 : -(m10 * x0) * d1;
+    const T x2 = (cc > 2) ? (T)0 : (cc == 2) ? d2 : -fma_(m21, x1, m20 * x0) * d2;
+    const T x3 = (cc == 3) ? d3 : -fma_(m32, x2, fma_(m31, x1, m30 * x0)) * d3;
+    const int first = UT ? cc : cc + 1;  // L's unit diagonal is implied
+    if (first <= 0) lu_at<T, UT>(X, b0, b0 + cc) = x0;
+    if (first <= 1) lu_at<T, UT>(X, b0 + 1, b0 + cc) = x1;
+    if (first <= 2) lu_at<T, UT>(X, b0 + 2, b0 + cc) = x2;
+    if (first <= 3) lu_at<T, UT>(X, b0 + 3, b0 + cc) = x3;
+}
+
+// inv(L) and inv(U)^T of the LU pair packed in X, in place, by the steps of
+// lower_inverse: the two go side by side, so that together they take the
+// barriers of one (the unit diagonal of L and the zeros beyond the triangles
+// are implied).  Ts: 2048 entries of scratch.
+template <typename T>
+__device__ __forceinline__ void lu_inverse(T (*X)[65], T *Ts, const T *dinv, int nb, int tid, int w) {
+    T *const TL = Ts, *const TU = Ts + 1024;
+    const int lane = tid & 63;
+    if (w == 0) lu_inv4<T, false>(X, dinv, lane);
+    else if (w == 1) lu_inv4<T, true>(X, dinv, lane);
+    __syncthreads();
+#define LU_JOIN(PHASE)                                                        \
+    if (w < 2) lu_join_valu<T, false, 4, PHASE>(X, TL, tid);                  \
+    else lu_join_valu<T, true, 4, PHASE>(X, TU, tid - 128);                   \
+    __syncthreads();
+    if (nb > 4) {
+        LU_JOIN(1)
+        LU_JOIN(2)
+    }
+#undef LU_JOIN
+#define LU_JOIN(PHASE)                                \
+    lu_join_valu<T, false, 8, PHASE>(X, TL, tid);     \
+    lu_join_valu<T, true, 8, PHASE>(X, TU, tid);      \
+    __syncthreads();
+    if (nb > 8) {
+        LU_JOIN(1)
+        LU_JOIN(2)
+    }
+#undef LU_JOIN
+#define LU_JOIN(PHASE)                                               \
+    if (w < 2) lu_join_mfma<T, false, 16, PHASE>(X, TL, lane, w);    \
+    else lu_join_mfma<T, true, 16, PHASE>(X, TU, lane, w - 2);       \
+    __syncthreads();
+    if (nb > 16) {
+        LU_JOIN(1)
+        LU_JOIN(2)
+    }
+#undef LU_JOIN
+#define LU_JOIN(PHASE)                                   \
+    lu_join_mfma<T, false, 32, PHASE>(X, TL, lane, w);   \
+    lu_join_mfma<T, true, 32, PHASE>(X, TU, lane, w);    \
+    __syncthreads();
+    if (nb > 32) {
+        LU_JOIN(1)
+        LU_JOIN(2)
+    }
+#undef LU_JOIN
+}
+
 // LU without pivoting of one 64-column diagonal sub-block (reference
 // kernels/core_zgetrfsp.c:63-106, getf2 with static pivoting +-thr).  During
 // the factorisation the square part of a cblk keeps its lower triangle
@@ -750,20 +852,24 @@ __global__ __launch_bounds__(256) void k_winv_merge(DevSymbol S, const WinvTile 
 // in the L panel, the strict upper part of U transposed in the U panel,
 // W1 = inv(L) (lower, unit diagonal), W2 = inv(U)^T (lower) and WB = inv(U)
 // (upper), with explicit zeros in the other triangles of the sub-block; the
-// inverses come from lower_inverse (recursive doubling, in place in LDS: U^T
-// first, then L rebuilt from the registers).
+// inverses come from lu_inverse.
+//
+// Bound by the latency of its 16 steps and the joins.  With the rows of U
+// published through LDS and read back per column, the two inverses one after
+// the other and the U panel's triangle walked across columns, 16 blocks took
+// 44.7 us in FP64 and 35.9 in FP32, 2048 blocks 173 and 95; now 31.5 and
+// 26.6, 136 and 79 (same roundings).
 template <typename T>
 __global__ __launch_bounds__(256) void k_getrf64(DevSymbol S, const int32_t *__restrict__ cblks, int kb,
                                                  T *__restrict__ lcoef, T *__restrict__ ucoef, T *__restrict__ w1,
                                                  T *__restrict__ w2, T *__restrict__ wb, double thr, int *stat) {
     __builtin_amdgcn_s_setprio(3);
-    __shared__ T fac[1024];
-    T(*colb)[4][64] = reinterpret_cast<T(*)[4][64]>(fac);
-    T(*rowb)[4][64] = reinterpret_cast<T(*)[4][64]>(fac + 512);
-    __shared__ T Ls[64][65];
+    __shared__ T fac[2048];
+    T(*colb)[4][64] = reinterpret_cast<T(*)[4][64]>(fac);  // [parity][w][row]
+    __shared__ T Ls[64][65];                               // L below the diagonal, U from it
     __shared__ T dinv[64];
-    T *Ts = fac;  // inverse scratch once the factor is done
-    const int tid = threadIdx.x, i = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, i = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = cblks[blockIdx.x];
     const int K = S.cblk_fcol[c + 1] - S.cblk_fcol[c];
     const int k0 = kb * 64;
@@ -771,123 +877,131 @@ __global__ __launch_bounds__(256) void k_getrf64(DevSymbol S, const int32_t *__r
     const int64_t ld = S.cblk_stride[c];
     T *PL = lcoef + S.cblk_coef[c] + k0 + (int64_t)k0 * ld;
     T *PU = ucoef + S.cblk_coef[c] + k0 + (int64_t)k0 * ld;
+    // both triangles walked down columns, into rows through LDS; the padding
+    // up to 64 is the identity
+    {
+        T vl[16], vu[16];
+        const int64_t row = min(i, nb - 1);
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const int64_t o = row + min(4 * u + w, nb - 1) * ld;
+            vl[u] = PL[o];
+            vu[u] = PU[o];
+        }
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const int j = 4 * u + w;
+            const bool pad = i >= nb || j >= nb;
+            if (i >= j) Ls[i][j] = !pad ? vl[u] : (i == j) ? (T)1 : (T)0;
+            if (i > j) Ls[j][i] = !pad ? vu[u] : (T)0;
+        }
+    }
+    __syncthreads();
     T a[16];
 #pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-        const int j = 4 * jj + w;
-        T v = (i == j) ? (T)1 : (T)0;
-        if (i < nb && j < nb) v = (j <= i) ? PL[i + (int64_t)j * ld] : PU[j + (int64_t)i * ld];
-        a[jj] = v;
-    }
+    for (int jj = 0; jj < 16; jj++) a[jj] = Ls[i][4 * jj + w];
     const T crit = (T)thr;
     int npiv = 0;
     auto piv = [&](T d, int col) -> T {
-        if (col < nb && pabs(d) < crit) {
-            d = (d < (T)0) ? -crit : crit;
-            npiv++;
-        }
-        return d;
+        const bool small = col < nb && pabs(d) < crit;
+        npiv += small;
+        return small ? ((d < (T)0) ? -crit : crit) : d;
     };
-    // blocks of 4 columns k..k+3: publish the block's 4 columns and 4 rows,
-    // eliminate the 4x4 diagonal block redundantly in every thread, then row
-    // i forms its 4 multipliers and column j its 4 rows of U from the
-    // published values, and the rank-4 update needs no second barrier
+    // Blocks of 4 columns k..k+3, as in potrf64_block: the columns are
+    // published through LDS, every thread eliminates the 4x4 diagonal block,
+    // and row i forms its 4 multipliers.  The block's rows of U in a column
+    // are held by lanes k..k+3 of the wave that owns the column: with the
+    // multipliers of those rows being the block's own L (0 in the rows above),
+    // one formula leaves U in them and the Schur complement below, reading
+    // each pivot row across lanes once it is done.  The four products are
+    // summed before they are subtracted: every entry is rounded once per
+    // block (four subtractions in turn doubled the factor's error).  The next
+    // block's columns go first, the others overlap its 4x4 chain.
+    T p0 = 0, p1 = 0, p2 = 0, p3 = 0;  // this row's multipliers of the last block
+    auto rank4 = [&](T x, int k) -> T {
+        T s = p0 * rlane(x, k);
+        s = fma_(p1, rlane(x - s, k + 1), s);
+        s = fma_(p2, rlane(x - s, k + 2), s);
+        s = fma_(p3, rlane(x - s, k + 3), s);
+        return x - s;
+    };
+    colb[0][w][i] = a[0];
 #pragma unroll
     for (int b4 = 0; b4 < 16; b4++) {
         const int k = 4 * b4;
         if (k >= nb) break;  // uniform: the padding needs no elimination
-        T(*cb)[64] = colb[b4 & 1];
-        T(*rb)[64] = rowb[b4 & 1];
-        cb[w][i] = a[b4];
-        if (i >= k && i < k + 4) {
-#pragma unroll
-            for (int jj = b4 + 1; jj < 16; jj++) rb[i - k][4 * jj + w] = a[jj];
-        }
         __syncthreads();
+        int ii = i;  // opaque: see potrf64_block
+        asm volatile("" : "+v"(ii));
+        T(*cb)[64] = colb[b4 & 1];
         // D(t, u) = cb[u][k + t]
-        const T u00 = piv(cb[0][k], k), r0 = recip(u00);
-        const T l10 = cb[0][k + 1] * r0, l20 = cb[0][k + 2] * r0, l30 = cb[0][k + 3] * r0;
-        const T u01 = cb[1][k], u02 = cb[2][k], u03 = cb[3][k];
-        const T u11 = piv(cb[1][k + 1] - l10 * u01, k + 1), r1 = recip(u11);
-        const T u12 = cb[2][k + 1] - l10 * u02, u13 = cb[3][k + 1] - l10 * u03;
-        const T l21 = (cb[1][k + 2] - l20 * u01) * r1, l31 = (cb[1][k + 3] - l30 * u01) * r1;
-        const T u22 = piv(cb[2][k + 2] - l20 * u02 - l21 * u12, k + 2), r2 = recip(u22);
-        const T u23 = cb[3][k + 2] - l20 * u03 - l21 * u13;
-        const T l32 = (cb[2][k + 3] - l30 * u02 - l31 * u12) * r2;
-        const T u33 = piv(cb[3][k + 3] - l30 * u03 - l31 * u13 - l32 * u23, k + 3), r3 = recip(u33);
-        if (i > k + 3) {
-            const T m0 = cb[0][i] * r0;
-            const T m1 = (cb[1][i] - m0 * u01) * r1;
-            const T m2 = (cb[2][i] - m0 * u02 - m1 * u12) * r2;
-            const T m3 = (cb[3][i] - m0 * u03 - m1 * u13 - m2 * u23) * r3;
-            a[b4] = (w == 0) ? m0 : (w == 1) ? m1 : (w == 2) ? m2 : m3;
+        const T d00 = cb[0][k], d10 = cb[0][k + 1], d20 = cb[0][k + 2], d30 = cb[0][k + 3];
+        const T u01 = cb[1][k], d11 = cb[1][k + 1], d21 = cb[1][k + 2], d31 = cb[1][k + 3];
+        const T u02 = cb[2][k], d12 = cb[2][k + 1], d22 = cb[2][k + 2], d32 = cb[2][k + 3];
+        const T u03 = cb[3][k], d13 = cb[3][k + 1], d23 = cb[3][k + 2], d33 = cb[3][k + 3];
+        const T e0 = cb[0][ii], e1 = cb[1][ii], e2 = cb[2][ii], e3 = cb[3][ii];
+        if (b4 >= 1) {
 #pragma unroll
-            for (int jj = b4 + 1; jj < 16; jj++) {
-                const int j = 4 * jj + w;
-                const T v0 = rb[0][j];
-                const T v1 = rb[1][j] - l10 * v0;
-                const T v2 = rb[2][j] - l20 * v0 - l21 * v1;
-                const T v3 = rb[3][j] - l30 * v0 - l31 * v1 - l32 * v2;
-                a[jj] -= m0 * v0 + m1 * v1 + m2 * v2 + m3 * v3;
-            }
-        } else if (i >= k) {
-            const int t = i - k;
-            // row t of the block: L strictly left of the diagonal, U from it
-            T e;
-            if (w == 0) e = (t == 0) ? u00 : (t == 1) ? l10 : (t == 2) ? l20 : l30;
-            else if (w == 1) e = (t == 0) ? u01 : (t == 1) ? u11 : (t == 2) ? l21 : l31;
-            else if (w == 2) e = (t == 0) ? u02 : (t == 1) ? u12 : (t == 2) ? u22 : l32;
-            else e = (t == 0) ? u03 : (t == 1) ? u13 : (t == 2) ? u23 : u33;
-            a[b4] = e;
-#pragma unroll
-            for (int jj = b4 + 1; jj < 16; jj++) {
-                const int j = 4 * jj + w;
-                const T v0 = rb[0][j];
-                const T v1 = rb[1][j] - l10 * v0;
-                const T v2 = rb[2][j] - l20 * v0 - l21 * v1;
-                const T v3 = rb[3][j] - l30 * v0 - l31 * v1 - l32 * v2;
-                a[jj] = (t == 0) ? v0 : (t == 1) ? v1 : (t == 2) ? v2 : v3;
-            }
+            for (int jj = b4 + 1; jj < 16; jj++) a[jj] = rank4(a[jj], k - 4);
+        }
+        const T u00 = piv(d00, k), r0 = recip(u00);
+        const T l10 = d10 * r0, l20 = d20 * r0, l30 = d30 * r0;
+        const T u11 = piv(d11 - l10 * u01, k + 1), r1 = recip(u11);
+        const T u12 = d12 - l10 * u02, u13 = d13 - l10 * u03;
+        const T l21 = (d21 - l20 * u01) * r1, l31 = (d31 - l30 * u01) * r1;
+        const T u22 = piv(d22 - l20 * u02 - l21 * u12, k + 2), r2 = recip(u22);
+        const T u23 = d23 - l20 * u03 - l21 * u13;
+        const T l32 = (d32 - l30 * u02 - l31 * u12) * r2;
+        const T u33 = piv(d33 - l30 * u03 - l31 * u13 - l32 * u23, k + 3), r3 = recip(u33);
+        asm volatile("" : "+v"(npiv));
+        const T m0 = e0 * r0;
+        const T m1 = (e1 - m0 * u01) * r1;
+        const T m2 = (e2 - m0 * u02 - m1 * u12) * r2;
+        const T m3 = (e3 - m0 * u03 - m1 * u13 - m2 * u23) * r3;
+        const int t = ii - k;
+        const bool below = t > 3;
+        p0 = below ? m0 : (t == 1) ? l10 : (t == 2) ? l20 : (t == 3) ? l30 : (T)0;
+        p1 = below ? m1 : (t == 2) ? l21 : (t == 3) ? l31 : (T)0;
+        p2 = below ? m2 : (t == 3) ? l32 : (T)0;
+        p3 = below ? m3 : (T)0;
+        // the block's own columns: L strictly left of the diagonal, U from it
+        T f;
+        if (w == 0) f = (t == 0) ? u00 : p0;
+        else if (w == 1) f = (t == 0) ? u01 : (t == 1) ? u11 : p1;
+        else if (w == 2) f = (t == 0) ? u02 : (t == 1) ? u12 : (t == 2) ? u22 : p2;
+        else f = (t == 0) ? u03 : (t == 1) ? u13 : (t == 2) ? u23 : (t == 3) ? u33 : p3;
+        if (t >= 0) a[b4] = f;
+        if (b4 < 15) {
+            a[b4 + 1] = rank4(a[b4 + 1], k);
+            colb[(b4 + 1) & 1][w][ii] = a[b4 + 1];
         }
     }
-    // U^T (lower, diagonal of U) in LDS for the first in-place inverse
 #pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-        const int j = 4 * jj + w;
-        Ls[j][i] = (j >= i) ? a[jj] : (T)0;
-        if (i < nb && j < nb) {
-            if (j <= i) PL[i + (int64_t)j * ld] = a[jj];
-            else PU[j + (int64_t)i * ld] = a[jj];
-        }
-    }
+    for (int jj = 0; jj < 16; jj++) Ls[i][4 * jj + w] = a[jj];
     if (tid == 0 && npiv) atomicAdd(&stat[0], npiv);
     __syncthreads();
-    if (tid < 64) dinv[tid] = recip(Ls[tid][tid]);
+    if (w == 0) dinv[i] = recip(Ls[i][i]);
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int j = 4 * u + w;
+        if (i < nb && j < nb) {
+            if (i >= j) PL[i + j * ld] = Ls[i][j];
+            if (i > j) PU[i + j * ld] = Ls[j][i];
+        }
+    }
     __syncthreads();
+    lu_inverse<T>(Ls, fac, dinv, nb, tid, w);
     T *W1 = w1 + S.cblk_winv[c] + k0 + (int64_t)k0 * K;
     T *W2 = w2 + S.cblk_winv[c] + k0 + (int64_t)k0 * K;
     T *WB = wb + S.cblk_winv[c] + k0 + (int64_t)k0 * K;
-    const int wu = __builtin_amdgcn_readfirstlane(w);
-    lower_inverse<T, false, false, true>(Ls, Ls, Ts, dinv, nb, tid, wu);  // inv(U^T)
-    for (int e = tid; e < 64 * 64; e += 256) {
-        const int lo = e & 63, hi = e >> 6;
-        if (lo < nb && hi < nb) {
-            W2[lo + (int64_t)hi * K] = Ls[lo][hi];
-            WB[lo + (int64_t)hi * K] = Ls[hi][lo];
+#pragma unroll 4
+    for (int u = 0; u < 16; u++) {
+        const int j = 4 * u + w;
+        if (i < nb && j < nb) {
+            W1[i + (int64_t)j * K] = lu_tri<T, false>(Ls, i, j);
+            W2[i + (int64_t)j * K] = lu_tri<T, true>(Ls, i, j);
+            WB[i + (int64_t)j * K] = lu_tri<T, true>(Ls, j, i);
         }
-    }
-    __syncthreads();
-    // then the unit lower L (its diagonal is not read)
-#pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-        const int j = 4 * jj + w;
-        Ls[i][j] = (j < i) ? a[jj] : (T)0;
-    }
-    __syncthreads();
-    lower_inverse<T, true, false, true>(Ls, Ls, Ts, dinv, nb, tid, wu);  // inv(L)
-    for (int e = tid; e < 64 * 64; e += 256) {
-        const int lo = e & 63, hi = e >> 6;
-        if (lo < nb && hi < nb) W1[lo + (int64_t)hi * K] = Ls[lo][hi];
     }
 }
 
