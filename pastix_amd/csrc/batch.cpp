@@ -9,6 +9,9 @@
 // the user numbering, and the same range in the permuted numbering since the
 // union ordering is the concatenation of the systems' orderings.
 #include "pastix_data.h"
+#include <algorithm>
+#include <atomic>
+#include <thread>
 
 using namespace pxa_api;
 
@@ -111,6 +114,46 @@ int publish_union(pastix_data_t *d, int mtx, int64_t N, const std::vector<int64_
     S.rowptr = d->u_rows.data();
     S.values = d->u_vals.data();
     return PASTIX_SUCCESS;
+}
+
+// The systems' values into the published union, when every system is a CSC
+// with exactly the union's index arrays in its range (so that the union
+// build_union would give differs by the values only).  False: some system
+// isn't, and nothing is written.
+bool refill_union(pastix_data_t *d, const spmatrix_t *const *spms) {
+    const std::vector<int64_t> &off = d->batch_off;
+    const int64_t nsys = (int64_t)off.size() - 1;
+    if (d->u_colptr.size() != (size_t)off.back() + 1 || d->u_vals.size() != d->u_rows.size()) return false;
+    for (int64_t s = 0; s < nsys; s++) {
+        const spmatrix_t *A = spms[s];
+        if (!A || A->fmttype != SpmCSC || A->mtxtype != d->u_spm.mtxtype || A->dof != 1 || !A->values ||
+            A->n != off[s + 1] - off[s] || (A->flttype != SpmDouble && A->flttype != SpmFloat))
+            return false;
+    }
+    std::atomic<bool> same{true};
+    std::atomic<int64_t> compared{0};
+    pxa_api::parallel_tasks(2 * nsys, 3 * (int64_t)d->u_rows.size(), [&](int64_t t) {
+        const int64_t s = t % nsys;
+        const spmatrix_t *A = spms[s];
+        const spm_int_t *c = A->colptr, *r = A->rowptr, *uc = d->u_colptr.data() + off[s];
+        const int64_t base = c[0], n = A->n, k0 = uc[0], e = uc[n] - k0, dr = off[s] - base;
+        if (t < nsys) {
+            bool ok = true;
+            for (int64_t j = 0; j <= n; j++) ok &= c[j] - base == uc[j] - k0;
+            const spm_int_t *ur = d->u_rows.data() + k0;
+            if (ok)
+                for (int64_t k = 0; k < e; k++) ok &= r[k] + dr == ur[k];
+            if (!ok) same = false;
+            compared++;
+            return;
+        }
+        while (compared < nsys) std::this_thread::yield();
+        double *v = d->u_vals.data() + k0;
+        if (!same) return;
+        if (A->flttype == SpmDouble) memcpy(v, A->values, e * sizeof(double));
+        else std::copy((const float *)A->values, (const float *)A->values + e, v);
+    });
+    return same;
 }
 
 // Ordering of one system: the caller's, or nested dissection of its graph.
@@ -319,6 +362,7 @@ extern "C" int pastix_amd_batch_analyze(pastix_data_t *d, pastix_int_t nsys, con
 
 extern "C" int pastix_amd_batch_numfact(pastix_data_t *d, const spmatrix_t *const *spms) {
     if (!d || !spms || d->batch_off.size() < 2) return PASTIX_ERR_BADPARAMETER;
+    if (refill_union(d, spms)) return pastix_task_numfact(d, &d->u_spm);
     const pastix_int_t nsys = (pastix_int_t)d->batch_off.size() - 1;
     const size_t nnz = d->u_rows.size();
     std::vector<int64_t> off;

@@ -335,6 +335,10 @@ double *Engine::host_block(int64_t count) {
     return h_pin_;
 }
 
+void *Engine::small_block(size_t bytes) {
+    return bytes <= SMALL_COPY ? host_block((int64_t)(SMALL_COPY / sizeof(double))) : nullptr;
+}
+
 int Engine::download_diag(double *h) {
     if (!d_diagout_) {
         d_diagout_ = (double *)alloc(n_ * sizeof(double));
@@ -872,30 +876,36 @@ int Engine::solve_host(const int64_t *perm, int flttype, void *b, int64_t ldb, i
         }
     }
     // permute on the host into the factor precision: xp[perm[i]] = b[i]
-    std::vector<char> tmp((size_t)n_ * nrhs * fsz);
+    const size_t bytes = (size_t)n_ * nrhs * fsz;
+    std::vector<char> big;
+    void *tmp = small_block(bytes);
+    if (!tmp) {
+        big.resize(bytes);
+        tmp = big.data();
+    }
     for (int r = 0; r < nrhs; r++) {
         for (int64_t i = 0; i < n_; i++) {
             const int64_t p = perm[i] + (int64_t)r * n_;
             if (flttype == 3) {
                 double v = ((const double *)b)[i + r * ldb];
-                if (prec_ == 2) ((float *)tmp.data())[p] = (float)v;
-                else ((double *)tmp.data())[p] = v;
+                if (prec_ == 2) ((float *)tmp)[p] = (float)v;
+                else ((double *)tmp)[p] = v;
             } else {
                 float v = ((const float *)b)[i + r * ldb];
-                if (prec_ == 2) ((float *)tmp.data())[p] = v;
-                else ((double *)tmp.data())[p] = v;
+                if (prec_ == 2) ((float *)tmp)[p] = v;
+                else ((double *)tmp)[p] = v;
             }
         }
     }
-    HIPCHK(hipMemcpyAsync(d_rhs_, tmp.data(), tmp.size(), hipMemcpyHostToDevice, stream_));
+    HIPCHK(hipMemcpyAsync(d_rhs_, tmp, bytes, hipMemcpyHostToDevice, stream_));
     int rc = solve_device(d_rhs_, n_, nrhs, seconds);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(tmp.data(), d_rhs_, tmp.size(), hipMemcpyDeviceToHost, stream_));
+    HIPCHK(hipMemcpyAsync(tmp, d_rhs_, bytes, hipMemcpyDeviceToHost, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
     for (int r = 0; r < nrhs; r++) {
         for (int64_t i = 0; i < n_; i++) {
             const int64_t p = perm[i] + (int64_t)r * n_;
-            double v = (prec_ == 2) ? (double)((float *)tmp.data())[p] : ((double *)tmp.data())[p];
+            double v = (prec_ == 2) ? (double)((float *)tmp)[p] : ((double *)tmp)[p];
             if (flttype == 3) ((double *)b)[i + r * ldb] = v;
             else ((float *)b)[i + r * ldb] = (float)v;
         }
@@ -930,22 +940,19 @@ int Engine::upload_matrix(const HostBcsc &bc) {
                 if (bc.cols[k] == i) cd[i] = k;
         diag_complete_ = std::find(cd.begin(), cd.end(), (int64_t)-1) == cd.end();
         d_csrdiag_ = upload(*this, cd);
-        csrdiag_ = cd;
         d_diag0_ = (double *)alloc(n_ * sizeof(double));
         if (!d_csrdiag_ || !d_diag0_) return -1;
         have_matrix_ = true;
     }
     // the cached diagonal positions hold only for the uploaded pattern
     if ((int64_t)bc.tvals.size() != csr_nnz_) return fail("matrix pattern changed without drop_matrix");
-    {
-        std::vector<double> dg(n_, 0.0);
-        diag_sum_ = 0;
-        for (int64_t i = 0; i < n_; i++)
-            if (csrdiag_[i] >= 0) dg[i] = bc.tvals[csrdiag_[i]];
-        for (int64_t i = 0; i < n_; i++) diag_sum_ += dg[i];
-        HIPCHK(hipMemcpy(d_diag0_, dg.data(), n_ * sizeof(double), hipMemcpyHostToDevice));
-    }
-    HIPCHK(hipMemcpyAsync(d_vals_, bc.tvals.data(), bc.tvals.size() * sizeof(double), hipMemcpyHostToDevice, stream_));
+    diag_sum_ = bc.diag_sum;
+    const void *h = bc.tvals.data();
+    const size_t bytes = bc.tvals.size() * sizeof(double);
+    if (void *pin = small_block(bytes)) h = memcpy(pin, h, bytes);
+    HIPCHK(hipMemcpyAsync(d_vals_, h, bytes, hipMemcpyHostToDevice, stream_));
+    launch_get_csr_diag(n_, d_csrdiag_, d_vals_, d_diag0_, stream_);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(stream_));
     return 0;
 }

@@ -41,6 +41,10 @@ class Engine {
     // Pinned host staging block of at least count doubles, kept and grown
     // between calls (freed with the engine); nullptr when hipHostMalloc fails.
     double *host_block(int64_t count);
+    // The same block for a copy of at most SMALL_COPY bytes, else (or without
+    // pinned memory) nullptr: the copy goes from the caller's memory.
+    void *small_block(size_t bytes);
+    static constexpr size_t SMALL_COPY = 1 << 20;
     // Numerical factorisation over all levels; seconds = device time.
     int factorize(double thr, int64_t *npiv, int *negdiag, double *seconds);
     // Solve in place on a device block (factor precision, permuted order).
@@ -310,7 +314,6 @@ class Engine {
     // diagonal positions: in the coefficient table (per permuted column) and
     // in the CSR values, with the original FP64 diagonal
     int64_t *d_diagpos_ = nullptr, *d_csrdiag_ = nullptr;
-    std::vector<int64_t> csrdiag_;  // host copy of the CSR diagonal positions (-1: absent)
     double *d_diag0_ = nullptr;
     double diag_sum_ = 0;
     bool diag_complete_ = false;
@@ -347,7 +350,9 @@ struct HostBcsc {
     std::vector<int64_t> rowptr;
     std::vector<int32_t> cols;
     std::vector<double> tvals;
-    double normF = 0, normInf = 0;
+    double normF = 0, normInf = 0, diag_sum = 0;
+    // row ranges the sums are taken over, and the batch they were cut for
+    std::vector<int64_t> chunks, chunk_batch;
     // A later input with the same pattern is refilled by one gather: the
     // input's format, type, size and index arrays as given, and per CSR
     // entry e the input value indices src[sptr[e] .. sptr[e+1]) summed into

@@ -132,6 +132,7 @@ void launch_seg_xpby(int64_t n, int R, int64_t ld, const int32_t *seg, int nseg,
 // vals[pos[i]] = d0[i] + delta where pos[i] >= 0 (diagonal of the CSR).
 template <typename T>
 void launch_add_diag(int64_t n, const int64_t *pos, double delta, T *coef, hipStream_t st);
+void launch_get_csr_diag(int64_t n, const int64_t *pos, const double *vals, double *d0, hipStream_t st);
 void launch_set_csr_diag(int64_t n, const int64_t *pos, const double *d0, double delta, double *vals, hipStream_t st);
 // Zeroes n ints with a kernel (usable inside a captured graph).
 // out[i] = coef[pos[i]] for i < n (the factor's diagonal, as FP64)

@@ -469,6 +469,16 @@ void launch_set_csr_diag(int64_t n, const int64_t *pos, const double *d0, double
     if (n > 0) hipLaunchKernelGGL(k_set_csr_diag, dim3(nblk(n)), dim3(256), 0, st, n, pos, d0, delta, vals);
 }
 
+// d0[i] = vals[pos[i]], 0 where the diagonal entry is absent (pos < 0)
+__global__ __launch_bounds__(256) void k_get_csr_diag(int64_t n, const int64_t *__restrict__ pos,
+                                                      const double *__restrict__ vals, double *__restrict__ d0) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) d0[i] = pos[i] >= 0 ? vals[pos[i]] : 0.0;
+}
+void launch_get_csr_diag(int64_t n, const int64_t *pos, const double *vals, double *d0, hipStream_t st) {
+    if (n > 0) hipLaunchKernelGGL(k_get_csr_diag, dim3(nblk(n)), dim3(256), 0, st, n, pos, vals, d0);
+}
+
 // out[i] = coef[pos[i]] (the factor's diagonal, widened to FP64)
 template <typename T>
 __global__ __launch_bounds__(256) void k_gather_diag(int64_t n, const int64_t *__restrict__ pos,
