@@ -9,7 +9,8 @@
 //                     registers (computed transposed so that stores walk down
 //                     target columns) and subtracted straight into C;
 //   k_update_seq    : tiles fed by several sources: each entry's product as
-//                     in k_update_direct, subtracted into C in entry order.
+//                     in k_update_direct, subtracted into C in entry order
+//                     (FP64) or summed in LDS and subtracted once (FP32).
 // MODE 0 (LL^t and the L side of LU) keeps pairs with block(p) >= block(q),
 // MODE 1 (U side of LU) keeps block(p) > block(q), as the reference's
 // iterblok >= blok / iterblok > blok loops.
@@ -41,12 +42,11 @@ template <typename T> struct UpdLds {
     StageBuf<T, UPD_CH> sb;
     int rmap[64], cmap[64], rblk[64], qblk[64];
 };
-template <typename T, int MODE>
-__device__ __forceinline__ void update_entry(const DevSymbol &S, const UpdX &x, const int32_t *__restrict__ shift,
-                                             const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
-                                             T *__restrict__ Ccoef, UpdLds<T> &l, int tid) {
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+template <typename T>
+__device__ __forceinline__ void update_product(Quad<T> &q, const DevSymbol &S, const UpdX &x,
+                                               const int32_t *__restrict__ shift, const T *__restrict__ Acoef,
+                                               const T *__restrict__ Bcoef, UpdLds<T> &l, int tid) {
+    const int lane = tid & 63;
     int mrow = 0, mblk = 0;
     if (tid < 128) {
         const int64_t r = x.rb + (tid < 64 ? min(lane, x.np - 1) : x.dq + min(lane, x.nq - 1));
@@ -57,7 +57,6 @@ __device__ __forceinline__ void update_entry(const DevSymbol &S, const UpdX &x, 
     g.start(Bcoef + x.a + x.dq, x.nq, x.ld, Acoef + x.a, x.np, x.ld, x.K, tid);
     if (tid < 64) mrow += shift[x.sbi + mblk];
     else mrow -= x.fcol;
-    Quad<T> q;
     q.zero();
     g.run(q, l.sb, tid);
     if (tid < 64) {
@@ -68,6 +67,15 @@ __device__ __forceinline__ void update_entry(const DevSymbol &S, const UpdX &x, 
         l.qblk[lane] = mblk;
     }
     __syncthreads();
+}
+template <typename T, int MODE>
+__device__ __forceinline__ void update_entry(const DevSymbol &S, const UpdX &x, const int32_t *__restrict__ shift,
+                                             const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
+                                             T *__restrict__ Ccoef, UpdLds<T> &l, int tid) {
+    Quad<T> q;
+    update_product(q, S, x, shift, Acoef, Bcoef, l, tid);
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
     if (wr < x.nq && wc < x.np) {
         const int64_t stf = x.stf;
         T *C = Ccoef + x.c;
@@ -92,25 +100,81 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
     update_entry<T, MODE>(S, xs[id], shift, Acoef, Bcoef, Ccoef, lds, threadIdx.x);
 }
 
-// Tiles fed by several sources: the entries in order, each one's product
-// computed in registers as in k_update_direct and subtracted straight into
-// C (C -= p1, then C -= p2, ..., the reference's source order), with a
+// Tiles fed by several sources.  FP64: the entries in order, each one's
+// product computed in registers as in k_update_direct and subtracted straight
+// into C (C -= p1, then C -= p2, ..., the reference's source order), with a
 // barrier between entries so that the next entry's read-modify-write of an
-// element another wave wrote sees it.  The direct kernel's LDS footprint
-// (no 64x64 accumulator), so six waves per SIMD instead of three.
+// element another wave wrote sees it (an LDS tile's 52 KB would allow three
+// waves per SIMD instead of five: 56.0 against 54.3 ms on the 80^3 Laplacian).
+// FP32: the products are summed in an LDS tile that is subtracted at the end:
+// one rounding at C's magnitude instead of one per entry (in turn, the FP32
+// solution of the 80^3 Laplacian was off by 8.1e-7 instead of 6.1e-7).
+template <typename T> struct UpdSum {
+    static constexpr int LD = 68;  // sixteen rows of columns four apart: different banks
+    T t[64 * LD];
+    __device__ __forceinline__ void zero(int tid) {
+        for (int k = tid; k < 64 * LD; k += 256) t[k] = (T)0;
+    }
+    // the entry's product at (row, column) of the panel, the tile's corner at (r0, c0)
+    template <int MODE>
+    __device__ __forceinline__ void add(const Quad<T> &q, const UpdX &x, int r0, int c0, const UpdLds<T> &l, int tid) {
+        const int lane = tid & 63, wave = tid >> 6;
+        const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+        if (wr >= x.nq || wc >= x.np) return;
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int qj = wr + m * 16 + Mfma<T>::drow(lane, r), pi = wc + n * 16 + (lane & 15);
+                    if (qj < x.nq && pi < x.np && ((MODE == 0) ? (l.rblk[pi] >= l.qblk[qj]) : (l.rblk[pi] > l.qblk[qj])))
+                        t[(l.cmap[qj] - c0) * LD + l.rmap[pi] - r0] += q.c[m][n][r];
+                }
+    }
+    // the tile (at C, `rows` x `cols` of it in the panel) minus the sums
+    __device__ __forceinline__ void apply(T *C, int64_t stf, int64_t rows, int cols, int tid) const {
+        const int r = tid & 63, c0 = tid >> 6;
+        T v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+            v[u] = C[min((int64_t)r, rows - 1) + min(c0 + 4 * u, cols - 1) * stf];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const T w = t[(c0 + 4 * u) * LD + r];
+            if (r < rows && c0 + 4 * u < cols && w != (T)0) C[r + (c0 + 4 * u) * stf] = v[u] - w;
+        }
+    }
+};
+template <> struct UpdSum<double> {};
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_update_seq(
     DevSymbol S, const UpdItem *__restrict__ items, int nitems, const UpdX *__restrict__ xs,
     const int32_t *__restrict__ shift, const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
     T *__restrict__ Ccoef) {
     __shared__ UpdLds<T> lds;
+    __shared__ UpdSum<T> sum;
     const int id = xcd_remap(blockIdx.x, gridDim.x);
     if (id >= nitems) return;
-    const int e0 = items[id].e0, e1 = items[id].e1;
-    for (int e = e0; e < e1; e++) {
+    const UpdItem it = items[id];
+    const int tid = threadIdx.x;
+    if constexpr (sizeof(T) == 4) sum.zero(tid);
+    for (int e = it.e0; e < it.e1; e++) {
         // the previous entry's stores and map reads are done by every wave
-        if (e > e0) __syncthreads();
-        update_entry<T, MODE>(S, xs[e], shift, Acoef, Bcoef, Ccoef, lds, threadIdx.x);
+        if (e > it.e0) __syncthreads();
+        if constexpr (sizeof(T) == 4) {
+            Quad<T> q;
+            update_product(q, S, xs[e], shift, Acoef, Bcoef, lds, tid);
+            sum.template add<MODE>(q, xs[e], it.r0, it.c0, lds, tid);
+        } else {
+            update_entry<T, MODE>(S, xs[e], shift, Acoef, Bcoef, Ccoef, lds, tid);
+        }
+    }
+    if constexpr (sizeof(T) == 4) {
+        __syncthreads();
+        const int64_t stf = xs[it.e0].stf;
+        sum.apply(Ccoef + xs[it.e0].c + it.r0 + it.c0 * stf, stf, stf - it.r0,
+                  S.cblk_fcol[it.f + 1] - S.cblk_fcol[it.f] - it.c0, tid);
     }
 }
 
@@ -318,7 +382,8 @@ void launch_update_seq(const DevSymbol &S, int mode, const UpdItem *items, int n
                        const int32_t *shift, const T *A, const T *B, T *C, bool beside, hipStream_t st) {
     if (n <= 0) return;
     const dim3 g(grid8(n)), b(256);
-    const size_t lds = beside ? BESIDE_LDS - sizeof(UpdLds<T>) : 0;
+    const size_t own = sizeof(UpdLds<T>) + (sizeof(T) == 4 ? sizeof(UpdSum<T>) : 0);
+    const size_t lds = beside ? BESIDE_LDS - own : 0;
     if (mode == 0) hipLaunchKernelGGL((k_update_seq<T, 0>), g, b, lds, st, S, items, n, xs, shift, A, B, C);
     else hipLaunchKernelGGL((k_update_seq<T, 1>), g, b, lds, st, S, items, n, xs, shift, A, B, C);
 }
