@@ -34,10 +34,16 @@ struct DevSymbol {
     const int32_t *cblk_btile;    // 2 cblknbr: backward strips [tb, te) of every cblk
 };
 
+// tiles of a narrow level that receive entries in at most this many columns
+// are launched apart from the others
+constexpr int NARROW_COLS = 24;
+
 // One target tile of a Schur-complement update: rows [r0,r0+64) x columns
 // [c0,c0+64) of cblk f's panel, fed by entries [e0,e1).
 struct UpdItem {
-    int32_t f, r0, c0, e0, e1, pad0, pad1, pad2;
+    int32_t f, r0, c0, e0, e1;
+    uint32_t cm0, cm1;  // bit j: column c0 + j receives an entry (narrow levels)
+    int32_t pad;
 };
 
 // One source contribution to a tile: rows [p0,p1) and columns [q0,q1) are

@@ -127,6 +127,7 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     lv_cblk_ptr_ = P.lv_cblk_ptr;
     schurfcol_ = (P.schur_cblk < cblknbr_) ? s.cblk_fcol[P.schur_cblk] : n_;
     // widest factored cblk of each level
+    lv_narrow_ = P.lv_narrow;
     lv_maxw_.assign(P.nlevels, 0);
     for (int32_t lv = 0; lv < P.nlevels; lv++)
         for (int32_t k = P.lv_cblk_ptr[lv]; k < P.lv_cblk_ptr[lv] + P.lv_fact_cnt[lv]; k++) {
@@ -266,11 +267,35 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
         };
         upd_x_.assign(items.size() + 1, 0);
         lv_two_phase_.assign(P.nlevels, 0);
+        lv_few_.assign(2 * P.nlevels, 0);
         for (int32_t lv = 0; lv < P.nlevels; lv++) {
             // two-phase levels: their products fit the workspace
             lv_two_phase_[lv] = P.lv_upd_ptr[lv + 1] > P.lv_upd_split[lv] && !P.lv_single_pass[lv] &&
                                 P.lv_wsize[lv] <= wcap_;
             const int32_t end = lv_two_phase_[lv] ? P.lv_upd_split[lv] : P.lv_upd_ptr[lv + 1];
+            if (P.lv_narrow[lv]) {
+                // the tiles of few touched columns first, on either side of
+                // the next-level split
+                for (int32_t t = P.lv_upd_split[lv]; t < P.lv_upd_ptr[lv + 1]; t++) {
+                    UpdItem &it = items[t];
+                    uint64_t m = 0;
+                    for (int32_t e = it.e0; e < it.e1; e++) {
+                        const UpdEntry &en = P.ents[e];
+                        for (int32_t q = en.q0; q < en.q1; q++)
+                            m |= (uint64_t)1 << (P.panel_grow[P.rowbase[en.s] + q] - s.cblk_fcol[it.f] - it.c0);
+                    }
+                    it.cm0 = (uint32_t)m;
+                    it.cm1 = (uint32_t)(m >> 32);
+                }
+                auto few = [](const UpdItem &it) {
+                    return __builtin_popcount(it.cm0) + __builtin_popcount(it.cm1) <= NARROW_COLS;
+                };
+                const auto b = items.begin();
+                const int32_t r[3] = {P.lv_upd_split[lv], P.lv_upd_mnext[lv], P.lv_upd_ptr[lv + 1]};
+                for (int k = 0; k < 2; k++)
+                    lv_few_[2 * lv + k] =
+                        (int32_t)(std::stable_partition(b + r[k], b + r[k + 1], few) - (b + r[k]));
+            }
             for (int32_t t = P.lv_upd_ptr[lv]; t < end; t++) upd_x_[t] = take(items[t]);
         }
         std::vector<UpdItem> leaf_out = P.leaf_out;
@@ -509,6 +534,7 @@ template <typename T> int Engine::factorize_t(double thr) {
         const int u0 = lv_upd_ptr_[lv], us = lv_upd_split_[lv], u1 = lv_upd_ptr_[lv + 1];
         const int w0 = lv_wt_ptr_[lv], w1 = lv_wt_ptr_[lv + 1];
         const bool two_phase = lv_two_phase_[lv] != 0;
+        const bool narrow = lv_narrow_[lv] != 0;
         T *Wk = (T *)d_wspace_;
         // one side of an update range: direct tiles [da, db), multi-source
         // tiles [ma, mb) with their product tiles [wa, wb); (A, B) are the
@@ -533,7 +559,14 @@ template <typename T> int Engine::factorize_t(double thr) {
                 prof_end(KC_GATHER, k, st);
             } else {
                 k = prof_begin(st);
-                launch_update_seq<T>(S_, mode, d_upd_ + ma, mb - ma, d_updx_, d_shift_, A, B, C, st == side_, st);
+                if (narrow) {
+                    const int r[3] = {us, lv_upd_mnext_[lv], u1};
+                    for (int s = 0; s < 2; s++)
+                        if (ma <= r[s] && r[s + 1] <= mb)
+                            launch_update_narrow<T>(S_, mode, d_upd_ + r[s], r[s + 1] - r[s], lv_few_[2 * lv + s],
+                                                    d_updx_, d_shift_, A, B, C, st);
+                } else
+                    launch_update_seq<T>(S_, mode, d_upd_ + ma, mb - ma, d_updx_, d_shift_, A, B, C, st == side_, st);
                 prof_end(KC_ACC, k, st);
             }
         };

@@ -207,6 +207,10 @@ class Engine {
     std::vector<int> slv_maxw_, slv_maxcw_;
     int64_t schurfcol_ = 0;
     std::vector<int> lv_maxw_;  // widest factored cblk of each level
+    std::vector<uint8_t> lv_narrow_;  // levels of narrow sources
+    // their tiles of few columns: the first of those facing the next level,
+    // the first of the others
+    std::vector<int32_t> lv_few_;
     // LU: 64x64 tiles on and below the diagonal of the factored cblks'
     // squares, level L's at [lv_sq_ptr_[L], lv_sq_ptr_[L + 1])
     PanelItem *d_sq_ = nullptr;

@@ -4,16 +4,21 @@
 // One workgroup owns each 64x64 tile of a target cblk's panel and applies, in
 // source order, every contribution of the level's sources that lands in it:
 // C[f] -= A[s](p rows) * B[s](q rows)^T scattered through the row/column maps
-// (no atomics, bitwise-reproducible).  Operands are staged through LDS.
+// (no atomics, bitwise-reproducible).
 //   k_update_direct : tiles fed by a single source: the product is kept in
 //                     registers (computed transposed so that stores walk down
 //                     target columns) and subtracted straight into C;
 //   k_update_seq    : tiles fed by several sources: each entry's product as
 //                     in k_update_direct, subtracted into C in entry order
-//                     (FP64) or summed in LDS and subtracted once (FP32).
+//                     (FP64) or summed in LDS and subtracted once (FP32);
+//   k_update_narrow : the same on levels of narrow sources, a wave per entry;
+//   k_update_wgemm, k_update_gather : the products of a level's sources into a
+//                     workspace, then summed up tile by tile.
 // MODE 0 (LL^t and the L side of LU) keeps pairs with block(p) >= block(q),
 // MODE 1 (U side of LU) keeps block(p) > block(q), as the reference's
 // iterblok >= blok / iterblok > blok loops.
+#include <type_traits>
+
 #include "dev_common.h"
 #include "dev_types.h"
 #include "dev_update.h"
@@ -110,7 +115,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
 // one rounding at C's magnitude instead of one per entry (in turn, the FP32
 // solution of the 80^3 Laplacian was off by 8.1e-7 instead of 6.1e-7).
 template <typename T> struct UpdSum {
-    static constexpr int LD = 68;  // sixteen rows of columns four apart: different banks
+    // four groups of sixteen rows, columns four (FP32) or one (FP64) apart:
+    // every bank once (twice)
+    static constexpr int LD = sizeof(T) == 4 ? 68 : 72;
     T t[64 * LD];
     __device__ __forceinline__ void zero(int tid) {
         for (int k = tid; k < 64 * LD; k += 256) t[k] = (T)0;
@@ -146,14 +153,13 @@ template <typename T> struct UpdSum {
         }
     }
 };
-template <> struct UpdSum<double> {};
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_update_seq(
     DevSymbol S, const UpdItem *__restrict__ items, int nitems, const UpdX *__restrict__ xs,
     const int32_t *__restrict__ shift, const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
     T *__restrict__ Ccoef) {
     __shared__ UpdLds<T> lds;
-    __shared__ UpdSum<T> sum;
+    __shared__ std::conditional_t<sizeof(T) == 4, UpdSum<T>, char> sum;
     const int id = xcd_remap(blockIdx.x, gridDim.x);
     if (id >= nitems) return;
     const UpdItem it = items[id];
@@ -175,6 +181,150 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         const int64_t stf = xs[it.e0].stf;
         sum.apply(Ccoef + xs[it.e0].c + it.r0 + it.c0 * stf, stf, stf - it.r0,
                   S.cblk_fcol[it.f + 1] - S.cblk_fcol[it.f] - it.c0, tid);
+    }
+}
+
+// The same for levels whose sources have at most NARROW_UPD columns (the
+// bottom of the tree), FP32 and FP64.  An entry there is 7 rows by 3 columns
+// and 7 source columns (lowest level of a 2D Laplacian) or 13 x 8 and 8 (27
+// points on 48^3): one or two 16x16 pieces, too little for a workgroup.  Every
+// wave takes an entry, operands straight from memory, and when its turn comes
+// adds the product to the tile's sums in LDS; they are subtracted once at the
+// end.  Entry order and one subtraction, as with the product workspace
+// (k_update_wgemm, k_update_gather), bit for bit.
+//
+// Bound by latency: descriptor, maps and operands are three loads deep.  So as
+// many tiles as possible at a time: only the columns that receive something
+// (cm0, cm1) have sums, and the tiles of at most NARROW_COLS of them, nearly
+// all, go apart from the others with two waves each.  Lowest level of the
+// 701x653 Laplacian, FP64 (35,210 tiles, 135,188 entries): 784 us through the
+// workspace, 465 with 64 columns of sums and four waves for every tile, 181 so
+// (16 columns 180, 32 columns 232); its five narrow levels 1578 -> 514 us,
+// numfact 4.0 -> 3.1 ms.  Subtracting entry by entry without LDS took 485 us,
+// but rounds every entry at the target's magnitude.  Panels below 2 GiB
+// (32-bit lane offsets).
+template <typename T, int MODE, int NW, int NC>
+__global__ __launch_bounds__(64 * NW) void k_update_narrow(DevSymbol S, const UpdItem *__restrict__ items, int nitems,
+                                                       const UpdX *__restrict__ xs, const int32_t *__restrict__ shift,
+                                                       const T *__restrict__ Acoef, const T *__restrict__ Bcoef,
+                                                       T *__restrict__ Ccoef) {
+    // row r of the tile's s-th touched column at [s * LD + r]
+    constexpr int LD = UpdSum<T>::LD;
+    __shared__ T sum[NC * LD];
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    if (id >= nitems) return;
+    const UpdItem it = items[id];
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr uint32_t SZ = sizeof(T);
+    auto at = [](const T *base, uint32_t bytes) -> T {
+        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
+    };
+    typedef typename Mfma<T>::v4 v4;
+    const uint64_t mask = ((uint64_t)it.cm1 << 32) | it.cm0;
+    const int nc = __popcll(mask);
+    for (int o = tid; o < nc * LD; o += 64 * NW) sum[o] = (T)0;
+    for (int eb = it.e0; eb < it.e1; eb += NW) {
+        const int e = eb + wave, ne = min(NW, it.e1 - eb);
+        const UpdX x = xs[min(e, it.e1 - 1)];
+        // row and column maps: lane l holds source row p0 + l, column q0 + l
+        const int32_t *pblk = S.panel_blk + x.rb, *pgrow = S.panel_grow + x.rb;
+        const int rp = min(lane, x.np - 1), rq = x.dq + min(lane, x.nq - 1);
+        const int pb = pblk[rp], qb = pblk[rq];
+        int pr = pgrow[rp] - it.r0;
+        const int qc = __popcll(mask & (((uint64_t)1 << (pgrow[rq] - x.fcol - it.c0)) - 1)) * LD;
+        const T *A = Acoef + x.a, *B = Bcoef + x.a + x.dq;
+        // 16x16 pieces, columns q by rows p, p first; lane offsets of a
+        // step's four source columns and of the last step's
+        const int npt = (x.np + 15) >> 4, nt = e < it.e1 ? npt * ((x.nq + 15) >> 4) : 0;
+        const int ns = (x.K + 3) >> 2, kl = x.K - 4 * (ns - 1);
+        const uint32_t ldb = x.ld * SZ, kv = kq * ldb, kvl = min(kq, kl - 1) * ldb;
+        auto product = [&](int q0, int p0) -> v4 {
+            const uint32_t ao = min(p0 + i, x.np - 1) * SZ, bo = min(q0 + i, x.nq - 1) * SZ;
+            v4 acc = {0, 0, 0, 0};
+#pragma unroll 1
+            for (int s = 0; s < ns; s += 2) {
+                T a[2], b[2];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int su = min(s + u, ns - 1);
+                    const uint32_t ko = su == ns - 1 ? kvl : kv;
+                    const int64_t so = (int64_t)(4 * su) * x.ld;
+                    a[u] = at(A + so, ao + ko);
+                    b[u] = at(B + so, bo + ko);
+                }
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const bool in = 4 * (s + u) + kq < x.K;
+                    acc = Mfma<T>::mma(in ? b[u] : (T)0, in ? a[u] : (T)0, acc);
+                }
+            }
+            return acc;
+        };
+        auto add = [&](int q0, int p0, const v4 &acc) {
+            const int row = __shfl(pr, p0 + i), bp = __shfl(pb, p0 + i);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int j = q0 + Mfma<T>::drow(lane, r);
+                const int col = __shfl(qc, j), bq = __shfl(qb, j);
+                if (p0 + i < x.np && j < x.nq && (MODE == 0 ? bp >= bq : bp > bq)) sum[col + row] += acc[r];
+            }
+        };
+        constexpr int NT = 4;  // pieces kept in registers until the wave's turn
+        v4 acc[NT];
+        int q0 = 0, p0 = 0;
+        auto next = [&] {
+            p0 += 16;
+            if (p0 >= x.np) {
+                p0 = 0;
+                q0 += 16;
+            }
+        };
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            if (t < nt) {
+                acc[t] = product(q0, p0);
+                next();
+            }
+        pr += shift[x.sbi + pb];
+        for (int w = 0; w < ne; w++) {
+            __syncthreads();
+            if (w != wave) continue;
+            q0 = p0 = 0;
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                if (t < nt) {
+                    add(q0, p0, acc[t]);
+                    next();
+                }
+            for (int t = NT; t < nt; t++) {
+                add(q0, p0, product(q0, p0));
+                next();
+            }
+        }
+    }
+    __syncthreads();
+    const int64_t stf = xs[it.e0].stf;
+    T *C = Ccoef + xs[it.e0].c + it.r0 + lane + it.c0 * stf;
+    // the touched columns in turn, wave w every NW-th; zeros are not touched
+    uint64_t left = mask;
+    for (int w = 0; w < wave; w++) left &= left - 1;
+    for (int s = wave; s < nc; s += 4 * NW) {
+        T v[4], c[4];
+        T *cp[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int su = s + u * NW;
+            cp[u] = C + (left ? __builtin_ctzll(left) : 0) * stf;
+#pragma unroll
+            for (int w = 0; w < NW; w++) left &= left - 1;
+            v[u] = su < nc ? sum[min(su, NC - 1) * LD + lane] : (T)0;
+            c[u] = (T)0;
+            if (v[u] != (T)0) c[u] = *cp[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (v[u] != (T)0) *cp[u] = c[u] - v[u];
     }
 }
 
@@ -389,6 +539,24 @@ void launch_update_seq(const DevSymbol &S, int mode, const UpdItem *items, int n
 }
 
 template <typename T>
+void launch_update_narrow(const DevSymbol &S, int mode, const UpdItem *items, int n, int few, const UpdX *xs,
+                          const int32_t *shift, const T *A, const T *B, T *C, hipStream_t st) {
+    if (n <= 0) return;
+    auto run = [&](auto kernel, int waves, const UpdItem *it, int m) {
+        if (m > 0)
+            hipLaunchKernelGGL(kernel, dim3(grid8(m)), dim3(64 * waves), 0, st, S, it, m, xs, shift, A, B, C);
+    };
+    constexpr int W = NARROW_COLS;
+    if (mode == 0) {
+        run(k_update_narrow<T, 0, 2, W>, 2, items, few);
+        run(k_update_narrow<T, 0, 4, 64>, 4, items + few, n - few);
+    } else {
+        run(k_update_narrow<T, 1, 2, W>, 2, items, few);
+        run(k_update_narrow<T, 1, 4, 64>, 4, items + few, n - few);
+    }
+}
+
+template <typename T>
 void launch_update_wgemm(const DevSymbol &S, const WTile *items, int n, const T *A, const T *B, T *W, hipStream_t st) {
     if (n <= 0) return;
     hipLaunchKernelGGL((k_update_wgemm<T>), dim3(grid8(n)), dim3(256), 0, st, S, items, n, A, B, W);
@@ -408,6 +576,8 @@ void launch_update_gather(const DevSymbol &S, int mode, const UpdItem *items, in
                                           const T *, T *, bool, hipStream_t);                                     \
     template void launch_update_seq<T>(const DevSymbol &, int, const UpdItem *, int, const UpdX *,                \
                                        const int32_t *, const T *, const T *, T *, bool, hipStream_t);            \
+    template void launch_update_narrow<T>(const DevSymbol &, int, const UpdItem *, int, int, const UpdX *,        \
+                                          const int32_t *, const T *, const T *, T *, hipStream_t);               \
     template void launch_update_wgemm<T>(const DevSymbol &, const WTile *, int, const T *, const T *, T *,        \
                                          hipStream_t);                                                            \
     template void launch_update_gather<T>(const DevSymbol &, int, const UpdItem *, int, const UpdEntry *,         \

@@ -95,6 +95,9 @@ Plan build_plan(const Symbol &s, const Layout &L, int64_t schur_cblk, const Plan
     P.lv_wt_ptr.assign(nl + 1, 0);
     P.lv_wsize.assign(nl, 0);
     P.lv_single_pass.assign(nl, 0);
+    P.lv_narrow.assign(nl, 0);
+    int64_t panel_max = 0;
+    for (int64_t c = 0; c < s.cblknbr(); c++) panel_max = std::max(panel_max, L.cblk_stride[c] * width(c));
     P.lv_panel_right.assign(nl, 0);
     std::vector<KeyEnt> ke;
     std::vector<Range> rr, cr;
@@ -177,7 +180,8 @@ Plan build_plan(const Symbol &s, const Layout &L, int64_t schur_cblk, const Plan
             it.e0 = (int32_t)P.ents.size();
             for (size_t t = k; t < e; t++) P.ents.push_back(ke[t].e);
             it.e1 = (int32_t)P.ents.size();
-            it.pad0 = it.pad1 = it.pad2 = 0;
+            it.cm0 = it.cm1 = 0;
+            it.pad = 0;
             out.push_back(it);
             k = e;
         }
@@ -286,15 +290,20 @@ Plan build_plan(const Symbol &s, const Layout &L, int64_t schur_cblk, const Plan
             (int32_t)(std::stable_partition(P.upd.begin() + split, P.upd.end(), next_level) - P.upd.begin());
         // levels whose multi-source tiles hold about two entries on average
         // are updated in one pass: the product workspace would write and
-        // re-read every product for little reuse of the target tile
+        // re-read every product for little reuse of the target tile; so are
+        // those of narrow sources
         {
             int64_t nm = 0, nme = 0;
             for (int32_t t = split; t < P.lv_upd_ptr[lv + 1]; t++) {
                 nm++;
                 nme += P.upd[t].e1 - P.upd[t].e0;
             }
-            P.lv_single_pass[lv] = nm > 0 && (knobs.sp(lv) >= 0 ? knobs.sp(lv) != 0
-                                                                : (double)nme <= SINGLE_PASS_ENTS * (double)nm);
+            int64_t mw = 0;
+            for (int32_t k = l0; k < lf; k++) mw = std::max<int64_t>(mw, width(P.lv_cblks[k]));
+            P.lv_narrow[lv] = mw <= NARROW_UPD && panel_max < NARROW_PANEL;
+            P.lv_single_pass[lv] =
+                nm > 0 && (knobs.sp(lv) >= 0 ? knobs.sp(lv) != 0
+                                             : P.lv_narrow[lv] || (double)nme <= SINGLE_PASS_ENTS * (double)nm);
         }
         const bool single = P.lv_single_pass[lv] != 0;
         // exact flops of the kept (p, q) pairs of every entry

@@ -12,6 +12,13 @@ namespace pxa {
 // a level whose multi-source tiles average at most this many entries skips
 // the product workspace (the one-pass update kernel sums its entries)
 constexpr double SINGLE_PASS_ENTS = 2.05;
+// levels whose sources have at most this many columns skip it too
+// (k_update_narrow): 181 to 74 us on the five levels below that of a 701x653
+// Laplacian, the workspace 784 to 88; with up to 22 and 32 columns a wave per
+// tile took as long as the workspace (64 and 66, 62 and 62 us), with 50 longer
+constexpr int64_t NARROW_UPD = 16;
+// largest panel (entries) on which that kernel's 32-bit byte offsets hold
+constexpr int64_t NARROW_PANEL = (int64_t)1 << 28;
 // levels with fewer 64-row panel tiles than this update their panels
 // right-looking (64-deep products over all later blocks)
 constexpr int64_t PANEL_RIGHT_ROWTILES = 200;
@@ -64,8 +71,9 @@ struct Plan {
     std::vector<int32_t> lv_wt_next;  // [lv_wt_ptr[L], lv_wt_next[L]): groups facing level L+1
     std::vector<int64_t> lv_wsize;
     // levels whose multi-source tiles are summed in one pass (no product
-    // tiles, lv_wsize 0): those averaging at most SINGLE_PASS_ENTS entries
-    std::vector<uint8_t> lv_single_pass;
+    // tiles, lv_wsize 0): those averaging at most SINGLE_PASS_ENTS entries and
+    // the narrow ones (lv_narrow)
+    std::vector<uint8_t> lv_single_pass, lv_narrow;
     int64_t wmax = 0;
     // ---- solve ----
     // Solve nodes: runs of consecutive factored cblks solved as one diagonal
