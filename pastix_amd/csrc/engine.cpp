@@ -324,10 +324,14 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     if (P.winv_tmax > 0 && !(d_tbuf_ = alloc((size_t)P.winv_tmax * fsz))) return -1;
     d_WB_ = alloc(winvnbr_ * fsz);
     if (d_WB_) HIPCHK(hipMemsetAsync(d_WB_, 0, winvnbr_ * fsz, stream_));
-    // right-hand sides of one sweep: up to 32, the kernels taking them in
-    // groups of 2 or 8 on the grid (the factor is read once per sweep); the
-    // dependency-driven solve runs 8 at a time
-    nrhs_chunk_ = 32;
+    // right-hand sides of one sweep: up to 64 (32 where the sweep's vectors
+    // would take over 4 GiB), the kernels taking them in groups of 16 or 32 on
+    // the grid.  The sweep of 64 costs hardly more launches' time than that of
+    // 32 (24 levels of 6 launches, most of them a few us long): three FP32
+    // preconditioner solves of 64 columns (56x48x60) and their CG 7.95 ms in
+    // halves, 6.04 ms at once; 128 at a time 6.01.
+    const int64_t column = (int64_t)fsz * (bwd_part_ + nyrows_ + n_);
+    nrhs_chunk_ = column * 64 <= ((int64_t)4 << 30) ? 64 : 32;
     d_part_ = alloc((size_t)std::max<int64_t>(bwd_part_, 1) * nrhs_chunk_ * fsz);
     d_ybuf_ = alloc((size_t)std::max<int64_t>(nyrows_, 1) * nrhs_chunk_ * fsz);
     d_z_ = alloc((size_t)std::max<int64_t>(n_, 1) * nrhs_chunk_ * fsz);

@@ -296,7 +296,7 @@ class Engine {
     void *d_L_ = nullptr, *d_U_ = nullptr, *d_W1_ = nullptr, *d_W2_ = nullptr;
     int *d_stat_ = nullptr;
     void *d_part_ = nullptr;
-    int nrhs_chunk_ = 8;
+    int nrhs_chunk_ = 32;
     void *d_rhs_ = nullptr;  // n x nrhs_cap work block in factor precision
     int64_t rhs_cap_ = 0;
     double *d_red_ = nullptr;  // reduction partials + scalars
