@@ -399,6 +399,14 @@ int Engine::download_coef(void *hL, void *hU) {
     return 0;
 }
 
+// Far tiles below which a level's updates stay in the main stream: less than a
+// tile per CU, they are over before the second stream's two waits are.  Whole
+// calls with the line at 0 / 100 / 200 / 400 / 1600 tiles: 20^3 Laplacian 1.60
+// / 1.52 / 1.52 / 1.56 / 1.57 ms, LDL^t 31x29x34 4.68 / 4.54 / 4.56 / 4.59 /
+// 4.64, FP32 LU 37x41x33 6.68 / 6.55 / 6.44 / 6.57 / 6.71; larger ones as
+// before with any.
+constexpr int BESIDE_TILES = 256;
+
 // Level L: factor the diagonal blocks of its cblks, solve their panels, then
 // apply every update these cblks send to later levels.
 int Engine::prof_begin(hipStream_t st) {
@@ -429,7 +437,9 @@ template <typename T> int Engine::factorize_t(double thr) {
     // beside the panels of level L+1.  The main stream waits for them before
     // issuing level L+1's updates: targets and workspace regions of the two
     // streams are then disjoint at every moment, and every target tile still
-    // receives its contributions level by level, as with one stream.
+    // receives its contributions level by level, as with one stream.  A level
+    // of few far tiles keeps them in the main stream, one launch with the near
+    // ones.
     bool side_open = false;
     size_t lv_first = 0;
     cur_lv_ = 0;
@@ -582,12 +592,14 @@ template <typename T> int Engine::factorize_t(double thr) {
                 part(st, 0, L, L, L, da, db, ma, mb, wa, wb);
             }
         };
-        if (!overlap) {
+        const int dn = lv_upd_dnext_[lv], mn = lv_upd_mnext_[lv], wn = lv_wt_next_[lv];
+        if (const int rc = winv_upto(lv + 1)) return rc;
+        if (!overlap || (us - dn) + (u1 - mn) < BESIDE_TILES) {
+            if (side_open) HIPCHK(hipStreamWaitEvent(stream_, ev_side_, 0));
+            side_open = false;
             sides(stream_, u0, us, us, u1, w0, w1);
             continue;
         }
-        const int dn = lv_upd_dnext_[lv], mn = lv_upd_mnext_[lv], wn = lv_wt_next_[lv];
-        if (const int rc = winv_upto(lv + 1)) return rc;
         HIPCHK(hipEventRecord(ev_panel_, stream_));
         if (side_open) HIPCHK(hipStreamWaitEvent(stream_, ev_side_, 0));
         sides(stream_, u0, dn, us, mn, w0, wn);
