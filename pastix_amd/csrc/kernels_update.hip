@@ -40,9 +40,9 @@ constexpr int UPD_CH = 16;
 // the rest in the tiles' first and last memory round trips: 80^3 Laplacian,
 // FP64, one stream, k_update_direct 20.9 ms (47 TFLOP/s; 21.9 with the maps
 // before the product and the descriptors behind three loads), k_update_seq
-// 14.0 ms (47 TFLOP/s); FP32 on 61x57x66 2.75 and 1.87 ms (the sum in an LDS
-// tile, one write of C for all entries, took 2.07).  Fire-and-forget atomic
-// subtraction instead of the load was slower.
+// 14.0 ms (47 TFLOP/s); FP32 on 61x57x66 2.8 and 1.9 ms (k_update_seq summing
+// in LDS 2.1).  Fire-and-forget atomic subtraction instead of the load was
+// slower.
 template <typename T> struct UpdLds {
     StageBuf<T, UPD_CH> sb;
     int rmap[64], cmap[64], rblk[64], qblk[64];
