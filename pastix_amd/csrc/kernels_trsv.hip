@@ -741,11 +741,18 @@ __global__ __launch_bounds__(256) void k_fwd_prod_m(DevSymbol S, const FwdItem *
         for (int t = 0; t < NC / 2; t++) lds[(zu + 2 * t) * ZP + zk] = (zk < kn) ? v[t] : (T)0;
         __syncthreads();
         if (kc + KC < K) zload(kc + KC);
-        // four steps' factor loads together, then their MFMAs
+        // four steps' factor loads together, then their MFMAs, summed from
+        // zero: one chain over all columns rounded at the whole sum's size
+        // each time (residuals of 32 right-hand sides up to 13 % larger)
         for (int s0 = 4 * ks; s0 < kn; s0 += 16 * KS) {
             T m[4][E];
 #pragma unroll
             for (int j = 0; j < 4; j++) ld_vec(P + (int64_t)(kc + min(s0 + 4 * KS * j + kq, kn - 1)) * ld, m[j]);
+            typename Mfma<T>::v4 p[E][NB];
+#pragma unroll
+            for (int e = 0; e < E; e++)
+#pragma unroll
+                for (int b = 0; b < NB; b++) p[e][b] = {0, 0, 0, 0};
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int s = s0 + 4 * KS * j, k = s + kq;
@@ -756,9 +763,13 @@ __global__ __launch_bounds__(256) void k_fwd_prod_m(DevSymbol S, const FwdItem *
                 for (int b = 0; b < NB; b++) {
                     const T a = lds[(16 * b + i) * ZP + k];
 #pragma unroll
-                    for (int e = 0; e < E; e++) acc[e][b] = Mfma<T>::mma(a, m[j][e], acc[e][b]);
+                    for (int e = 0; e < E; e++) p[e][b] = Mfma<T>::mma(a, m[j][e], p[e][b]);
                 }
             }
+#pragma unroll
+            for (int e = 0; e < E; e++)
+#pragma unroll
+                for (int b = 0; b < NB; b++) acc[e][b] += p[e][b];
         }
     }
     __syncthreads();
@@ -841,6 +852,9 @@ __global__ __launch_bounds__(256) void k_bwd_prod_m(DevSymbol S, const BwdItem *
         __syncthreads();
         if (more) xload();
         if (live) {
+            typename Mfma<T>::v4 p[NB];  // see k_fwd_prod_m
+#pragma unroll
+            for (int b = 0; b < NB; b++) p[b] = {0, 0, 0, 0};
 #pragma unroll
             for (int g = 0; g < NG; g++) {
 #pragma unroll
@@ -849,9 +863,11 @@ __global__ __launch_bounds__(256) void k_bwd_prod_m(DevSymbol S, const BwdItem *
                 for (int b = 0; b < NB; b++) {
                     const T *a = &lds[(16 * b + i) * XP + RR * rs + 4 * E * g + E * kq];
 #pragma unroll
-                    for (int e = 0; e < E; e++) acc[b] = Mfma<T>::mma(a[e], m[g][e], acc[b]);
+                    for (int e = 0; e < E; e++) p[b] = Mfma<T>::mma(a[e], m[g][e], p[b]);
                 }
             }
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[b] += p[b];
         }
     }
     T *out = part + (int64_t)it.slot * nrhs + (int64_t)u0 * K;
@@ -1047,12 +1063,14 @@ __global__ __launch_bounds__(256) void k_diag_gemm16(DevSymbol S, const DiagItem
                 }
             }
         }
+        typename Mfma<T>::v4 p = {0, 0, 0, 0};  // see k_fwd_prod_m
 #pragma unroll
         for (int j = 0; j < U; j++) {
             if (kb0 + 4 * G * j >= k1) break;  // uniform
 #pragma unroll
-            for (int e = 0; e < E; e++) acc = Mfma<T>::mma(a[j][e], m[j][e], acc);
+            for (int e = 0; e < E; e++) p = Mfma<T>::mma(a[j][e], m[j][e], p);
         }
+        acc += p;
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) red[wave][Mfma<T>::drow(lane, q)][i] = acc[q];
