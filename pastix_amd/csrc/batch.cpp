@@ -17,15 +17,23 @@ using namespace pxa_api;
 
 namespace {
 
-int publish_union(pastix_data_t *d, int mtx, int64_t N, const std::vector<int64_t> &cp,
-                  const std::vector<int32_t> &rows, std::vector<double> &vals);
+// A union that is not the instance's yet (lower triangle when symmetric, FP64
+// values): system offsets and CSC.
+struct Union {
+    int mtx = 0;
+    std::vector<int64_t> off, cp;
+    std::vector<int32_t> rows;
+    std::vector<double> vals;
+};
 
 // The union by concatenation, when every system is a CSC whose rows
 // increase strictly within each column (lower-triangle entries only when
 // symmetric): that is already the union's sorted, duplicate-free CSC.
-bool concat_union(pastix_int_t nsys, const spmatrix_t *const *spms, bool values, std::vector<int64_t> &off,
-                  std::vector<int64_t> &cp, std::vector<int32_t> &rows, std::vector<double> &vals) {
-    const int mtx = spms[0]->mtxtype;
+bool concat_union(pastix_int_t nsys, const spmatrix_t *const *spms, bool values, Union &u) {
+    const int mtx = u.mtx;
+    std::vector<int64_t> &off = u.off, &cp = u.cp;
+    std::vector<int32_t> &rows = u.rows;
+    std::vector<double> &vals = u.vals;
     int64_t nnz = 0;
     for (pastix_int_t s = 0; s < nsys; s++) {
         const spmatrix_t *A = spms[s];
@@ -60,20 +68,18 @@ bool concat_union(pastix_int_t nsys, const spmatrix_t *const *spms, bool values,
     return true;
 }
 
-// Union CSC of the systems (lower triangle when symmetric, FP64 values).
-int build_union(pastix_data_t *d, pastix_int_t nsys, const spmatrix_t *const *spms, bool values,
-                std::vector<int64_t> &off) {
+// Union CSC of the systems.
+int build_union(pastix_int_t nsys, const spmatrix_t *const *spms, bool values, Union &un) {
+    if (!spms[0]) return PASTIX_ERR_BADPARAMETER;
+    std::vector<int64_t> &off = un.off;
     off.assign(nsys + 1, 0);
-    const int mtx = spms[0]->mtxtype;
+    const int mtx = un.mtx = spms[0]->mtxtype;
     for (pastix_int_t s = 0; s < nsys; s++) {
         const spmatrix_t *A = spms[s];
         if (!A || A->mtxtype != mtx || A->n <= 0 || A->dof != 1) return PASTIX_ERR_BADPARAMETER;
         if (values && A->flttype != SpmDouble && A->flttype != SpmFloat) return PASTIX_ERR_BADPARAMETER;
     }
-    std::vector<int64_t> cp;
-    std::vector<int32_t> rows;
-    std::vector<double> vals;
-    if (concat_union(nsys, spms, values, off, cp, rows, vals)) return publish_union(d, mtx, off[nsys], cp, rows, vals);
+    if (concat_union(nsys, spms, values, un)) return PASTIX_SUCCESS;
     Triplets u;
     for (pastix_int_t s = 0; s < nsys; s++) {
         const spmatrix_t *A = spms[s];
@@ -90,20 +96,20 @@ int build_union(pastix_data_t *d, pastix_int_t nsys, const spmatrix_t *const *sp
         }
         off[s + 1] = off[s] + A->n;
     }
-    const int64_t N = off[nsys];
-    triplets_to_csc(N, u, nullptr, cp, rows, vals, false);
-    if (!values) vals.assign(rows.size(), 1.0);
-    return publish_union(d, mtx, N, cp, rows, vals);
+    triplets_to_csc(off[nsys], u, nullptr, un.cp, un.rows, un.vals, false);
+    if (!values) un.vals.assign(un.rows.size(), 1.0);
+    return PASTIX_SUCCESS;
 }
 
-int publish_union(pastix_data_t *d, int mtx, int64_t N, const std::vector<int64_t> &cp,
-                  const std::vector<int32_t> &rows, std::vector<double> &vals) {
-    d->u_colptr.assign(cp.begin(), cp.end());
-    d->u_rows.assign(rows.begin(), rows.end());
-    d->u_vals.swap(vals);
+// Makes it the instance's union, the one later batches are compared with.
+void publish_union(pastix_data_t *d, Union &u) {
+    const int64_t N = u.off.back();
+    d->u_colptr.assign(u.cp.begin(), u.cp.end());
+    d->u_rows.assign(u.rows.begin(), u.rows.end());
+    d->u_vals.swap(u.vals);
     spmatrix_t &S = d->u_spm;
     memset(&S, 0, sizeof(S));
-    S.mtxtype = (spm_mtxtype_t)mtx;
+    S.mtxtype = (spm_mtxtype_t)u.mtx;
     S.flttype = SpmDouble;
     S.fmttype = SpmCSC;
     S.gN = S.n = S.gNexp = S.nexp = N;
@@ -113,7 +119,6 @@ int publish_union(pastix_data_t *d, int mtx, int64_t N, const std::vector<int64_
     S.colptr = d->u_colptr.data();
     S.rowptr = d->u_rows.data();
     S.values = d->u_vals.data();
-    return PASTIX_SUCCESS;
 }
 
 // The systems' values into the published union, when every system is a CSC
@@ -302,9 +307,10 @@ int pxa_api::refine_block(pastix_data_t *d, int R, const double *B, double *X, c
 extern "C" int pastix_amd_batch_analyze(pastix_data_t *d, pastix_int_t nsys, const spmatrix_t *const *spms,
                                         const pastix_order_t *const *orders) {
     if (!d || nsys < 1 || !spms) return PASTIX_ERR_BADPARAMETER;
-    std::vector<int64_t> off;
-    int rc = build_union(d, nsys, spms, true, off);
+    Union un;
+    int rc = build_union(nsys, spms, true, un);
     if (rc) return rc;
+    const std::vector<int64_t> &off = un.off;
     // concatenated ordering
     const int64_t N = off[nsys];
     std::vector<pastix_int_t> perm(N), rang, tree;
@@ -340,6 +346,7 @@ extern "C" int pastix_amd_batch_analyze(pastix_data_t *d, pastix_int_t nsys, con
         uo.rangtab = rang.data();
         uo.treetab = tree.data();
     }
+    publish_union(d, un);
     const pastix_int_t saved = d->iparm[IPARM_ORDERING], saved_lo = d->ext[PXA_IPARM_LEVEL_ORDER];
     d->iparm[IPARM_ORDERING] = PastixOrderPersonal;
     d->ext[PXA_IPARM_LEVEL_ORDER] = 0;
@@ -364,14 +371,16 @@ extern "C" int pastix_amd_batch_numfact(pastix_data_t *d, const spmatrix_t *cons
     if (!d || !spms || d->batch_off.size() < 2) return PASTIX_ERR_BADPARAMETER;
     if (refill_union(d, spms)) return pastix_task_numfact(d, &d->u_spm);
     const pastix_int_t nsys = (pastix_int_t)d->batch_off.size() - 1;
-    const size_t nnz = d->u_rows.size();
-    std::vector<int64_t> off;
-    int rc = build_union(d, nsys, spms, true, off);
+    Union un;
+    const int rc = build_union(nsys, spms, true, un);
     if (rc) return rc;
-    if (off != d->batch_off || d->u_rows.size() != nnz) {
+    // a refused batch leaves the analysed union as it is: the next call's
+    // systems are compared with that
+    if (un.off != d->batch_off || un.rows.size() != d->u_rows.size()) {
         err_print("pastix_amd_batch_numfact", "the systems differ from the analysed batch");
         return PASTIX_ERR_BADPARAMETER;
     }
+    publish_union(d, un);
     return pastix_task_numfact(d, &d->u_spm);
 }
 
