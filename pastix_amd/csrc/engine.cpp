@@ -721,20 +721,31 @@ hipGraphExec_t Engine::solve_graph(void *dx, int64_t ldx, int nrhs, bool user) {
     return ex;
 }
 
+// The captured solves, dropped when a block that they work in moves.
+void Engine::drop_solve_graphs() {
+    if (solve_graphs_.empty()) return;
+    (void)hipStreamSynchronize(stream_);
+    for (SolveGraph &g : solve_graphs_) (void)hipGraphExecDestroy(g.exec);
+    solve_graphs_.clear();
+}
+
+// The work block of nrhs right-hand sides.
+int Engine::reserve_rhs(int nrhs) {
+    if (rhs_cap_ >= (int64_t)nrhs * n_) return 0;
+    drop_solve_graphs();
+    release(d_rhs_);
+    rhs_cap_ = (int64_t)nrhs * n_;
+    d_rhs_ = alloc(rhs_cap_ * ((prec_ == 2) ? sizeof(float) : sizeof(double)));
+    if (d_rhs_) return 0;
+    rhs_cap_ = 0;
+    return -1;
+}
+
 // Device solve in the user ordering: permute into the work block, solve,
 // permute back (the timed region includes both permutations).
 int Engine::solve_user_device(void *db, int64_t ldb, int nrhs, double *seconds) {
     if (!d_perm_) return fail("permutation not uploaded");
-    const size_t fsz = (prec_ == 2) ? sizeof(float) : sizeof(double);
-    if (rhs_cap_ < (int64_t)nrhs * n_) {
-        release(d_rhs_);
-        rhs_cap_ = (int64_t)nrhs * n_;
-        d_rhs_ = alloc(rhs_cap_ * fsz);
-        if (!d_rhs_) {
-            rhs_cap_ = 0;
-            return -1;
-        }
-    }
+    if (reserve_rhs(nrhs)) return -1;
     HIPCHK(hipEventRecord(ev0_, stream_));
     if (use_graph) {
         hipGraphExec_t ex = solve_graph(db, ldb, nrhs, true);
@@ -915,15 +926,7 @@ int Engine::solve_device(void *dx, int64_t ldx, int nrhs, double *seconds) {
 
 int Engine::solve_host(const int64_t *perm, int flttype, void *b, int64_t ldb, int nrhs, double *seconds) {
     const size_t fsz = (prec_ == 2) ? sizeof(float) : sizeof(double);
-    if (rhs_cap_ < (int64_t)nrhs * n_) {
-        release(d_rhs_);
-        rhs_cap_ = (int64_t)nrhs * n_;
-        d_rhs_ = alloc(rhs_cap_ * fsz);
-        if (!d_rhs_) {
-            rhs_cap_ = 0;
-            return -1;
-        }
-    }
+    if (reserve_rhs(nrhs)) return -1;
     // permute on the host into the factor precision: xp[perm[i]] = b[i]
     const size_t bytes = (size_t)n_ * nrhs * fsz;
     std::vector<char> big;
@@ -1142,6 +1145,7 @@ void Engine::release_work() {
     release(d_bscal_);
     release(d_bsvec_);
     release(d_cpart_);
+    drop_solve_graphs();
     release(d_rhs_);
     sr_cap_ = bvec_cap_ = bscal_cap_ = bsvec_cap_ = cpart_cap_ = rhs_cap_ = 0;
 }

@@ -283,6 +283,8 @@ class Engine {
     int enqueue_factorize(double thr);
     int enqueue_solve(void *dx, int64_t ldx, int nrhs, bool user);
     hipGraphExec_t solve_graph(void *dx, int64_t ldx, int nrhs, bool user);
+    void drop_solve_graphs();
+    int reserve_rhs(int nrhs);
     struct Span {
         int cls, e0, e1, lv;
     };
