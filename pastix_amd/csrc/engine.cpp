@@ -44,16 +44,79 @@ int Engine::fail(const std::string &m) {
     return -1;
 }
 
-void *Engine::alloc(size_t bytes) {
+// hipMalloc on the engine's device (a solve may allocate: the calling thread's
+// may be another one), nullptr without a trace when there is no room
+void *Engine::try_alloc(size_t bytes) {
     void *p = nullptr;
     if (bytes == 0) bytes = 8;
-    if (hipMalloc(&p, bytes + LOAD_PAD) != hipSuccess) {
-        fail("hipMalloc of " + std::to_string(bytes) + " bytes failed");
+    int cur = dev_;
+    (void)hipGetDevice(&cur);
+    if (cur != dev_) (void)hipSetDevice(dev_);
+    const hipError_t e = hipMalloc(&p, bytes + LOAD_PAD);
+    if (cur != dev_) (void)hipSetDevice(cur);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         return nullptr;
     }
     owned_.push_back(Owned{p, bytes});
     bytes_ += (int64_t)bytes;
     return p;
+}
+
+void *Engine::alloc(size_t bytes) {
+    void *p = try_alloc(bytes);
+    // the sweeps' wider vectors are given up for anything else
+    if (!p && nrhs_chunk_ > SWEEP_COLS && !alloc_sweep(SWEEP_COLS)) p = try_alloc(bytes);
+    if (!p) fail("hipMalloc of " + std::to_string(bytes) + " bytes failed");
+    return p;
+}
+
+// The vectors of a sweep of that many right-hand sides, in the place of those
+// there were (no sweep is under way); nothing is held when it fails.
+int64_t Engine::sweep_bytes(int cols) const {
+    return (int64_t)(prec_ == 2 ? sizeof(float) : sizeof(double)) * cols * (bwd_part_ + nyrows_ + n_);
+}
+int Engine::alloc_sweep(int cols) {
+    const size_t fsz = (prec_ == 2) ? sizeof(float) : sizeof(double);
+    drop_solve_graphs();
+    release(d_part_);
+    release(d_ybuf_);
+    release(d_z_);
+    nrhs_chunk_ = 0;
+    const size_t ny = (size_t)std::max<int64_t>(nyrows_, 1) * cols * fsz;
+    d_part_ = try_alloc((size_t)std::max<int64_t>(bwd_part_, 1) * cols * fsz);
+    d_ybuf_ = d_part_ ? try_alloc(ny) : nullptr;
+    d_z_ = d_ybuf_ ? try_alloc((size_t)std::max<int64_t>(n_, 1) * cols * fsz) : nullptr;
+    // The update-buffer entries of the Schur cblks' own rows are never
+    // written (Schur cblks are not sources) and the Interface forward sweep
+    // subtracts every entry of a Schur row: they must read as zero.
+    if (!d_z_ || (schurfcol_ < n_ && hipMemsetAsync(d_ybuf_, 0, ny, stream_) != hipSuccess)) {
+        release(d_part_);
+        release(d_ybuf_);
+        release(d_z_);
+        return -1;
+    }
+    nrhs_chunk_ = cols;
+    return 0;
+}
+
+// Before a solve of nrhs right-hand sides.  The first one of more than
+// SWEEP_COLS widens the sweeps to 64, where their vectors take at most 4 GiB
+// and at most a quarter of the memory left: sweeps of 64 cost hardly more
+// launches' time than those of 32 (24 levels of 6 launches, most of them a few
+// us long): three FP32 preconditioner solves of 64 columns (56x48x60) and
+// their CG 7.95 ms in halves, 6.04 ms at once; 128 at a time 6.01.  An
+// instance that never sees so many holds the vectors of 32 (FP32 96^3: 1.77
+// GiB less of 12.1).
+int Engine::reserve_sweep(int nrhs) {
+    if (nrhs_chunk_ == 0 && alloc_sweep(SWEEP_COLS)) return fail("no device memory for the solve");
+    if (nrhs <= SWEEP_COLS || nrhs_chunk_ >= SWEEP_WIDE || keep_sweep) return 0;
+    size_t freeb = 0, totb = 0;
+    if (sweep_bytes(SWEEP_WIDE) > ((int64_t)4 << 30) || hipMemGetInfo(&freeb, &totb) != hipSuccess ||
+        wide_sweep_bytes() > (int64_t)(freeb / 4))
+        return 0;
+    if (alloc_sweep(SWEEP_WIDE) && alloc_sweep(SWEEP_COLS)) return fail("no device memory for the solve");
+    return 0;
 }
 
 void Engine::release_ptr(void *p) {
@@ -324,26 +387,9 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     if (P.winv_tmax > 0 && !(d_tbuf_ = alloc((size_t)P.winv_tmax * fsz))) return -1;
     d_WB_ = alloc(winvnbr_ * fsz);
     if (d_WB_) HIPCHK(hipMemsetAsync(d_WB_, 0, winvnbr_ * fsz, stream_));
-    // right-hand sides of one sweep: up to 64 (32 where the sweep's vectors
-    // would take over 4 GiB), the kernels taking them in groups of 16 or 32 on
-    // the grid.  The sweep of 64 costs hardly more launches' time than that of
-    // 32 (24 levels of 6 launches, most of them a few us long): three FP32
-    // preconditioner solves of 64 columns (56x48x60) and their CG 7.95 ms in
-    // halves, 6.04 ms at once; 128 at a time 6.01.
-    const int64_t column = (int64_t)fsz * (bwd_part_ + nyrows_ + n_);
-    nrhs_chunk_ = column * 64 <= ((int64_t)4 << 30) ? 64 : 32;
-    d_part_ = alloc((size_t)std::max<int64_t>(bwd_part_, 1) * nrhs_chunk_ * fsz);
-    d_ybuf_ = alloc((size_t)std::max<int64_t>(nyrows_, 1) * nrhs_chunk_ * fsz);
-    d_z_ = alloc((size_t)std::max<int64_t>(n_, 1) * nrhs_chunk_ * fsz);
-    if (!d_z_) return -1;
-    if (!d_WB_ || !d_ybuf_) return -1;
-    // The update-buffer entries of the Schur cblks' own rows are never
-    // written (Schur cblks are not sources) and the Interface forward sweep
-    // subtracts every entry of a Schur row: they must read as zero.
-    if (schurfcol_ < n_)
-        HIPCHK(hipMemsetAsync(d_ybuf_, 0, (size_t)std::max<int64_t>(nyrows_, 1) * nrhs_chunk_ * fsz, stream_));
+    if (!d_WB_ || alloc_sweep(SWEEP_COLS)) return fail("no device memory for the solve");
     d_red_ = (double *)alloc((size_t)(512 * 32 + 64) * sizeof(double));
-    if (!d_part_ || !d_red_ || !d_stat_) return -1;
+    if (!d_red_ || !d_stat_) return -1;
     HIPCHK(hipStreamSynchronize(stream_));
     inited_ = true;
     return 0;
@@ -745,7 +791,7 @@ int Engine::reserve_rhs(int nrhs) {
 // permute back (the timed region includes both permutations).
 int Engine::solve_user_device(void *db, int64_t ldb, int nrhs, double *seconds) {
     if (!d_perm_) return fail("permutation not uploaded");
-    if (reserve_rhs(nrhs)) return -1;
+    if (reserve_sweep(nrhs) || reserve_rhs(nrhs)) return -1;
     HIPCHK(hipEventRecord(ev0_, stream_));
     if (use_graph) {
         hipGraphExec_t ex = solve_graph(db, ldb, nrhs, true);
@@ -907,6 +953,7 @@ template <typename T> int Engine::solve_t(T *x, int64_t ldx, int nrhs) {
 
 int Engine::solve_device(void *dx, int64_t ldx, int nrhs, double *seconds) {
     if (!inited_) return fail("engine not initialised");
+    if (reserve_sweep(nrhs)) return -1;
     HIPCHK(hipEventRecord(ev0_, stream_));
     if (use_graph) {
         hipGraphExec_t ex = solve_graph(dx, ldx, nrhs, false);
@@ -1131,6 +1178,7 @@ double Engine::dot(const double *x, const double *y) {
 }
 
 int Engine::precond(double *dv) {
+    if (reserve_sweep(1)) return -1;
     if (prec_ == 3) return solve_t<double>(dv, n_, 1);
     launch_d2s(n_, dv, d_svec_, stream_);
     int rc = solve_t<float>(d_svec_, n_, 1);
@@ -1163,6 +1211,7 @@ int64_t Engine::work_bytes(int R) const {
 // zb = M^{-1} rb, R columns
 int Engine::precond_block(const double *rb, double *zb, int R) {
     const int64_t nr = n_ * (int64_t)R;
+    if (reserve_sweep(R)) return -1;
     if (prec_ == 3) {
         launch_copy(nr, rb, zb, stream_);
         return solve_t<double>(zb, n_, R);

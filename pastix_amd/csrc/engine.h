@@ -100,6 +100,12 @@ class Engine {
     hipStream_t stream() const { return stream_; }
     int64_t n() const { return n_; }
     void *alloc(size_t bytes);
+    // Device bytes that sweeps of SWEEP_WIDE right-hand sides take beyond
+    // those of SWEEP_COLS; reserve_sweep makes room for a solve of nrhs.
+    static constexpr int SWEEP_COLS = 32, SWEEP_WIDE = 64;
+    int64_t wide_sweep_bytes() const { return sweep_bytes(SWEEP_WIDE) - sweep_bytes(SWEEP_COLS); }
+    int reserve_sweep(int nrhs);
+    bool keep_sweep = false;  // sweeps stay as wide as they are
     // frees a buffer from alloc() (no-op on nullptr) and sets it to nullptr
     template <typename P> void release(P *&p) {
         release_ptr((void *)p);
@@ -284,6 +290,9 @@ class Engine {
     int enqueue_solve(void *dx, int64_t ldx, int nrhs, bool user);
     hipGraphExec_t solve_graph(void *dx, int64_t ldx, int nrhs, bool user);
     void drop_solve_graphs();
+    void *try_alloc(size_t bytes);
+    int64_t sweep_bytes(int cols) const;
+    int alloc_sweep(int cols);
     int reserve_rhs(int nrhs);
     struct Span {
         int cls, e0, e1, lv;
@@ -298,7 +307,7 @@ class Engine {
     void *d_L_ = nullptr, *d_U_ = nullptr, *d_W1_ = nullptr, *d_W2_ = nullptr;
     int *d_stat_ = nullptr;
     void *d_part_ = nullptr;
-    int nrhs_chunk_ = 32;
+    int nrhs_chunk_ = 0;  // right-hand sides of one sweep (0: its vectors aren't there)
     void *d_rhs_ = nullptr;  // n x nrhs_cap work block in factor precision
     int64_t rhs_cap_ = 0;
     double *d_red_ = nullptr;  // reduction partials + scalars

@@ -76,9 +76,12 @@ struct PastixSlotOps final : pxa::ServeOps {
         }
         int it = 0;
         double res = 0;
+        // no memory beyond what was admitted: the sweeps stay as they are
+        d->engine->keep_sweep = true;
         if (!rc && d->engine->refine_user(dB, n, dX, n, (int)R, std::vector<int64_t>{0, n}, 1, true, true,
                                           (int)d->iparm[IPARM_ITERMAX], 1, refine_eps(d), &it, &res))
             rc = PASTIX_ERR_INTERNAL;
+        d->engine->keep_sweep = false;
         c0 = 0;
         for (const pxa::SolveCols &r : batch) {
             if (!rc && hipMemcpy2DAsync(r.b, (size_t)r.ldb * sizeof(double), dX + (size_t)c0 * n, col, col,
@@ -113,9 +116,6 @@ extern "C" int pastix_amd_server_create(pastix_amd_server_t **srv, pastix_data_t
             d->iparm[IPARM_FACTORIZATION] == PastixFactGETRF || is_ldlt(d) || d->schurfcol < d->n)
             return PASTIX_ERR_BADPARAMETER;
     }
-    auto *S = new pastix_amd_server_s();
-    S->ops.slots.assign(slots, slots + nslots);
-    S->ops.n = slots[0]->n;
     // the work budget: IPARM_GPU_MEMORY_PERCENTAGE of the memory left free
     size_t freeb = 0, totb = 0;
     (void)hipSetDevice((int)slots[0]->ext[PXA_IPARM_DEVICE]);
@@ -123,6 +123,20 @@ extern "C" int pastix_amd_server_create(pastix_amd_server_t **srv, pastix_data_t
     const pastix_int_t pct =
         std::max<pastix_int_t>(1, std::min<pastix_int_t>(100, slots[0]->iparm[IPARM_GPU_MEMORY_PERCENTAGE]));
     const int64_t budget = (int64_t)((double)freeb * (double)pct / 100.0);
+    // merged solves of many right-hand sides take wider sweeps where those
+    // fit half of what the budget leaves free: nothing that it admits without
+    // them is refused
+    int64_t wide = 0;
+    for (int k = 0; k < nslots; k++) wide += slots[k]->engine->wide_sweep_bytes();
+    if (wide <= ((int64_t)freeb - budget) / 2)
+        for (int k = 0; k < nslots; k++) {
+            (void)hipSetDevice((int)slots[k]->ext[PXA_IPARM_DEVICE]);
+            if (slots[k]->engine->reserve_sweep((int)std::min<pastix_int_t>(max_rhs, pxa::Engine::SWEEP_WIDE)))
+                return PASTIX_ERR_OUTOFMEMORY;
+        }
+    auto *S = new pastix_amd_server_s();
+    S->ops.slots.assign(slots, slots + nslots);
+    S->ops.n = slots[0]->n;
     S->core = std::make_unique<pxa::ServeCore>(&S->ops, nslots, (int64_t)max_rhs, budget, PASTIX_ERR_OUTOFMEMORY);
     *srv = S;
     return PASTIX_SUCCESS;
