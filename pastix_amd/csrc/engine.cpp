@@ -395,23 +395,29 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     return 0;
 }
 
-double *Engine::host_block(int64_t count) {
-    if (h_pin_cap_ < count) {
-        if (h_pin_) (void)hipHostFree(h_pin_);
+bool Engine::grow_pinned(int64_t count) {
+    if (h_pin_cap_ >= count) return true;
+    if (h_pin_) (void)hipHostFree(h_pin_);
+    h_pin_ = nullptr;
+    h_pin_cap_ = 0;
+    if (hipHostMalloc((void **)&h_pin_, (size_t)count * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        // the error is this call's: the check after the next launches must
+        // not find it
+        (void)hipGetLastError();
         h_pin_ = nullptr;
-        h_pin_cap_ = 0;
-        if (hipHostMalloc((void **)&h_pin_, (size_t)count * sizeof(double), hipHostMallocDefault) != hipSuccess) {
-            h_pin_ = nullptr;
-            fail("hipHostMalloc of " + std::to_string(count * sizeof(double)) + " bytes failed");
-            return nullptr;
-        }
-        h_pin_cap_ = count;
+        return false;
     }
+    h_pin_cap_ = count;
+    return true;
+}
+
+double *Engine::host_block(int64_t count) {
+    if (!grow_pinned(count)) fail("hipHostMalloc of " + std::to_string(count * sizeof(double)) + " bytes failed");
     return h_pin_;
 }
 
 void *Engine::small_block(size_t bytes) {
-    return bytes <= SMALL_COPY ? host_block((int64_t)(SMALL_COPY / sizeof(double))) : nullptr;
+    return bytes <= SMALL_COPY && grow_pinned((int64_t)(SMALL_COPY / sizeof(double))) ? h_pin_ : nullptr;
 }
 
 int Engine::download_diag(double *h) {

@@ -291,6 +291,7 @@ class Engine {
     hipGraphExec_t solve_graph(void *dx, int64_t ldx, int nrhs, bool user);
     void drop_solve_graphs();
     void *try_alloc(size_t bytes);
+    bool grow_pinned(int64_t count);
     int64_t sweep_bytes(int cols) const;
     int alloc_sweep(int cols);
     int reserve_rhs(int nrhs);
