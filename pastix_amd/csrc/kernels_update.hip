@@ -201,8 +201,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
 // workspace, 465 with 64 columns of sums and four waves for every tile, 181 so
 // (16 columns 180, 32 columns 232); its five narrow levels 1578 -> 514 us,
 // numfact 4.0 -> 3.1 ms.  Subtracting entry by entry without LDS took 485 us,
-// but rounds every entry at the target's magnitude.  Panels below 2 GiB
-// (32-bit lane offsets).
+// but rounds every entry at the target's magnitude.  Source panels of at most
+// NARROW_ROWS rows (32-bit lane offsets of up to three columns).
 template <typename T, int MODE, int NW, int NC>
 __global__ __launch_bounds__(64 * NW) void k_update_narrow(DevSymbol S, const UpdItem *__restrict__ items, int nitems,
                                                        const UpdX *__restrict__ xs, const int32_t *__restrict__ shift,

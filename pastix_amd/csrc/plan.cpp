@@ -96,8 +96,6 @@ Plan build_plan(const Symbol &s, const Layout &L, int64_t schur_cblk, const Plan
     P.lv_wsize.assign(nl, 0);
     P.lv_single_pass.assign(nl, 0);
     P.lv_narrow.assign(nl, 0);
-    int64_t panel_max = 0;
-    for (int64_t c = 0; c < s.cblknbr(); c++) panel_max = std::max(panel_max, L.cblk_stride[c] * width(c));
     P.lv_panel_right.assign(nl, 0);
     std::vector<KeyEnt> ke;
     std::vector<Range> rr, cr;
@@ -298,9 +296,12 @@ Plan build_plan(const Symbol &s, const Layout &L, int64_t schur_cblk, const Plan
                 nm++;
                 nme += P.upd[t].e1 - P.upd[t].e0;
             }
-            int64_t mw = 0;
-            for (int32_t k = l0; k < lf; k++) mw = std::max<int64_t>(mw, width(P.lv_cblks[k]));
-            P.lv_narrow[lv] = mw <= NARROW_UPD && panel_max < NARROW_PANEL;
+            int64_t mw = 0, ml = 0;
+            for (int32_t k = l0; k < lf; k++) {
+                mw = std::max<int64_t>(mw, width(P.lv_cblks[k]));
+                ml = std::max<int64_t>(ml, L.cblk_stride[P.lv_cblks[k]]);
+            }
+            P.lv_narrow[lv] = mw <= NARROW_UPD && ml <= NARROW_ROWS;
             P.lv_single_pass[lv] =
                 nm > 0 && (knobs.sp(lv) >= 0 ? knobs.sp(lv) != 0
                                              : P.lv_narrow[lv] || (double)nme <= SINGLE_PASS_ENTS * (double)nm);

@@ -17,8 +17,9 @@ constexpr double SINGLE_PASS_ENTS = 2.05;
 // Laplacian, the workspace 784 to 88; with up to 22 and 32 columns a wave per
 // tile took as long as the workspace (64 and 66, 62 and 62 us), with 50 longer
 constexpr int64_t NARROW_UPD = 16;
-// largest panel (entries) on which that kernel's 32-bit byte offsets hold
-constexpr int64_t NARROW_PANEL = (int64_t)1 << 28;
+// most rows of a source's panel: that kernel's lane offsets, up to three
+// columns and 64 rows of a source in bytes, have 32 bits (targets have 64)
+constexpr int64_t NARROW_ROWS = (int64_t)1 << 27;
 // levels with fewer 64-row panel tiles than this update their panels
 // right-looking (64-deep products over all later blocks)
 constexpr int64_t PANEL_RIGHT_ROWTILES = 200;
