@@ -161,8 +161,9 @@ int pastix_amd_fact_times(const pastix_data_t *pastix_data, double out[8]);
  * update of one level per span), 1 single-source update tiles
  * (k_update_direct), 2 multi-source product tiles (k_update_wgemm), 3
  * multi-source ordered sums (k_update_gather), 4 single-pass multi-source
- * update (k_update_seq, levels of few entries per tile and levels whose
- * products exceed the workspace),
+ * updates (k_update_narrow on levels of sources of at most 16 columns, else
+ * k_update_seq: levels of few entries per tile and levels whose products
+ * exceed the workspace),
  * 5 the leaf region's persistent task launch (PXA_IPARM_LEAF_TASKS).
  * Every span of classes 1-4 is exactly one kernel launch (LU runs the L
  * and U sides as separate launches). */
@@ -174,7 +175,7 @@ int pastix_amd_kernel_times(const pastix_data_t *pastix_data, double out[12]);
  * L side (block(p) >= block(q)), out[2], out[3] the same for the U side of
  * LU (block(p) > block(q)), out[4] the flops of the multi-source product
  * tiles as computed (one side), out[5], out[6] the multi-source tiles of
- * single-pass levels (k_update_seq), L and U side, out[7] the updates inside
+ * single-pass levels (k_update_narrow, k_update_seq), L and U side, out[7] the updates inside
  * the leaf region's persistent launch.  With that launch on, out[0..6] count
  * what the level kernels run: the region's levels leave them and its
  * updates into the supernodes above it join out[0] and out[5]. */

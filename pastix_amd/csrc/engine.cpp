@@ -624,15 +624,23 @@ template <typename T> int Engine::factorize_t(double thr) {
                 launch_update_gather<T>(S_, mode, d_upd_ + ma, mb - ma, d_ents_, d_shift_, d_wgrp_, Wk, C, st);
                 prof_end(KC_GATHER, k, st);
             } else {
-                k = prof_begin(st);
+                // one launch to a span: narrow levels have the tiles of few
+                // columns and the others on either side of the next-level split
                 if (narrow) {
                     const int r[3] = {us, lv_upd_mnext_[lv], u1};
-                    for (int s = 0; s < 2; s++)
-                        if (ma <= r[s] && r[s + 1] <= mb)
-                            launch_update_narrow<T>(S_, mode, d_upd_ + r[s], r[s + 1] - r[s], lv_few_[2 * lv + s],
-                                                    d_updx_, d_shift_, A, B, C, st);
-                } else
-                    launch_update_seq<T>(S_, mode, d_upd_ + ma, mb - ma, d_updx_, d_shift_, A, B, C, st == side_, st);
+                    for (int s = 0; s < 4; s++) {
+                        const int a = r[s / 2], b = r[s / 2 + 1], few = a + lv_few_[2 * lv + s / 2];
+                        const int t0 = s % 2 ? few : a, t1 = s % 2 ? b : few;
+                        if (ma > a || b > mb || t1 <= t0) continue;
+                        k = prof_begin(st);
+                        launch_update_narrow<T>(S_, mode, d_upd_ + t0, t1 - t0, s % 2 == 0, d_updx_, d_shift_, A, B,
+                                                C, st);
+                        prof_end(KC_ACC, k, st);
+                    }
+                    return;
+                }
+                k = prof_begin(st);
+                launch_update_seq<T>(S_, mode, d_upd_ + ma, mb - ma, d_updx_, d_shift_, A, B, C, st == side_, st);
                 prof_end(KC_ACC, k, st);
             }
         };

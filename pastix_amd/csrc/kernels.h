@@ -14,10 +14,10 @@ void launch_update_direct(const DevSymbol &S, int mode, const UpdX *xs, int n, c
 template <typename T>
 void launch_update_seq(const DevSymbol &S, int mode, const UpdItem *items, int n, const UpdX *xs,
                        const int32_t *shift, const T *A, const T *B, T *C, bool beside, hipStream_t st);
-// One-pass update of the multi-source tiles of a level of narrow sources: the
-// first `few` items receive entries in at most NARROW_COLS columns.
+// One-pass update of multi-source tiles of a level of narrow sources that
+// receive entries in at most NARROW_COLS columns (few) or in any number.
 template <typename T>
-void launch_update_narrow(const DevSymbol &S, int mode, const UpdItem *items, int n, int few, const UpdX *xs,
+void launch_update_narrow(const DevSymbol &S, int mode, const UpdItem *items, int n, bool few, const UpdX *xs,
                           const int32_t *shift, const T *A, const T *B, T *C, hipStream_t st);
 // Two-phase update of the multi-source tiles: dense product tiles into the
 // level workspace W, then the per-target-tile ordered sum.

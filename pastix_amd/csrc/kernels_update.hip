@@ -539,21 +539,15 @@ void launch_update_seq(const DevSymbol &S, int mode, const UpdItem *items, int n
 }
 
 template <typename T>
-void launch_update_narrow(const DevSymbol &S, int mode, const UpdItem *items, int n, int few, const UpdX *xs,
+void launch_update_narrow(const DevSymbol &S, int mode, const UpdItem *items, int n, bool few, const UpdX *xs,
                           const int32_t *shift, const T *A, const T *B, T *C, hipStream_t st) {
     if (n <= 0) return;
-    auto run = [&](auto kernel, int waves, const UpdItem *it, int m) {
-        if (m > 0)
-            hipLaunchKernelGGL(kernel, dim3(grid8(m)), dim3(64 * waves), 0, st, S, it, m, xs, shift, A, B, C);
+    auto run = [&](auto kernel, int waves) {
+        hipLaunchKernelGGL(kernel, dim3(grid8(n)), dim3(64 * waves), 0, st, S, items, n, xs, shift, A, B, C);
     };
     constexpr int W = NARROW_COLS;
-    if (mode == 0) {
-        run(k_update_narrow<T, 0, 2, W>, 2, items, few);
-        run(k_update_narrow<T, 0, 4, 64>, 4, items + few, n - few);
-    } else {
-        run(k_update_narrow<T, 1, 2, W>, 2, items, few);
-        run(k_update_narrow<T, 1, 4, 64>, 4, items + few, n - few);
-    }
+    if (few) mode == 0 ? run(k_update_narrow<T, 0, 2, W>, 2) : run(k_update_narrow<T, 1, 2, W>, 2);
+    else mode == 0 ? run(k_update_narrow<T, 0, 4, 64>, 4) : run(k_update_narrow<T, 1, 4, 64>, 4);
 }
 
 template <typename T>
@@ -576,7 +570,7 @@ void launch_update_gather(const DevSymbol &S, int mode, const UpdItem *items, in
                                           const T *, T *, bool, hipStream_t);                                     \
     template void launch_update_seq<T>(const DevSymbol &, int, const UpdItem *, int, const UpdX *,                \
                                        const int32_t *, const T *, const T *, T *, bool, hipStream_t);            \
-    template void launch_update_narrow<T>(const DevSymbol &, int, const UpdItem *, int, int, const UpdX *,        \
+    template void launch_update_narrow<T>(const DevSymbol &, int, const UpdItem *, int, bool, const UpdX *,       \
                                           const int32_t *, const T *, const T *, T *, hipStream_t);               \
     template void launch_update_wgemm<T>(const DevSymbol &, const WTile *, int, const T *, const T *, T *,        \
                                          hipStream_t);                                                            \
