@@ -7,6 +7,10 @@
 
 namespace pxa {
 
+// xs[it.e0 .. it.e1) of every item: the plan's entries ents[from[t] ...) of
+// item t as the one-pass kernels read them (items of from[t] < 0: none).
+void launch_update_entries(const DevSymbol &S, const UpdItem *items, int n, const int32_t *from, const UpdEntry *ents,
+                           UpdX *xs, hipStream_t st);
 // direct: every item has exactly one entry (no LDS accumulation).
 template <typename T>
 void launch_update_direct(const DevSymbol &S, int mode, const UpdX *xs, int n, const int32_t *shift, const T *A,

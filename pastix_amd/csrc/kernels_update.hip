@@ -26,6 +26,40 @@
 
 namespace pxa {
 
+// The one-pass kernels' entries from the plan's, once per engine: sixteen
+// lanes to an item.
+__global__ __launch_bounds__(256) void k_update_entries(DevSymbol S, const UpdItem *__restrict__ items, int n,
+                                                        const int32_t *__restrict__ from,
+                                                        const UpdEntry *__restrict__ ents, UpdX *__restrict__ xs) {
+    const int id = blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (id >= n || from[id] < 0) return;
+    const UpdItem it = items[id];
+    const UpdEntry *src = ents + from[id];
+    const int64_t c = S.cblk_coef[it.f];
+    const int stf = S.cblk_stride[it.f], fcol = S.cblk_fcol[it.f];
+    for (int e = threadIdx.x & 15; e < it.e1 - it.e0; e += 16) {
+        const UpdEntry en = src[e];
+        UpdX x{};
+        x.a = S.cblk_coef[en.s] + en.p0;
+        x.c = c;
+        x.rb = S.cblk_rowbase[en.s] + en.p0;
+        x.K = S.cblk_fcol[en.s + 1] - S.cblk_fcol[en.s];
+        x.ld = S.cblk_stride[en.s];
+        x.stf = stf;
+        x.np = en.p1 - en.p0;
+        x.nq = en.q1 - en.q0;
+        x.dq = en.q0 - en.p0;
+        x.sbi = en.sb - en.ib0;
+        x.fcol = fcol;
+        xs[it.e0 + e] = x;
+    }
+}
+void launch_update_entries(const DevSymbol &S, const UpdItem *items, int n, const int32_t *from, const UpdEntry *ents,
+                           UpdX *xs, hipStream_t st) {
+    if (n > 0)
+        hipLaunchKernelGGL(k_update_entries, dim3((n + 15) / 16), dim3(256), 0, st, S, items, n, from, ents, xs);
+}
+
 // K columns staged per LDS chunk in the single-tile GEMMs (16 measured
 // faster than 32 on gfx950: the smaller LDS footprint keeps 6 workgroups per
 // CU resident; two buffers of 8 columns with one barrier each were no faster,
