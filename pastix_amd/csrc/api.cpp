@@ -635,6 +635,23 @@ struct RowSums {
     double f2 = 0, ninf = 0, diag = 0;
 };
 
+// Rows are summed in chunks that end at the systems of a batch, the chunks in
+// order, so that the sums don't depend on the threads: up to 512 rows and
+// 32,768 entries (by rows alone, the 1500 of a dense matrix were three chunks
+// for sixteen threads: 2.1 ms instead of 0.6).
+static void cut_chunks(pxa::HostBcsc &bc, const std::vector<int64_t> &systems) {
+    bc.chunk_batch = systems;
+    bc.chunks.assign(1, 0);
+    std::vector<int64_t> ends(systems);
+    ends.push_back(bc.n);
+    for (int64_t e : ends)
+        for (int64_t i = bc.chunks.back(); i < e;) {
+            const int64_t i0 = i++;
+            while (i < e && i < i0 + 512 && bc.rowptr[i + 1] - bc.rowptr[i0] <= (1 << 15)) i++;
+            bc.chunks.push_back(i);
+        }
+}
+
 // Rows [bc.chunks[c], bc.chunks[c+1]) of the permuted matrix: the sums of
 // bc.tvals, which `value(e)` refills first (the values are summed while they
 // are in cache).
@@ -725,17 +742,9 @@ extern "C" int pastix_subtask_spm2bcsc(pastix_data_t *d, spmatrix_t *spm) {
     }
     if (spm->n != d->n) { err_print("pastix_subtask_spm2bcsc", "matrix size differs from the analysed one"); return PASTIX_ERR_BADPARAMETER; }
     pxa::HostBcsc &bc = d->bcsc;
-    // rows are summed in chunks that end at the systems of a batch, the chunks
-    // in order: the sums don't depend on the threads
     const bool batch = d->batch_off.size() > 2 && d->batch_off.back() == d->n;
-    if (bc.chunks.empty() || bc.chunks.back() != d->n || bc.chunk_batch != (batch ? d->batch_off : std::vector<int64_t>())) {
-        bc.chunk_batch = batch ? d->batch_off : std::vector<int64_t>();
-        bc.chunks.assign(1, 0);
-        std::vector<int64_t> ends(bc.chunk_batch);
-        ends.push_back(d->n);
-        for (int64_t e : ends)
-            while (bc.chunks.back() < e) bc.chunks.push_back(std::min(e, bc.chunks.back() + 512));
-    }
+    const std::vector<int64_t> systems = batch ? d->batch_off : std::vector<int64_t>();
+    if (bc.in_fmt >= 0 && bc.chunk_batch != systems) cut_chunks(bc, systems);
     std::vector<RowSums> sums;
     // the analysed pattern again: the permuted values by one gather
     if (!refill_values(spm, bc, sums)) {
@@ -749,6 +758,7 @@ extern "C" int pastix_subtask_spm2bcsc(pastix_data_t *d, spmatrix_t *spm) {
         bc.src.resize(tsrc.size());
         for (size_t q = 0; q < tsrc.size(); q++) bc.src[q] = t.src[tsrc[q]];
         keep_pattern(spm, bc);
+        cut_chunks(bc, systems);
         bc.cmap.clear();
         bc.cmap_facto = -1;
         if (d->engine) d->engine->drop_matrix();
