@@ -661,15 +661,14 @@ template <class V> static RowSums chunk_rows(pxa::HostBcsc &bc, int64_t c, const
     double *v = bc.tvals.data();
     for (int64_t e = bc.rowptr[i0]; e < bc.rowptr[i1]; e++) v[e] = value(e);
     for (int64_t i = i0; i < i1; i++) {
-        double r = 0, r2 = 0, dg = 0;
+        double r = 0, r2 = 0;
         for (int64_t e = bc.rowptr[i]; e < bc.rowptr[i + 1]; e++) {
             r2 += v[e] * v[e];
             r += std::fabs(v[e]);
-            dg += bc.cols[e] == i ? v[e] : 0.0;  // a select: a branch here is missed once per row
         }
         s.f2 += r2;
         s.ninf = std::max(s.ninf, r);
-        s.diag += dg;
+        s.diag += bc.diag[i] >= 0 ? v[bc.diag[i]] : 0.0;
     }
     return s;
 }
@@ -759,6 +758,10 @@ extern "C" int pastix_subtask_spm2bcsc(pastix_data_t *d, spmatrix_t *spm) {
         for (size_t q = 0; q < tsrc.size(); q++) bc.src[q] = t.src[tsrc[q]];
         keep_pattern(spm, bc);
         cut_chunks(bc, systems);
+        bc.diag.assign(bc.n, -1);
+        for (int64_t i = 0; i < bc.n; i++)
+            for (int64_t e = bc.rowptr[i]; e < bc.rowptr[i + 1]; e++)
+                if (bc.cols[e] == i) bc.diag[i] = e;
         bc.cmap.clear();
         bc.cmap_facto = -1;
         if (d->engine) d->engine->drop_matrix();

@@ -1049,12 +1049,8 @@ int Engine::upload_matrix(const HostBcsc &bc) {
         d_cols_ = upload(*this, bc.cols);
         d_vals_ = (double *)alloc(bc.tvals.size() * sizeof(double));
         if (!d_rowptr_ || !d_cols_ || !d_vals_) return -1;
-        std::vector<int64_t> cd(n_, -1);
-        for (int64_t i = 0; i < n_; i++)
-            for (int64_t k = bc.rowptr[i]; k < bc.rowptr[i + 1]; k++)
-                if (bc.cols[k] == i) cd[i] = k;
-        diag_complete_ = std::find(cd.begin(), cd.end(), (int64_t)-1) == cd.end();
-        d_csrdiag_ = upload(*this, cd);
+        diag_complete_ = std::find(bc.diag.begin(), bc.diag.end(), (int64_t)-1) == bc.diag.end();
+        d_csrdiag_ = upload(*this, bc.diag);
         d_diag0_ = (double *)alloc(n_ * sizeof(double));
         if (!d_csrdiag_ || !d_diag0_) return -1;
         have_matrix_ = true;

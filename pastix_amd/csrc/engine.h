@@ -367,6 +367,7 @@ struct HostBcsc {
     std::vector<int32_t> cols;
     std::vector<double> tvals;
     double normF = 0, normInf = 0, diag_sum = 0;
+    std::vector<int64_t> diag;  // every row's diagonal entry (-1: not stored)
     // row ranges the sums are taken over, and the batch they were cut for
     std::vector<int64_t> chunks, chunk_batch;
     // A later input with the same pattern is refilled by one gather: the
