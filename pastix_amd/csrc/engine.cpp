@@ -993,7 +993,7 @@ int Engine::solve_host(const int64_t *perm, int flttype, void *b, int64_t ldb, i
     // permute on the host into the factor precision: xp[perm[i]] = b[i]
     const size_t bytes = (size_t)n_ * nrhs * fsz;
     std::vector<char> big;
-    void *tmp = small_block(bytes);
+    void *tmp = bytes <= SMALL_SOLVE ? small_block(bytes) : nullptr;
     if (!tmp) {
         big.resize(bytes);
         tmp = big.data();

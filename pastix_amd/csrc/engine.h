@@ -45,6 +45,13 @@ class Engine {
     // pinned memory) nullptr: the copy goes from the caller's memory.
     void *small_block(size_t bytes);
     static constexpr size_t SMALL_COPY = 1 << 20;
+    // Right-hand sides of a host solve go through it up to half of that: they
+    // are permuted into and out of it, which costs more the larger it is.
+    // Host part of a solve, from the pinned block and from the heap (one of
+    // two times, as the copy happens to be staged): 62 KB 63-79 and 113-128
+    // us, 210 KB 87-92 and 87-101, 364 KB 122 and 116-130, 500 KB 140-158 and
+    // 132 or 330, 711 KB 193-242 and 162-194, 976 KB 253-307 and 207-232.
+    static constexpr size_t SMALL_SOLVE = SMALL_COPY / 2;
     // Numerical factorisation over all levels; seconds = device time.
     int factorize(double thr, int64_t *npiv, int *negdiag, double *seconds);
     // Solve in place on a device block (factor precision, permuted order).
