@@ -102,12 +102,12 @@ int Engine::alloc_sweep(int cols) {
 
 // Before a solve of nrhs right-hand sides.  The first one of more than
 // SWEEP_COLS widens the sweeps to 64, where their vectors take at most 4 GiB
-// and at most a quarter of the memory left: sweeps of 64 cost hardly more
-// launches' time than those of 32 (24 levels of 6 launches, most of them a few
-// us long): three FP32 preconditioner solves of 64 columns (56x48x60) and
-// their CG 7.95 ms in halves, 6.04 ms at once; 128 at a time 6.01.  An
-// instance that never sees so many holds the vectors of 32 (FP32 96^3: 1.77
-// GiB less of 12.1).
+// and the wider ones at most a quarter of the memory left: sweeps of 64 cost
+// hardly more launches' time than those of 32 (24 levels of 6 launches, most
+// of them a few us long): three FP32 preconditioner solves of 64 columns
+// (56x48x60) and their CG 7.95 ms in halves, 6.04 ms at once; 128 at a time
+// 6.01.  A large instance that never sees so many holds the vectors of 32
+// (FP32 96^3: 1.77 GiB less of 12.1).
 int Engine::reserve_sweep(int nrhs) {
     if (nrhs_chunk_ == 0 && alloc_sweep(SWEEP_COLS)) return fail("no device memory for the solve");
     if (nrhs <= SWEEP_COLS || nrhs_chunk_ >= SWEEP_WIDE || keep_sweep) return 0;
@@ -389,7 +389,10 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     if (P.winv_tmax > 0 && !(d_tbuf_ = alloc((size_t)P.winv_tmax * fsz))) return -1;
     d_WB_ = alloc(winvnbr_ * fsz);
     if (d_WB_) HIPCHK(hipMemsetAsync(d_WB_, 0, winvnbr_ * fsz, stream_));
-    if (!d_WB_ || alloc_sweep(SWEEP_COLS)) return fail("no device memory for the solve");
+    // (of 64 at once where they are small: making room later took 5.8 ms of
+    // the first 64-column solve of a system that is solved in 0.3)
+    if (!d_WB_ || ((wide_sweep_bytes() > SWEEP_SMALL || alloc_sweep(SWEEP_WIDE)) && alloc_sweep(SWEEP_COLS)))
+        return fail("no device memory for the solve");
     d_red_ = (double *)alloc((size_t)(512 * 32 + 64) * sizeof(double));
     if (!d_red_ || !d_stat_) return -1;
     HIPCHK(hipStreamSynchronize(stream_));

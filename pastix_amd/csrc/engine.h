@@ -109,7 +109,9 @@ class Engine {
     void *alloc(size_t bytes);
     // Device bytes that sweeps of SWEEP_WIDE right-hand sides take beyond
     // those of SWEEP_COLS; reserve_sweep makes room for a solve of nrhs.
+    // Instances where they take at most SWEEP_SMALL have them from the start.
     static constexpr int SWEEP_COLS = 32, SWEEP_WIDE = 64;
+    static constexpr int64_t SWEEP_SMALL = (int64_t)256 << 20;
     int64_t wide_sweep_bytes() const { return sweep_bytes(SWEEP_WIDE) - sweep_bytes(SWEEP_COLS); }
     int reserve_sweep(int nrhs);
     bool keep_sweep = false;  // sweeps stay as wide as they are

@@ -1,6 +1,6 @@
-"""Device memory of the solve sweeps: the vectors of 32 right-hand sides until
-a call of more (then of 64), none beyond a server's budget, and the results
-before and after they are replaced."""
+"""Device memory of the solve sweeps: the vectors of 64 right-hand sides where
+they are small, else of 32 until a call of more, none beyond a server's budget,
+and the results before and after they are replaced."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ from tests.helpers import analyse
 
 pytestmark = pytest.mark.gpu
 F = pastix.factotype
-GRID = (13, 12, 11)
+SMALL, LARGE = (13, 12, 11), (66, 65, 64)
 
 
 def _berr(A, x, b):
@@ -18,11 +18,12 @@ def _berr(A, x, b):
 
 
 @pytest.mark.parametrize("prec", [spm.SpmDouble, spm.SpmFloat])
-@pytest.mark.parametrize("facto", [F.LLT, F.LU])
-def test_first_call_of_many(facto, prec):
-    A = spm.laplacian7(*GRID, diag=6.0) if facto == F.LLT else spm.convection_diffusion27(*GRID, seed=3)
+@pytest.mark.parametrize("facto,grid", [(F.LLT, SMALL), (F.LU, SMALL), (F.LLT, LARGE)])
+def test_first_call_of_many(facto, grid, prec):
+    A = spm.laplacian7(*grid, diag=6.0) if facto == F.LLT else spm.convection_diffusion27(*grid, seed=3)
     n, fsz = A.shape[0], 8 if prec == spm.SpmDouble else 4
-    h, S, _ = analyse(A, facto == F.LLT, facto, grid=GRID, min_bs=16, max_bs=40)
+    big = {"min_bs": 16, "max_bs": 40} if grid == SMALL else {}
+    h, S, _ = analyse(A, facto == F.LLT, facto, grid=grid, **big)
     pastix.set_amd_iparm(h, pastix.amd_iparm.factor_precision, prec)
     pastix.task_numfact(h, S)
 
@@ -36,11 +37,14 @@ def test_first_call_of_many(facto, prec):
     base = solve(1)
     assert solve(32) == base + 31 * n * fsz   # the permuted right-hand sides
     wide = solve(33)
-    # 32 more columns of the sweep: z and more
-    assert wide - base > 32 * n * fsz + 32 * n * fsz
+    if grid == SMALL:
+        assert wide == base + 32 * n * fsz
+    else:
+        # 32 more columns of the sweep, more than 256 MiB
+        assert wide - base > 32 * n * fsz + (256 << 20)
     assert solve(64) == wide + 31 * n * fsz
     assert solve(1) == wide + 31 * n * fsz
-    assert solve(130) == wide + 97 * n * fsz
+    assert solve(70) == wide + 37 * n * fsz
     pastix.finalize(h)
 
 
@@ -75,21 +79,28 @@ def test_interface_sweep_of_many():
     assert np.abs(got[0] - got[1]).max() <= 1e-13 * np.abs(got[1]).max()
 
 
-@pytest.mark.parametrize("percentage,max_rhs,wider", [(95, 64, True), (95, 32, False), (100, 64, False)])
-def test_server(percentage, max_rhs, wider):
+@pytest.mark.parametrize("grid,percentage,max_rhs,wider", [(LARGE, 95, 64, True), (LARGE, 95, 32, False),
+                                                            (LARGE, 100, 64, False), (SMALL, 95, 64, False)])
+def test_server(grid, percentage, max_rhs, wider):
     """A server's slots take the wider sweeps at its creation, from the memory
     its budget leaves free, or not at all."""
-    A = spm.laplacian7(*GRID, coef=(1.0, 1.0, 0.01))
+    A = spm.laplacian7(*grid, coef=(1.0, 1.0, 0.01))
     n = A.shape[0]
     S = spm.Spm(A, symmetric=True)
     ip, dp = pastix.initParam()
     ip[pastix.iparm.factorization] = F.LLT
     ip[pastix.iparm.refinement] = pastix.refine.CG
     ip[pastix.iparm.gpu_memory_percentage] = percentage
+    ip[pastix.iparm.ordering] = pastix.order.Personal
     h = pastix.init(ip, dp)
     pastix.set_amd_iparm(h, pastix.amd_iparm.factor_precision, spm.SpmFloat)
     pastix.set_amd_iparm(h, pastix.amd_iparm.resident_input, 1)
-    pastix.task_analyze(h, S)
+    o = pastix.orderGrid(*grid)
+    h.order = o
+    pastix.subtask_order(h, S, o)
+    pastix.subtask_symbfact(h)
+    pastix.subtask_reordering(h)
+    pastix.subtask_blend(h)
     pastix.task_numfact(h, S)
     before = pastix.device_bytes(h)
     srv = pastix.Server([h], max_rhs=max_rhs)
