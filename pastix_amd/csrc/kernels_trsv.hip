@@ -684,13 +684,23 @@ __global__ __launch_bounds__(64) void k_bwd_diag_tiny(DevSymbol S, const DiagIte
 // ---------------------------------------------------------------------------
 // Several right-hand sides: the same sweeps as products on the matrix cores,
 // sixteen right-hand sides to an MFMA block and NB blocks to a workgroup, so
-// that the factor crosses once for up to 16 NB of them.  Bound by the levels'
-// memory latency (a 53x47x50 factor is 0.46 GB).  The vector kernels these
-// replace took two (diagonal steps) or eight columns at a time and read the
-// factor again for the next ones: 53x47x50 FP64, 2 columns 1165 -> 847 us, 8
-// 1484 -> 917, 32 3212 -> 1305; FP32 867 -> 601, 1154 -> 655, 2477 -> 904.
-// Products are formed
-// transposed, D(u, row) = sum_k Y(k, u) M(row, k): a lane's results of one
+// that a panel crosses once for up to 16 NB of them (a node's inverse once for
+// up to 16).  Bound by the levels' memory latency (a 53x47x50 factor is 0.46
+// GB).  The vector kernels these replace took two (diagonal steps) or eight
+// columns at a time and read the factor again for the next ones: 53x47x50
+// FP64, 2 columns 1165 -> 847 us, 8 1484 -> 917, 32 3212 -> 1267; FP32 867 ->
+// 601, 1154 -> 655, 2477 -> 904.
+//
+// The vector kernels' sums were spread over up to 64 lanes and waves.  To
+// round as little, an accumulator takes no chain of MFMAs longer than sixteen
+// inner indices (four in the diagonal steps of narrow nodes): each is summed
+// from zero and then added.  Residuals of 2 to 64 right-hand sides over the
+// vector kernels' (LL^t, LDL^t and LU of 2D and 3D grids), mean and largest:
+// with 64 rows, 32 or 64 indices of a wide inverse and all of a narrow one to
+// a chain 1.06 and 1.11 in FP64, 1.08 and 1.15 in FP32; so 0.985 and 0.993,
+// 0.988 and 0.996, for 0.7 % of the time of 32 columns.
+//
+// Products are formed transposed, D(u, row) = sum_k Y(k, u) M(row, k): a lane's results of one
 // MFMA register belong to one right-hand side, so sixteen lanes store
 // consecutive rows.  Rows and right-hand sides that do not exist repeat an
 // existing one (their results are not stored); inner indices beyond the last
@@ -855,11 +865,13 @@ __global__ __launch_bounds__(256) void k_bwd_prod_m(DevSymbol S, const BwdItem *
         __syncthreads();
         if (more) xload();
         if (live) {
-            typename Mfma<T>::v4 p[NB];  // see k_fwd_prod_m
-#pragma unroll
-            for (int b = 0; b < NB; b++) p[b] = {0, 0, 0, 0};
+            constexpr int GS = 4 / E;  // groups of 16 rows
+            typename Mfma<T>::v4 p[NB];
 #pragma unroll
             for (int g = 0; g < NG; g++) {
+                if (g % GS == 0)
+#pragma unroll
+                    for (int b = 0; b < NB; b++) p[b] = {0, 0, 0, 0};
 #pragma unroll
                 for (int e = 0; e < E; e++) m[g][e] = (RR * rs + 4 * E * g + E * kq + e < rn) ? m[g][e] : (T)0;
 #pragma unroll
@@ -868,9 +880,10 @@ __global__ __launch_bounds__(256) void k_bwd_prod_m(DevSymbol S, const BwdItem *
 #pragma unroll
                     for (int e = 0; e < E; e++) p[b] = Mfma<T>::mma(a[e], m[g][e], p[b]);
                 }
-            }
+                if (g % GS == GS - 1)
 #pragma unroll
-            for (int b = 0; b < NB; b++) acc[b] += p[b];
+                    for (int b = 0; b < NB; b++) acc[b] += p[b];
+            }
         }
     }
     T *out = part + (int64_t)it.slot * nrhs + (int64_t)u0 * K;
@@ -992,10 +1005,14 @@ __global__ __launch_bounds__(64 * W) void k_diag_narrow_m(DevSymbol S, const Dia
 #pragma unroll
     for (int b = 0; b < NB; b++) acc[b] = {0, 0, 0, 0};
 #pragma unroll
-    for (int s = 0; s < 4 * W; s++) {
+    for (int s = 0; s < 4 * W; s += 2) {
         if (s >= s0 && s < s1) {  // uniform in the wave
 #pragma unroll
-            for (int b = 0; b < NB; b++) acc[b] = Mfma<T>::mma(y[16 * b + i][4 * s + kq], m[s], acc[b]);
+            for (int b = 0; b < NB; b++) {
+                const typename Mfma<T>::v4 zero = {0, 0, 0, 0};
+                acc[b] += Mfma<T>::mma(y[16 * b + i][4 * s + kq], m[s], zero) +
+                          Mfma<T>::mma(y[16 * b + i][4 * s + 4 + kq], m[s + 1], zero);
+            }
         }
     }
     if (ro + i < K) {
@@ -1066,14 +1083,17 @@ __global__ __launch_bounds__(256) void k_diag_gemm16(DevSymbol S, const DiagItem
                 }
             }
         }
-        typename Mfma<T>::v4 p = {0, 0, 0, 0};  // see k_fwd_prod_m
 #pragma unroll
-        for (int j = 0; j < U; j++) {
-            if (kb0 + 4 * G * j >= k1) break;  // uniform
+        for (int j0 = 0; j0 < U; j0 += 4 / E) {
+            typename Mfma<T>::v4 p = {0, 0, 0, 0};
 #pragma unroll
-            for (int e = 0; e < E; e++) p = Mfma<T>::mma(a[j][e], m[j][e], p);
+            for (int j = j0; j < j0 + 4 / E; j++) {
+                if (kb0 + 4 * G * j >= k1) break;  // uniform
+#pragma unroll
+                for (int e = 0; e < E; e++) p = Mfma<T>::mma(a[j][e], m[j][e], p);
+            }
+            acc += p;
         }
-        acc += p;
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) red[wave][Mfma<T>::drow(lane, q)][i] = acc[q];
