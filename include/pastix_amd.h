@@ -271,7 +271,10 @@ int pastix_amd_refactorize(pastix_data_t *pastix_data);
 int pastix_amd_refactorize_shift(pastix_data_t *pastix_data, double delta);
 
 /* Device memory held by the instance's engine, in bytes (factor, inverses,
- * plan, work space, input copy). */
+ * plan, work space, input copy).  It grows with the right-hand sides of a call
+ * (their work blocks; in the first call of more than 32 also the vectors of
+ * wider solve sweeps, where those of 32 are over 256 MiB and memory is to be
+ * had). */
 int pastix_amd_device_bytes(const pastix_data_t *pastix_data, int64_t *bytes);
 
 /* ---- Serving loop (no counterpart in the reference) ----------------------
@@ -289,7 +292,9 @@ int pastix_amd_device_bytes(const pastix_data_t *pastix_data, int64_t *bytes);
  *          runs on a slot whose version has no solve left while other slots
  *          keep solving, each slot on its own HIP stream.
  * One worker thread per slot.  b must stay valid until the request is
- * waited for. */
+ * waited for.  With max_rhs over 32 the slots take wider solve sweeps at the
+ * server's creation, if all of them fit half of the memory that the work
+ * budget leaves free. */
 typedef struct pastix_amd_server_s pastix_amd_server_t;
 int pastix_amd_server_create(pastix_amd_server_t **srv, pastix_data_t **slots, int nslots, pastix_int_t max_rhs);
 int pastix_amd_server_submit_solve(pastix_amd_server_t *srv, pastix_int_t nrhs, double *b, pastix_int_t ldb,

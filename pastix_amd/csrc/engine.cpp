@@ -287,7 +287,7 @@ int Engine::init(int device, const Symbol &s, const Layout &L, const Plan &P, in
     const size_t fsz = (prec_ == 2) ? sizeof(float) : sizeof(double);
     // level workspace of the two-phase update: the largest level's products,
     // capped at a quarter of the free device memory (levels above the cap
-    // keep the single-pass LDS-accumulating kernel)
+    // are updated in one pass)
     {
         size_t freeb = 0, totb = 0;
         HIPCHK(hipMemGetInfo(&freeb, &totb));

@@ -669,8 +669,7 @@ __global__ __launch_bounds__(256) void k_winv_leaves(DevSymbol S, const WinvLeaf
     }
 }
 
-// 64-deep staging chunks: the late rounds have few tiles per launch, so each
-// workgroup's chunk latency is not hidden by others
+// columns staged per chunk of the merges' products
 constexpr int WINV_CH = 16;
 
 template <typename T, int PHASE>
